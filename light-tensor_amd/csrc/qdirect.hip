@@ -93,10 +93,10 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 	}
 }
 
-// Returns -1 when the problem is not a small NT product with 16-byte aligned rows.
-int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b)
+// Whether the problem is a small NT product with 16-byte aligned rows that this kernel is the one for.
+bool qdirect_takes(const QProblem& p)
 {
-	if (!(p.a_ks == 1 && p.b_ks == 1 && p.vec_ok && p.K % 16 == 0 && p.M >= 1 && p.N >= 1 && p.K >= 1)) return -1;
+	if (!(p.a_ks == 1 && p.b_ks == 1 && p.vec_ok && p.K % 16 == 0 && p.M >= 1 && p.N >= 1 && p.K >= 1)) return false;
 	const int64_t tiles = (int64_t)ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16);
 	// Up to 8192 tiles, as long as this kernel is ahead of the 128 x 128 direct-to-LDS tiles where those apply (at least
 	// 64 output columns, K >= 512 or at least 64 such tiles: qgemm_dispatch).  It takes about 2.3 us + 4.1 us per million
@@ -107,7 +107,7 @@ int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 	// 1024 x 1000 x 1024: 16.8 and 8.6; 128 x 4096 x 1024: 9.6 and 7.4; 128 x 1024 x 16384: 30.3 and 23.3.  A few output
 	// columns make poor use of 128-column tiles and stay here (4096 x 50 x 5760, l-ten's quantized MNIST layer at a large
 	// batch: 22.5 us).
-	if (tiles > 8192 || p.K > 16384) return -1;
+	if (tiles > 8192 || p.K > 16384) return false;
 	const uint64_t tiles128 = ceil_div((uint64_t)p.M, 128) * ceil_div((uint64_t)p.N, 128);
 	// (from 64 output columns on: half-empty 128-column tiles still beat this kernel on long or many rows, 4096 x 100 x 9216 58 -> 25
 	// us, 16384 x 64 x 1024 17 -> 7.5 us; at 50 columns, l-ten's layer above, they are level)
@@ -117,8 +117,16 @@ int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 		const int splits = (tiles128 <= 64 && p.K >= 8192) ? (tiles128 <= 32 ? 4 : 2) : (tiles128 <= 32 && p.K >= 4096) ? 2 : 1;
 		const double here = 2.3 + 4.1e-6 * (double)tiles * p.K;
 		const double there = 5.4 + 0.0026 * p.K / splits + (splits > 1 ? 4.0 : 0.0) + (p.N % 4 != 0 ? 2.0 : 0.0) + (p.K % 128 != 0 ? 2.5 : 0.0);
-		if (here >= there) return -1;
+		if (here >= there) return false;
 	}
+	return true;
+}
+
+// Returns -1 when the problem is not one for this kernel.
+int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b)
+{
+	if (!qdirect_takes(p)) return -1;
+	const int64_t tiles = (int64_t)ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16);
 	const int coef_a = 128 - zp_b, coef_b = 128 - zp_a;
 	const dim3 grid((unsigned)tiles);
 	if (p.K <= 1024) {

@@ -360,7 +360,7 @@ static int qgemm_dispatch(const QProblem& p, int out, const SplitScratch* scratc
 			choice = 4;
 	}
 	if (choice >= 20) {
-		const int rc = qgemm_fast_dispatch(p, out, choice);
+		const int rc = choice >= 60 ? qgemm_wave_dispatch(p, out, choice) : qgemm_fast_dispatch(p, out, choice);
 		if (fast_only) return rc;
 		LTEN_HIP_REQUIRE(rc >= 0, "qgemm: forced fast variant %d does not fit this problem", choice);
 		return rc;
@@ -560,6 +560,24 @@ static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const u
 	p.cterm = nullptr;
 	p.rterm = nullptr;
 	const bool may_stream = get_option(OPT_QSKINNY) != 2 && get_option(OPT_QGEMM_TILE) == 0 && get_option(OPT_QGEMM_SPLIT) < 2;  // (a forced tile or split goes to the tiles)
+	const int coef_a = 128 - zpB, coef_b = 128 - zpA;
+	const bool terms = coef_a != 0 || coef_b != 0 || bias != nullptr;
+	// Prepared weights come with their byte sums: the tiled kernels then work out every zero-point term themselves
+	// and this call is one launch.
+	QProblem f = p;
+	const bool fused = weights_prepared && weight_sums != nullptr && terms;
+	if (fused) {
+		f.wsum = weight_sums;
+		f.bias = bias;
+		f.coef_a = coef_a;
+		f.coef_b = coef_b;
+		f.konst = (int32_t)((uint32_t)p.konst + (uint32_t)(128 * k_pad) * (uint32_t)coef_b);  // the kept weight sums count no padding
+	}
+	// few tiles: the wavefronts of a workgroup share K (options that name another kernel keep it)
+	if (weights_prepared && (fused || !terms) && may_stream && get_option(OPT_QSKINNY) == 0 && get_option(OPT_QGEMM_SPLIT) == 0) {
+		const int variant = qgemm_wave_choose(f, qdirect_takes(p));
+		if (variant != 0 && qgemm_wave_dispatch(f, out, variant) == 0) return 0;
+	}
 	// below a megabyte of weights the one-launch kernel's many small workgroups win (option "qskinny" 1: stream anyway)
 	const bool large_weights = N * K >= (1ull << 20) || get_option(OPT_QSKINNY) == 1;
 	if (M <= 32 && large_weights && may_stream) {
@@ -580,19 +598,8 @@ static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const u
 		}
 	}
 
-	const int coef_a = 128 - zpB, coef_b = 128 - zpA;
-	// Prepared weights come with their byte sums: the tiled kernels then work out every zero-point term themselves
-	// and this call is one launch.
-	if (weights_prepared && weight_sums != nullptr && (coef_a != 0 || coef_b != 0 || bias != nullptr)) {
-		QProblem f = p;
-		f.wsum = weight_sums;
-		f.bias = bias;
-		f.coef_a = coef_a;
-		f.coef_b = coef_b;
-		f.konst = (int32_t)((uint32_t)p.konst + (uint32_t)(128 * k_pad) * (uint32_t)coef_b);  // the kept weight sums count no padding
-		if (qgemm_dispatch(f, out, scratch ? &scratch->split : nullptr, true) == 0) return 0;
-	}
-	if (coef_a != 0 || coef_b != 0 || bias != nullptr) {
+	if (fused && qgemm_dispatch(f, out, scratch ? &scratch->split : nullptr, true) == 0) return 0;
+	if (terms) {
 		if (scratch != nullptr) {
 			LTEN_HIP_REQUIRE(M + N <= scratch->terms_ints, "quantized_matmul: M + N = %llu exceeds the %llu rows and columns the static scratch holds",
 			                 (unsigned long long)(M + N), (unsigned long long)scratch->terms_ints);

@@ -113,9 +113,14 @@ int qskinny_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 
 // One-launch kernel for small NT products (qdirect.hip); computes its own zero-point sums.  -1 = does not fit.
 int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b);
+bool qdirect_takes(const QProblem& p);  // whether it will: it fits and is ahead of the 128 x 128 tiles
 
 // Dispatch of the tuned square-ish kernels (qgemm_fast.hip).  Returns -1 when no fast variant fits.
 int qgemm_fast_dispatch(const QProblem& p, int out, int variant);
+// Tiles whose wavefronts share K, for prepared weights (qgemm_wave.hip).  dispatch: -1 = does not fit; choose: the variant
+// expected to be ahead of the kernel the product would take otherwise (direct_takes: that is qdirect.hip's), 0 = none.
+int qgemm_wave_dispatch(const QProblem& p, int out, int variant);
+int qgemm_wave_choose(const QProblem& p, bool direct_takes);
 // Split-K launch; scratch == nullptr takes the library's own buffers (allocated on first use), otherwise the
 // caller's SplitScratch (the entry point that allocates nothing hands in its static device array).
 struct SplitScratch {

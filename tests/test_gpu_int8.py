@@ -850,3 +850,55 @@ def test_cfg3_shape_with_general_zero_points_full_size(gpu, wl, zp):
     want = exact_acc(X, W, zp[0], zp[1])
     mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
     assert np.array_equal(dY.numpy(np.uint8, (M, N)), requant_numpy(want, mult, zp[2]))
+
+
+@pytest.mark.parametrize("tile", [61, 62, 63, 64])
+@pytest.mark.parametrize("shape", [(1, 16, 16), (31, 31, 112), (32, 32, 128), (33, 36, 144), (64, 64, 512), (65, 65, 1040), (63, 100, 1999),
+                                   (100, 48, 1152), (17, 130, 2064)])
+def test_tiles_whose_wavefronts_share_k(gpu, ob, shape, tile):
+    """Prepared weights on the tiles whose wavefronts share K: fewer k-steps than wavefronts, one more than the ring holds, a
+    partial last k-step and padded rows, rows and columns on, below and past the tile's, N a multiple of 16, of 4 and of
+    neither, every zero-point form, a bias on and off a 16-byte boundary.  The oracle's bytes."""
+    M, N, K = shape
+    rng = np.random.default_rng(M * 5 + N * 3 + K + tile)
+    X = rng.integers(0, 256, (M, K), dtype=np.uint8)
+    W = rng.integers(0, 256, (N, K), dtype=np.uint8)
+    l, D = gpu.lib(), gpu.DeviceBuffer
+    Kp = (K + 15) // 16 * 16
+    dX, dW, dWp, dS, dY, ws = D.from_numpy(X), D.from_numpy(W), D(N * Kp), D(4 * N), D(M * N + 16), D(4 * (M + N))
+    gpu.check(l.lten_hip_fcq_prepare_weights(dW.ptr, dWp.ptr, N, K, dS.ptr))
+    bias = rng.integers(-5000, 5000, N + 1).astype(np.int32)
+    dbias = D.from_numpy(bias)
+    gpu.set_option("qgemm_tile", tile)
+    try:
+        for zp in (*ZP_FUSED, [128, 128, 7]):
+            for bias_off in (None, 0, 1):
+                for mult in (0.02 * 0.013 / (0.9 * K / 512), 1.5):
+                    sc = [0.02, 0.013, 0.9 * K / 512] if mult < 1 else [1.5, 1.0, 1.0]
+                    b = None if bias_off is None else bias[bias_off:bias_off + N]
+                    gpu.check(l.lten_hip_fill_u8(dY.ptr, M * N + 16, 0xA5))
+                    gpu.check(l.lten_hip_fcq_forward_prepared(1, M, K, N, dX.ptr, dWp.ptr, dS.ptr, None if b is None else dbias.ptr + 4 * bias_off,
+                                                              gpu.qparams3(sc, zp), dY.ptr, ws.ptr))
+                    assert "_k4_" in gpu.last_kernel() or "_k8_" in gpu.last_kernel(), gpu.last_kernel()
+                    want, _ = ob.quantized_matmul(X, W, np.array(sc, np.float32), np.array(zp, np.uint8), bias=b)
+                    got = dY.numpy(np.uint8, (M * N + 16,))
+                    assert np.array_equal(got[:M * N].reshape(M, N), want), (shape, tile, zp, bias_off, gpu.last_kernel())
+                    assert (got[M * N:] == 0xA5).all(), "bytes behind the output were written"
+    finally:
+        gpu.set_option("qgemm_tile", 0)
+
+
+@pytest.mark.parametrize("shape", [(256, 4096, 4096), (64, 4096, 4096), (17, 2260, 2256), (130, 1024, 8192), (300, 961, 1456), (48, 7646, 5152)])
+def test_middling_batches_on_prepared_weights(gpu, shape):
+    """Layers the library itself sends to those tiles: every output against the closed form."""
+    M, N, K = shape
+    rng = np.random.default_rng(sum(shape))
+    X = rng.integers(0, 256, (M, K), dtype=np.uint8)
+    W = rng.integers(0, 256, (N, K), dtype=np.uint8)
+    bias = rng.integers(-20000, 20000, N).astype(np.int32)
+    for zp in ([128, 128, 128], [17, 125, 100]):
+        sc = [0.02, 0.02, 0.02 * np.sqrt(K)]
+        got, kern = fcq(gpu, gpu.lib().lten_hip_fcq_forward_prepared, X, W, sc, zp, bias, prepared=True)
+        assert "_k4_" in kern or "_k8_" in kern, kern
+        mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
+        assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])), (shape, zp, kern)
