@@ -19,6 +19,7 @@
 // operands contiguous in K, the shape its MFMA tiles are built for) into int32 sums, and a pass that adds l-ten's
 // per-position bias, requantizes and stores in NCHW order.  When the workspace that needs would exceed 2 GiB the
 // call follows l-ten's own decomposition image by image: im2col_u8, then the GEMM with the weights on the left.
+// Layers with more work than launches run as two: pixels of channels, then an implicit GEMM (convq_pixels.hip).
 #include <algorithm>
 #include "conv_common.h"
 #include "qgemm_common.h"
@@ -34,7 +35,13 @@ int conv2dq_image_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w,
 int conv2dq_band_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
                           float zp_out, void* y, bool out_acc);
 
+bool conv2dq_image_takes(const ConvGeo& g, const uint8_t* w);
 double conv2dq_band_estimate_us(const ConvGeo& g);
+double conv2dq_band_us(const ConvGeo& g);
+// two launches, any window: the input as pixels of channels, then an implicit GEMM (convq_pixels.hip); -1 = not a shape for it
+int conv2dq_pixels_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
+                            float zp_out, uint8_t* y, void* workspace, uint64_t workspace_bytes, int forced);
+double conv2dq_pixels_us(const ConvGeo& g, const void* workspace, uint64_t workspace_bytes);
 
 // ND = dwords of packed taps a thread holds (4 taps each): 4, 8, 12 or 16, the smallest that covers K.
 template <int OUT, int ND>
@@ -271,6 +278,24 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	volatile float ab = qp[1].scale * qp[0].scale;
 	const float mult = ab / qp[2].scale, zp_out = (float)qp[2].zero_point;
 
+	const BatchedPlan bp = batched_plan(g);
+	// whether the three launches below are ahead of the band kernel (see there)
+	const bool rows_ahead = get_option(OPT_CONV_VARIANT) == 0 && bp.ok && workspace != nullptr &&
+	                        conv2dq_band_estimate_us(g) > 30.0 + 1.3e-6 * (double)bp.rows * (double)bp.Kp;
+	// Bytes out of a layer with some work: pixels of channels and an implicit GEMM (convq_pixels.hip; int32 sums, which only
+	// checks ask for, keep the kernels below).  Ahead of the three launches and of the decomposition image by image wherever
+	// those were taken (1.6 to 5 times over 60 layers); ahead of the band kernel by the two estimates, with a margin for
+	// their errors (8 x 116 x 24 x 24 -> 25 channels 3 x 3: 12.9 -> 8.0 us, 12 x 18 x 56 x 56 -> 144: 28.2 -> 11.2; 11 x 36 x
+	// 14 x 14 -> 32 stays, 7.4 against 8).  Option "conv_variant" 11 to 16 forces a tile.
+	const int variant = get_option(OPT_CONV_VARIANT);
+	if (!out_acc && (variant == 0 || variant > 10) && (variant > 10 || (K <= CQ_MAXK ? Cout >= 48 : !conv2dq_image_takes(g, w)))) {
+		const uint64_t bytes = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);
+		const double here = conv2dq_pixels_us(g, workspace, bytes), band = rows_ahead && K > CQ_MAXK ? -1.0 : conv2dq_band_us(g);
+		if (here >= 0.0 && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
+			const int rc = conv2dq_pixels_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), workspace, bytes, variant > 10 ? variant - 10 : 0);
+			if (rc >= 0) return rc;
+		}
+	}
 	// Windows of at most 64 taps for 48 output channels and more: the band kernel's matrix cores are ahead of the dot
 	// products below, which issue at a quarter of the vector rate (8 x 16 x 56 x 56 -> 64 channels 2 x 2, stride 2: 26.5
 	// -> 6.9 us; 8 x 64 x 56 x 56 -> 256 channels 1 x 1: 30.0 -> 16.6 us; 64 x 3 x 224 x 224 -> 64 channels 3 x 3: 181 ->
@@ -293,7 +318,6 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 
 	// small images with a longer window (l-ten's quantized MNIST conv2): still one launch, no workspace (convq_image.hip;
 	// option "conv_variant" 2 keeps such shapes on the three launches below, 3 skips the small-image kernel)
-	const BatchedPlan bp = batched_plan(g);
 	if (get_option(OPT_CONV_VARIANT) == 0 || get_option(OPT_CONV_VARIANT) == 3) {
 		int rc = get_option(OPT_CONV_VARIANT) == 3 ? -1 : conv2dq_image_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, out_acc);
 		if (rc >= 0) return rc;
@@ -301,8 +325,6 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 		// it needs in LDS -- unless long windows leave a workgroup so few pixels and channels that it stages more than it
 		// computes and the three launches below are ahead, which take 30 us + 1.3 us per MB of patch rows (32 x 1024 x 14
 		// x 14 -> 256 channels 1 x 1: 132 us on bands, 43 below; 32 x 128 x 28 x 28 -> 256 channels 3 x 3 stride 2: 55 and 44)
-		const bool rows_ahead = get_option(OPT_CONV_VARIANT) == 0 && bp.ok && workspace != nullptr &&
-		                        conv2dq_band_estimate_us(g) > 30.0 + 1.3e-6 * (double)bp.rows * (double)bp.Kp;
 		if (!rows_ahead) rc = conv2dq_band_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, out_acc);
 		if (rc >= 0) return rc;
 	}

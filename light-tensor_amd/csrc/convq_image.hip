@@ -14,6 +14,7 @@
 //   sum (a - zpA)(b - zpB) = sum a'b' + (128 - zpB) SA + (128 - zpA) SB + K (zpA zpB - 16384),
 // a' = a - 128, SA / SB the byte sums of a position's window and of a channel's weights.  Taps past K hold 0x80 in the
 // window (a' = 0) and signed zeros in the weights.
+#include <algorithm>
 #include "conv_common.h"
 #include "qgemm_common.h"
 
@@ -633,6 +634,24 @@ double conv2dq_band_estimate_us(const ConvGeo& g)
 	return wgs * ((double)pl.RH * pl.RW * pl.PP + (double)pl.ncb * 16 * pl.wpitch) / 1.3e6;
 }
 
+// The same, term by term, where the other side of the choice is the two launches of convq_pixels.hip (negative: no plan):
+// per workgroup of a round of 512 a start, the region's bytes, the weights' by the way they are staged, k-steps times
+// passes, and the output.  Fitted to 180 layers (14 % rms, 38 % at most).
+double conv2dq_band_us(const ConvGeo& g)
+{
+	BandPlan pl;
+	if (!band_plan(g, pl)) return -1.0;
+	const int T = g.kh * g.kw;
+	const int64_t HW = (int64_t)g.Ho * g.Wo;
+	const double wgs = (double)g.N * ((g.Ho + pl.TB - 1) / pl.TB) * ((((g.Cout + 15) / 16) + pl.ncb - 1) / pl.ncb);
+	const double region = 1e-4 * (double)pl.RH * pl.RW * pl.PP * (g.W % 4 != 0 ? 1.1 : 1.0);
+	const double weights = 1e-4 * (double)pl.ncb * 16 * pl.wpitch * (g.Cin % 4 == 0 ? 1.07 : (int64_t)g.Cin * T % 4 == 0 ? 6.8 : 3.8);
+	const int passes = ((pl.TB * g.Wo + 15) / 16 + 15) / 16;
+	const double us = std::max(1.0, wgs / 512) * (2.34 * region + weights + 0.195 * (pl.Kp / 64) * passes + 3.82) +
+	                  1.23e-6 * (double)g.N * (double)HW * g.Cout * (HW % 4 != 0 ? 1.94 : 1.0);
+	return std::max(us, 4.5);
+}
+
 // 0 = launched; -1 = not a shape for this route
 int conv2dq_band_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
                           float zp_out, void* y, bool out_acc)
@@ -658,12 +677,10 @@ int conv2dq_band_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, 
 	return 0;
 }
 
-// 0 = launched; -1 = not a shape for this route
-int conv2dq_image_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
-                           float zp_out, void* y, bool out_acc)
+// Whether the small-image kernel is the one for this call.
+static bool image_takes(const ConvGeo& g, const uint8_t* w, ImagePlan& pl)
 {
-	ImagePlan pl;
-	if (!image_plan(g, pl)) return -1;
+	if (!image_plan(g, pl)) return false;
 	// The band kernel, where it applies, is ahead whenever it can permute the weights in registers (1 x 1, 3 x 3, 5 x 5 or
 	// 7 x 7 windows of a multiple of four channels: 16 x 64 x 14 x 14 -> 64 channels 3 x 3 takes 19.4 us here and 10.0 there,
 	// 1 x 16 x 32 x 32 -> 32 7.0 and 5.4) and otherwise once the workgroups of this kernel, each of which stages the
@@ -673,7 +690,21 @@ int conv2dq_image_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w,
 	const int taps = g.kh * g.kw;
 	const bool permuted = (g.Cin & 3) == 0 && (taps == 1 || taps == 9 || taps == 25 || taps == 49) && (reinterpret_cast<uintptr_t>(w) & 3) == 0;
 	BandPlan other;
-	if ((permuted || staged > (16ll << 20)) && band_plan(g, other)) return -1;
+	return !((permuted || staged > (16ll << 20)) && band_plan(g, other));
+}
+
+bool conv2dq_image_takes(const ConvGeo& g, const uint8_t* w)
+{
+	ImagePlan pl;
+	return image_takes(g, w, pl);
+}
+
+// 0 = launched; -1 = not a shape for this route
+int conv2dq_image_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
+                           float zp_out, void* y, bool out_acc)
+{
+	ImagePlan pl;
+	if (!image_takes(g, w, pl)) return -1;
 	const int per_image = (g.Ho * g.Wo + CQI_POS - 1) / CQI_POS;
 	const dim3 grid((unsigned)(g.N * per_image));
 	// windows that cannot reach outside the image need no bounds checks on the way

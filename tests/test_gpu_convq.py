@@ -153,3 +153,73 @@ def test_conv2dq_long_windows_on_small_maps_take_the_three_launches(gpu, ob):
     finally:
         gpu.set_option("conv_variant", 0)
     assert np.array_equal(acc3, want_acc) and np.array_equal(y3, want_y)
+
+
+def conv2dq_at(gpu, geo, x, w, sc, zp, bias, off):
+    """conv2dq_forward with every tensor `off` bytes past its buffer's start (the bias 4 off); the output between guard bytes."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    D = gpu.DeviceBuffer
+    put = lambda a, o: D.from_numpy(np.concatenate([np.zeros(o, np.uint8), a.reshape(-1).view(np.uint8)]))
+    dx, dw = put(x, off), put(w, off)
+    db = put(bias, 4 * off) if bias is not None else None
+    count = N * Cout * ((H + 2 * ph - kh) // sh + 1) * ((W + 2 * pw - kw) // sw + 1)
+    ws_bytes = int(gpu.lib().lten_hip_conv2dq_workspace_bytes(*geo))
+    ws, dy = D(ws_bytes + 64), D(count + off + 32)
+    gpu.check(gpu.lib().lten_hip_fill_u8(dy.ptr, count + off + 32, 0xA5))
+    gpu.check(gpu.lib().lten_hip_fill_u8(ws.ptr, ws_bytes + 64, 0x5A))
+    gpu.check(gpu.lib().lten_hip_conv2dq_forward(*geo, dx.ptr + off, dw.ptr + off, db.ptr + 4 * off if db else None, gpu.qparams3(sc, zp),
+                                                 dy.ptr + off, ws.ptr))
+    got = dy.numpy(np.uint8, (count + off + 32,))
+    assert (got[:off] == 0xA5).all() and (got[off + count:] == 0xA5).all(), "bytes beside the output were written"
+    assert (ws.numpy(np.uint8, (ws_bytes + 64,))[ws_bytes:] == 0x5A).all(), "bytes behind the workspace were written"
+    return got[off:off + count]
+
+
+PIXEL_GEOS = [(1, 16, 8, 8, 32, 3, 3, 1, 1, 1, 1),       # one tile, whole chunks
+              (3, 17, 5, 7, 33, 3, 3, 1, 1, 1, 1),       # 35 positions an image, a channel past a chunk, one past a tile
+              (5, 1, 1, 3, 2, 1, 3, 0, 1, 1, 1),         # images of three pixels
+              (2, 20, 9, 11, 65, 5, 5, 2, 2, 2, 2),      # stride 2, 30 positions an image
+              (1, 70, 13, 9, 100, 3, 5, 0, 2, 2, 1),     # two blocks of channels, the second nearly empty, oblong window
+              (4, 64, 16, 16, 130, 3, 3, 1, 1, 1, 1),    # whole k-steps, stores of 16 positions
+              (2, 250, 6, 6, 40, 1, 1, 0, 0, 1, 1),      # 1 x 1, no border
+              (2, 130, 7, 7, 48, 5, 5, 2, 2, 1, 1),      # a long reduction
+              (9, 6, 12, 10, 64, 4, 2, 3, 0, 3, 2)]      # borders above and below only, wider than the window reaches
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("geo", PIXEL_GEOS)
+def test_conv2dq_pixels_tiles_vs_oracle(gpu, ob, geo, tile):
+    """The two-launch route, every tile forced: remainders of positions, channels, chunks and k-steps, images that end inside a
+    group of 16 positions, tensors on and off their alignment, all zero-point forms and both epilogues."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo) + tile)
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    Ho, Wo = ob.conv_out_hw(H, W, kh, kw, ph, pw, sh, sw)
+    gpu.set_option("conv_variant", 10 + tile)
+    took = False
+    try:
+        for i, (sc, zp, with_bias) in enumerate((([1 / 255, 0.01, 0.05], [0, 128, 128], False), ([0.02, 0.013, 0.9], [17, 250, 100], True),
+                                                 ([1.5, 1.0, 1.0], [200, 3, 9], True))):
+            bias = rng.integers(-9999, 9999, Ho * Wo).astype(np.int32) if with_bias else None
+            want, _ = ob.conv2dq_forward(geo, x, w, sc, zp, bias=bias)
+            got = conv2dq_at(gpu, geo, x, w, sc, zp, bias, i)
+            took |= gpu.last_kernel() == "conv2dq_pixels"
+            assert np.array_equal(got.reshape(want.shape), want), (geo, tile, zp, gpu.last_kernel())
+    finally:
+        gpu.set_option("conv_variant", 0)
+    assert took or geo[0] == 9, geo   # (the last one's pixels do not fit the workspace: strides of 3 and 2)
+
+
+@pytest.mark.parametrize("geo", [(8, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), (8, 116, 24, 24, 25, 3, 3, 1, 1, 1, 1), (3, 134, 30, 31, 70, 5, 5, 2, 2, 1, 1),
+                                 (6, 100, 33, 35, 60, 3, 3, 1, 1, 2, 2), (24, 17, 64, 64, 96, 1, 1, 0, 0, 1, 1)])
+def test_conv2dq_layers_the_library_sends_to_the_two_launches(gpu, ob, geo):
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo))
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    sc, zp = [0.02, 0.013, 0.02 * np.sqrt(Cin * kh * kw)], [17, 125, 100]
+    want, _ = ob.conv2dq_forward(geo, x, w, sc, zp)
+    got = conv2dq_at(gpu, geo, x, w, sc, zp, None, 0)
+    assert gpu.last_kernel() == "conv2dq_pixels", gpu.last_kernel()
+    assert np.array_equal(got.reshape(want.shape), want)
