@@ -1155,9 +1155,9 @@ int sgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, float alpha, c
 		if (rowsum != nullptr) below -= 5.0 + 4.0 * (double)(K * M) / 3e6;  // the column sums then take a launch of their own
 		double plan_us = 1e30;
 		if (below > 0.0 && (plan_us = fast_plan(tA, tB, M, N, K, batch, variant, slices, kc, below)) < below && variant != 0) {
-			// fp16 pairs (sgemm_pairs.hip): half the matrix products, and three launches more.  Only where the sums they take the place of
+			// fp16 pairs (sgemm_pairs.hip): half the matrix products, and two or three launches more.  Only where the sums they take the place of
 			// are longer than 1024: shorter ones lose less to rounding than the pieces do (K = 512: 1.28e-7 against 1.6e-7).
-			if (kc > 1024 * (uint64_t)sgemm_fast_groups(variant) && sgemm_pairs_estimate(M, N, K, batch) < 0.95 * plan_us) {
+			if (kc > 1024 * (uint64_t)sgemm_fast_groups(variant) && sgemm_pairs_estimate(tA, tB, M, N, K, batch) < 0.95 * plan_us) {
 				const uint64_t bytes = sgemm_pairs_bytes(M, N, K, batch);
 				const bool relu = relu_done != nullptr && batch == 1 && (relu_out != nullptr || relu_in != nullptr);
 				SProblem pp = p;

@@ -48,7 +48,7 @@ bool sgemm_fast_takes(const SProblem& p, int tA, int tB, int variant);
 int sgemm_fast_groups(int variant);  // groups of wavefronts that a tile cuts K into
 // The tiles on fp16 pairs (sgemm_pairs.hip): -1 when they do not take the problem; what they take in us, and of library memory.
 int sgemm_pairs_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, void* scratch);
-double sgemm_pairs_estimate(uint64_t M, uint64_t N, uint64_t K, uint64_t batch);
+double sgemm_pairs_estimate(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint64_t batch);
 uint64_t sgemm_pairs_bytes(uint64_t M, uint64_t N, uint64_t K, uint64_t batch);
 double sgemm_fast_estimate(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint64_t batch, int* variant);
 // What a product of row-major operands on 16-byte boundaries takes on the kernels sgemm_run picks, in us, and the bytes of

@@ -1,13 +1,14 @@
 // fp32 GEMM tiles of 128 x 128 on the fp16 matrix cores (fp16_pairs.h): three matrix products stand for one where the bf16 pieces
 // of sgemm_fast.hip need six.
 //
-// Four launches: the range of every row of op(A) and column of op(B) (one read of the operands); their pieces, in the order in which
-// the tiles want them in LDS; the tiles, which load them straight into LDS; and the bf16 tiles of the same size, for tiles that were
-// marked as not to be multiplied so: all other workgroups of that launch end at once.
+// Up to four launches: the range of every row of op(A) and column of op(B); their pieces, in the order in which the tiles want them in
+// LDS (contiguous in k they come with the ranges); the tiles, which load them straight into LDS; and the bf16 tiles of the same size,
+// for tiles that were marked as not to be multiplied so: all other workgroups of that launch end at once.
 //
 // What bounds it: the power limit.  A loop of nothing but matrix instructions on such pieces reaches 1180 TFLOP/s of fp16, 393 of
 // products (bf16 pieces: 1883 and 314: the 11 significand bits cost 1.6 times the energy of 8), the tiles 1110 to 1200.  At 4096^3
-// they take 343-370 us, the ranges 28, the pieces 47 and the last launch 2.6; together 423-441 us where the bf16 tiles took 575-613.
+// they take 343-370 us, ranges and pieces 43-45 (both operands contiguous in k) to 75, the last launch 2.6; together 394-412 us where
+// the bf16 tiles took 575-613.
 // 2-norm error against float64 on N(0,1): K = 1024 1.85e-7 -> 1.68e-7, 2048 2.72e-7 (128-wide tiles) and 7.0e-7 (256 x 256) -> 1.71e-7, 4096
 // 3.96e-7 and 1.00e-6 -> 1.75e-7.  What the pieces themselves lose is 1.1e-7 of it; a product of two values is off by 2^-21 of itself at most.
 #include "common.h"
@@ -23,68 +24,90 @@ namespace lten_hip {
 
 typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));  // rows need not start on 16-byte boundaries
 
-struct RangeOperand {
+// An operand: rows of op(A) or columns of op(B), both called rows here.
+struct PackOperand {
 	const float* values;
 	int64_t ld, stride;
 	int rows, K, batch;
-	int along_k;  // a row's values lie one behind the other
-	int* info;    // [batch][rows]
+	int along_k;      // a row's values lie one behind the other
+	int* info;        // [batch][rows]
+	uint8_t* images;
 };
 
-constexpr int range_threads = 1024, range_rows_k = range_threads / 64, range_rows_across = 32;
+// The pieces: [problem][128 rows][16 of k][leading, rest][octet of k][row][8 fp16], zeros past the matrix: 8 KB for 128 rows and 16 of k.
+constexpr int pair_tile = 128;
+constexpr int image_rows = pair_tile, image_k = 16, image_bytes = image_rows * image_k * 4;
+constexpr int fold_steps = 32;  // (even)
 
-static uint64_t range_blocks(const RangeOperand& o)
+// The first launch: a workgroup of 16 wavefronts takes
+//   16 rows that are contiguous in k, K of at most 4096: it holds them in registers, so their ranges and pieces cost one read of them;
+//   16 rows contiguous in k, any K: their ranges, a wavefront a row;
+//   32 rows contiguous along the row index (a line of memory): their ranges, 128 of k at a time.
+// The second launch makes the pieces of what was not held.  All of it is bound by memory.  At 4096 x 4096 each: two operands
+// contiguous in k 75 us in two launches, 45 in one; rows across (16 of them, 64 bytes a load) 75 and 91, so those take two.
+constexpr int range_threads = 1024, held_k = 4096, rows_along = range_threads / 64, rows_across = 32;
+
+static bool held(const PackOperand& o) { return o.along_k && o.K <= held_k; }
+static uint64_t row_blocks(const PackOperand& o) { return ceil_div(o.rows, image_rows); }
+static uint64_t range_blocks(const PackOperand& o)
 {
-	return o.along_k ? ceil_div((uint64_t)o.rows * o.batch, range_rows_k) : ceil_div(o.rows, range_rows_across) * o.batch;
+	if (held(o)) return row_blocks(o) * (image_rows / rows_along) * o.batch;  // (the rows that fill the last image too)
+	return o.along_k ? ceil_div((uint64_t)o.rows * o.batch, rows_along) : ceil_div(o.rows, rows_across) * o.batch;
 }
 
-// Bound by the read of the operands.  Rows contiguous in k: a wavefront per row.  Contiguous along the row index: a
-// workgroup per 32 rows (a line of memory), 128 of k at a time.
-__global__ __launch_bounds__(range_threads) void sgemm_row_range_kernel(RangeOperand a, RangeOperand b, int a_blocks)
-{
-	const bool is_a = (int)blockIdx.x < a_blocks;
-	const RangeOperand o = is_a ? a : b;
-	const int block = is_a ? blockIdx.x : blockIdx.x - a_blocks;
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	uint32_t largest[4] = { 0, 0, 0, 0 }, smallest[4] = { ~0u, ~0u, ~0u, ~0u };
-	auto see = [&](int e, float v) {
+// The bits of the largest magnitude among some values, and of the smallest but zero less one.
+struct ValueRange {
+	uint32_t largest = 0, smallest = ~0u;
+	__device__ __forceinline__ void see(float v)
+	{
 		const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-		largest[e] = max(largest[e], bits);
-		smallest[e] = min(smallest[e], bits - 1u);  // (zeros do not count)
-	};
-	if (o.along_k) {
-		const int64_t row = (int64_t)block * range_rows_k + wave;
-		if (row >= (int64_t)o.rows * o.batch) return;
-		const int bz = (int)(row / o.rows), r = (int)(row - (int64_t)bz * o.rows);
-		const float* v = o.values + bz * o.stride + (int64_t)r * o.ld;
-		int k = 4 * lane;
-		for (; k + 3 * 256 + 3 < o.K; k += 4 * 256) {
-			f4_any q[4];
-#pragma unroll
-			for (int u = 0; u < 4; u++) q[u] = *reinterpret_cast<const f4_any*>(v + k + u * 256);
-#pragma unroll
-			for (int u = 0; u < 4; u++)
-#pragma unroll
-				for (int e = 0; e < 4; e++) see(e, q[u][e]);
-		}
-		for (; k < o.K; k += 256)
-#pragma unroll
-			for (int e = 0; e < 4; e++) see(e, v[min(k + e, o.K - 1)]);
-		uint32_t hi = max(max(largest[0], largest[1]), max(largest[2], largest[3])), lo = min(min(smallest[0], smallest[1]), min(smallest[2], smallest[3]));
-#pragma unroll
-		for (int d = 32; d > 0; d >>= 1) {
-			hi = max(hi, (uint32_t)__shfl_xor((int)hi, d, 64));
-			lo = min(lo, (uint32_t)__shfl_xor((int)lo, d, 64));
-		}
-		if (lane == 0) o.info[row] = row_info(hi, lo);
-		return;
+		largest = max(largest, bits);
+		smallest = min(smallest, bits - 1u);
 	}
-	__shared__ uint32_t seen[2][range_threads / 64][range_rows_across];
-	const int blocks = (o.rows + range_rows_across - 1) / range_rows_across, bz = block / blocks, r0 = (block - bz * blocks) * range_rows_across;
+	__device__ __forceinline__ void see(uint32_t l, uint32_t s)
+	{
+		largest = max(largest, l);
+		smallest = min(smallest, s);
+	}
+	__device__ __forceinline__ void see_lane(int mask) { see((uint32_t)__shfl_xor((int)largest, mask, 64), (uint32_t)__shfl_xor((int)smallest, mask, 64)); }
+};
+
+__device__ __forceinline__ void range_along(const PackOperand& o, int block)
+{
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int64_t row = (int64_t)block * rows_along + wave;
+	if (row >= (int64_t)o.rows * o.batch) return;
+	const int bz = (int)(row / o.rows), r = (int)(row - (int64_t)bz * o.rows);
+	const float* v = o.values + bz * o.stride + (int64_t)r * o.ld;
+	ValueRange range[4];
+	int k = 4 * lane;
+	for (; k + 3 * 256 + 3 < o.K; k += 4 * 256) {
+		f4_any q[4];
+#pragma unroll
+		for (int u = 0; u < 4; u++) q[u] = *reinterpret_cast<const f4_any*>(v + k + u * 256);
+#pragma unroll
+		for (int u = 0; u < 4; u++)
+#pragma unroll
+			for (int e = 0; e < 4; e++) range[e].see(q[u][e]);
+	}
+	for (; k < o.K; k += 256)
+#pragma unroll
+		for (int e = 0; e < 4; e++) range[e].see(v[min(k + e, o.K - 1)]);
+#pragma unroll
+	for (int e = 1; e < 4; e++) range[0].see(range[e].largest, range[e].smallest);
+#pragma unroll
+	for (int d = 32; d > 0; d >>= 1) range[0].see_lane(d);
+	if (lane == 0) o.info[row] = row_info(range[0].largest, range[0].smallest);
+}
+
+__device__ __forceinline__ void range_across(const PackOperand& o, int block, uint32_t (&seen)[2][16][rows_across])
+{
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int blocks = (o.rows + rows_across - 1) / rows_across, bz = block / blocks, r0 = (block - bz * blocks) * rows_across;
 	// (at least four rows; the last lanes' four rows are moved back inside and seen twice)
-	const int first = min(r0 + 4 * (lane & 7), o.rows - 4);
-	const float* v = o.values + bz * o.stride + first;
+	const float* v = o.values + bz * o.stride + min(r0 + 4 * (lane & 7), o.rows - 4);
 	constexpr int KS = range_threads / 8;
+	ValueRange range[4];
 	int k = wave * 8 + (lane >> 3);
 	for (; k + 7 * KS < o.K; k += 8 * KS) {
 		f4_any q[8];
@@ -93,59 +116,113 @@ __global__ __launch_bounds__(range_threads) void sgemm_row_range_kernel(RangeOpe
 #pragma unroll
 		for (int u = 0; u < 8; u++)
 #pragma unroll
-			for (int e = 0; e < 4; e++) see(e, q[u][e]);
+			for (int e = 0; e < 4; e++) range[e].see(q[u][e]);
 	}
 	for (; k < o.K; k += KS) {
 		const f4_any q = *reinterpret_cast<const f4_any*>(v + (int64_t)k * o.ld);
 #pragma unroll
-		for (int e = 0; e < 4; e++) see(e, q[e]);
+		for (int e = 0; e < 4; e++) range[e].see(q[e]);
 	}
 #pragma unroll
 	for (int e = 0; e < 4; e++) {
 #pragma unroll
-		for (int d = 32; d >= 8; d >>= 1) {
-			largest[e] = max(largest[e], (uint32_t)__shfl_xor((int)largest[e], d, 64));
-			smallest[e] = min(smallest[e], (uint32_t)__shfl_xor((int)smallest[e], d, 64));
-		}
+		for (int d = 32; d >= 8; d >>= 1) range[e].see_lane(d);
 		if (lane < 8) {
-			seen[0][wave][4 * lane + e] = largest[e];
-			seen[1][wave][4 * lane + e] = smallest[e];
+			seen[0][wave][4 * lane + e] = range[e].largest;
+			seen[1][wave][4 * lane + e] = range[e].smallest;
 		}
 	}
 	__syncthreads();
-	if (threadIdx.x >= range_rows_across) return;
-	uint32_t hi = 0, lo = ~0u;
+	if (threadIdx.x >= rows_across) return;
+	ValueRange all;
 #pragma unroll
-	for (int w = 0; w < range_threads / 64; w++) {
-		hi = max(hi, seen[0][w][threadIdx.x]);
-		lo = min(lo, seen[1][w][threadIdx.x]);
-	}
+	for (int w = 0; w < 16; w++) all.see(seen[0][w][threadIdx.x], seen[1][w][threadIdx.x]);
 	const int row = min(r0 + (int)(threadIdx.x & ~3u), o.rows - 4) + (int)(threadIdx.x & 3);
-	o.info[(int64_t)bz * o.rows + row] = row_info(hi, lo);
+	o.info[(int64_t)bz * o.rows + row] = row_info(all.largest, all.smallest);
 }
 
-// The pieces: [problem][128 rows][16 of k][leading, rest][octet of k][row][8 fp16], zeros past the matrix: 8 KB for 128 rows and 16 of k.
-constexpr int pair_tile = 128;
-constexpr int image_rows = pair_tile, image_k = 16, image_bytes = image_rows * image_k * 4;
-constexpr int fold_steps = 32;  // (even)
+// lane -> (row lane / 4, octet of k lane % 4): a line of 16 rows a load, 512 of k a trip.
+__device__ __forceinline__ void range_and_pieces(const PackOperand& o, int block, uint32_t (&seen)[2][16][rows_across], int (&infos)[rows_along])
+{
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int RB = (o.rows + image_rows - 1) / image_rows, KB = (o.K + image_k - 1) / image_k, groups = RB * (image_rows / rows_along);
+	const int bz = block / groups, r0 = (block - bz * groups) * rows_along, row = r0 + (lane >> 2);
+	const float* const v = o.values + bz * o.stride + (int64_t)row * o.ld;
+	constexpr int TRIPS = held_k / 512;
+	float x[TRIPS][8];
+#pragma unroll
+	for (int j = 0; j < TRIPS; j++) {
+		const int k = j * 512 + wave * 32 + (lane & 3) * 8;
+		if (row < o.rows && k + 8 <= o.K) {
+			const f4_any q0 = *reinterpret_cast<const f4_any*>(v + k), q1 = *reinterpret_cast<const f4_any*>(v + k + 4);
+#pragma unroll
+			for (int e = 0; e < 4; e++) {
+				x[j][e] = q0[e];
+				x[j][4 + e] = q1[e];
+			}
+		} else {
+#pragma unroll
+			for (int e = 0; e < 8; e++) x[j][e] = row < o.rows && k + e < o.K ? v[k + e] : 0.0f;
+		}
+	}
+	ValueRange range[4];
+#pragma unroll
+	for (int j = 0; j < TRIPS; j++)
+#pragma unroll
+		for (int e = 0; e < 8; e++) range[e & 3].see(x[j][e]);
+#pragma unroll
+	for (int e = 1; e < 4; e++) range[0].see(range[e].largest, range[e].smallest);
+	range[0].see_lane(1);
+	range[0].see_lane(2);
+	if ((lane & 3) == 0) {
+		seen[0][wave][lane >> 2] = range[0].largest;
+		seen[1][wave][lane >> 2] = range[0].smallest;
+	}
+	__syncthreads();
+	if (threadIdx.x < rows_along) {
+		ValueRange all;
+#pragma unroll
+		for (int w = 0; w < 16; w++) all.see(seen[0][w][threadIdx.x], seen[1][w][threadIdx.x]);
+		const int info = row_info(all.largest, all.smallest);
+		infos[threadIdx.x] = info;
+		if (r0 + (int)threadIdx.x < o.rows) o.info[(int64_t)bz * o.rows + r0 + threadIdx.x] = info;
+	}
+	__syncthreads();
+	const float scale = __builtin_ldexpf(1.0f, infos[lane >> 2] >> 8);
+	uint8_t* const image = o.images + ((int64_t)bz * RB + r0 / image_rows) * KB * image_bytes + (r0 % image_rows + (lane >> 2)) * 16;
+#pragma unroll
+	for (int j = 0; j < TRIPS; j++) {
+		const int k = j * 512 + wave * 32 + (lane & 3) * 8;
+		if (k >= KB * image_k) continue;
+		uint4 hi, lo;
+		pair8(x[j], scale, hi, lo);
+		uint4* to = reinterpret_cast<uint4*>(image + (int64_t)(k / image_k) * image_bytes + (k % image_k / 8) * (image_rows * 16));
+		to[0] = hi;
+		to[image_bytes / 2 / 16] = lo;
+	}
+}
+
+__global__ __launch_bounds__(range_threads) void sgemm_pairs_range_kernel(PackOperand a, PackOperand b, int a_blocks)
+{
+	__shared__ uint32_t seen[2][16][rows_across];
+	__shared__ int infos[rows_along];
+	const bool is_a = (int)blockIdx.x < a_blocks;
+	const PackOperand o = is_a ? a : b;
+	const int block = is_a ? blockIdx.x : blockIdx.x - a_blocks;
+	if (!o.along_k) range_across(o, block, seen);
+	else if (o.K > held_k) range_along(o, block);
+	else range_and_pieces(o, block, seen, infos);
+}
+
+// Contiguous in k: two lanes read 64 bytes of a row, a wavefront writes two pieces of 512 bytes twice.  Contiguous along the row index:
+// the lanes of a wavefront read 64 rows of one k, and write 1 KB twice.
 constexpr int pack_steps = 8;  // images that a workgroup makes one behind the other along k
+static uint64_t pack_blocks(const PackOperand& o) { return held(o) ? 0 : row_blocks(o) * o.batch * ceil_div(ceil_div(o.K, image_k), pack_steps); }
 
-struct PackOperand {
-	RangeOperand from;
-	uint8_t* images;
-};
-
-static int row_blocks(const RangeOperand& o) { return (o.rows + image_rows - 1) / image_rows; }
-static int k_blocks(int K) { return (K + image_k - 1) / image_k; }
-static uint64_t pack_blocks(const RangeOperand& o) { return (uint64_t)row_blocks(o) * o.batch * ceil_div(k_blocks(o.K), pack_steps); }
-
-// Bound by memory: a read of the operand and as many bytes written.  Contiguous in k: four lanes read a line of a row, a wavefront
-// writes four pieces of 256 bytes.  Contiguous along the row index: the lanes of a wavefront read 64 rows of one k, and write 1 KB.
-__global__ __launch_bounds__(256) void sgemm_pack_kernel(PackOperand a, PackOperand b, int a_blocks)
+__global__ __launch_bounds__(256) void sgemm_pairs_pack_kernel(PackOperand a, PackOperand b, int a_blocks)
 {
 	const bool is_a = (int)blockIdx.x < a_blocks;
-	const RangeOperand o = is_a ? a.from : b.from;
-	uint8_t* const images = is_a ? a.images : b.images;
+	const PackOperand o = is_a ? a : b;
 	const int block = is_a ? blockIdx.x : blockIdx.x - a_blocks;
 	const int RB = (o.rows + image_rows - 1) / image_rows, KB = (o.K + image_k - 1) / image_k, KG = (KB + pack_steps - 1) / pack_steps;
 	const int kg = block % KG, rb = (block / KG) % RB, bz = block / KG / RB;
@@ -176,7 +253,7 @@ __global__ __launch_bounds__(256) void sgemm_pack_kernel(PackOperand a, PackOper
 		}
 		uint4 hi, lo;
 		pair8(x, scale, hi, lo);
-		uint4* to = reinterpret_cast<uint4*>(images + (((int64_t)bz * RB + rb) * KB + kb) * image_bytes + oct * (image_rows * 16) + r * 16);
+		uint4* to = reinterpret_cast<uint4*>(o.images + (((int64_t)bz * RB + rb) * KB + kb) * image_bytes + oct * (image_rows * 16) + r * 16);
 		to[0] = hi;
 		to[image_bytes / 2 / 16] = lo;
 	}
@@ -400,11 +477,12 @@ uint64_t sgemm_pairs_bytes(uint64_t M, uint64_t N, uint64_t K, uint64_t batch)
 // What the four launches take, in us (as for the tiles of sgemm_fast.hip: a start, a tile's edge, a k-step of 16 of a CU's tiles, the clock
 // that comes back when part of the chip is idle; and the operands' way through the first two launches).  Fitted to 47 products of 256 to
 // 6000 rows and columns and a K of 1024 to 6000; off by 4 % in the mean.
-double sgemm_pairs_estimate(uint64_t M, uint64_t N, uint64_t K, uint64_t batch)
+double sgemm_pairs_estimate(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint64_t batch)
 {
 	const double tiles = (double)(ceil_div(M, pair_tile) * ceil_div(N, pair_tile) * batch), rounds = std::ceil(tiles / 256.0), steps = (double)ceil_div(K, image_k);
 	const double per_step = tiles <= 256.0 ? 0.324 * (0.61 + 0.39 * tiles / 256.0) : std::max(0.324, 0.31 * rounds);
-	return 19.5 + 3.5 * rounds + steps * per_step + 1.6e-6 * (double)(M + N) * (double)K * (double)batch;
+	auto value = [&](bool along_k) { return along_k && K <= (uint64_t)held_k ? 0.9e-6 : 1.6e-6; };
+	return 19.5 + 3.5 * rounds + steps * per_step + (value(!tA) * (double)M + value(tB) * (double)N) * (double)K * (double)batch;
 }
 
 int sgemm_pairs_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, void* scratch)
@@ -416,29 +494,31 @@ int sgemm_pairs_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, void
 		at += align256(bytes);
 		return here;
 	};
-	const int KB = k_blocks(p.K);
-	PackOperand a = { { p.A, p.lda, p.stride_a, p.M, p.K, p.stride_a == 0 ? 1 : (int)batch, !tA, nullptr }, nullptr };
-	PackOperand b = { { p.B, p.ldb, p.stride_b, p.N, p.K, p.stride_b == 0 ? 1 : (int)batch, tB, nullptr }, nullptr };
+	const int64_t KB = (int64_t)ceil_div(p.K, image_k);
+	PackOperand a = { p.A, p.lda, p.stride_a, p.M, p.K, p.stride_a == 0 ? 1 : (int)batch, !tA, nullptr, nullptr };
+	PackOperand b = { p.B, p.ldb, p.stride_b, p.N, p.K, p.stride_b == 0 ? 1 : (int)batch, tB, nullptr, nullptr };
 	PairProblem q = {};
 	q.p = p;
-	const int64_t a_bytes = (int64_t)row_blocks(a.from) * KB * image_bytes, b_bytes = (int64_t)row_blocks(b.from) * KB * image_bytes;
-	q.a_images = a.images = reinterpret_cast<uint8_t*>(take(a_bytes * a.from.batch));
-	q.b_images = b.images = reinterpret_cast<uint8_t*>(take(b_bytes * b.from.batch));
-	q.a_info = a.from.info = reinterpret_cast<int*>(take(4ull * p.M * a.from.batch));
-	q.b_info = b.from.info = reinterpret_cast<int*>(take(4ull * p.N * b.from.batch));
-	q.a_stride = a.from.batch > 1 ? a_bytes : 0;
-	q.b_stride = b.from.batch > 1 ? b_bytes : 0;
-	q.a_info_stride = a.from.batch > 1 ? p.M : 0;
-	q.b_info_stride = b.from.batch > 1 ? p.N : 0;
+	const int64_t a_bytes = (int64_t)row_blocks(a) * KB * image_bytes, b_bytes = (int64_t)row_blocks(b) * KB * image_bytes;
+	q.a_images = a.images = reinterpret_cast<uint8_t*>(take(a_bytes * a.batch));
+	q.b_images = b.images = reinterpret_cast<uint8_t*>(take(b_bytes * b.batch));
+	q.a_info = a.info = reinterpret_cast<int*>(take(4ull * p.M * a.batch));
+	q.b_info = b.info = reinterpret_cast<int*>(take(4ull * p.N * b.batch));
+	q.a_stride = a.batch > 1 ? a_bytes : 0;
+	q.b_stride = b.batch > 1 ? b_bytes : 0;
+	q.a_info_stride = a.batch > 1 ? p.M : 0;
+	q.b_info_stride = b.batch > 1 ? p.N : 0;
 	q.marks = reinterpret_cast<uint8_t*>(at);
 
-	const uint64_t a_range = range_blocks(a.from), b_range = range_blocks(b.from), a_pack = pack_blocks(a.from), b_pack = pack_blocks(b.from);
+	const uint64_t a_range = range_blocks(a), b_range = range_blocks(b), a_pack = pack_blocks(a), b_pack = pack_blocks(b);
 	const uint64_t tiles = ceil_div(p.M, pair_tile) * ceil_div(p.N, pair_tile);
 	if (a_range + b_range >= (1ull << 31) || a_pack + b_pack >= (1ull << 31) || tiles >= (1ull << 31)) return -1;
-	sgemm_row_range_kernel<<<dim3((unsigned)(a_range + b_range)), dim3(range_threads), 0, stream()>>>(a.from, b.from, (int)a_range);
+	sgemm_pairs_range_kernel<<<dim3((unsigned)(a_range + b_range)), dim3(range_threads), 0, stream()>>>(a, b, (int)a_range);
 	LTEN_HIP_LAUNCH_CHECK();
-	sgemm_pack_kernel<<<dim3((unsigned)(a_pack + b_pack)), dim3(256), 0, stream()>>>(a, b, (int)a_pack);
-	LTEN_HIP_LAUNCH_CHECK();
+	if (a_pack + b_pack != 0) {
+		sgemm_pairs_pack_kernel<<<dim3((unsigned)(a_pack + b_pack)), dim3(256), 0, stream()>>>(a, b, (int)a_pack);
+		LTEN_HIP_LAUNCH_CHECK();
+	}
 	sgemm_pairs_kernel<<<dim3((unsigned)tiles, 1, (unsigned)batch), dim3(256), 0, stream()>>>(q);
 	LTEN_HIP_LAUNCH_CHECK();
 	SProblem left = p;

@@ -12,9 +12,9 @@ NAME = "sgemm_fast_128x128_pairs"
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [(131, 133, 16 * 5 + 7), (64, 58, 48), (128, 256, 1), (257, 130, 16 * 33 + 5), (140, 129, 16 * 64), (1100, 1030, 40)])
+@pytest.mark.parametrize("M,N,K", [(131, 133, 16 * 5 + 7), (64, 58, 48), (128, 256, 1), (257, 130, 16 * 33 + 5), (140, 129, 16 * 64), (1100, 1030, 40), (130, 133, 4100)])
 def test_edges_in_all_layouts(gpu, M, N, K, tA, tB):
-    """Partial tiles and k-steps, one k-step, a fold after 512 of K.  Integers of up to 22 bits in the sum: exact.  alpha, beta, padded odd rows."""
+    """Partial tiles and k-steps, one k-step, a fold after 512 of K, rows too long to be held.  Integers: exact.  alpha, beta, padded odd rows."""
     rng = np.random.default_rng(M + K + 2 * tA + tB)
     A = rng.integers(-8, 9, (M, K)).astype(np.float32)
     B = rng.integers(-8, 9, (K, N)).astype(np.float32)
