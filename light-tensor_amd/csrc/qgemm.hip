@@ -461,10 +461,11 @@ __global__ __launch_bounds__(256) void qgemm_transpose_rows_kernel(const uint8_t
 	}
 }
 
-// k_pad: the last k_pad bytes of every row of A and B are padding (QProblem::k_pad); the call that pads passes it
+// k_pad: the last k_pad bytes of every row of A and B are padding (QProblem::k_pad); the call that pads passes it.
+// a_row, not 0: the rows of A are not padded but a_row = K - k_pad bytes apart; -1 where no kernel takes that.
 static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const uint8_t* A, const uint8_t* B, void* C,
                      int out_acc, const lten_hip_qparams* qp, const int32_t* bias, int32_t* workspace,
-                     bool weights_prepared = false, const RunScratch* scratch = nullptr, const int32_t* weight_sums = nullptr, int k_pad = 0)
+                     bool weights_prepared = false, const RunScratch* scratch = nullptr, const int32_t* weight_sums = nullptr, int k_pad = 0, uint64_t a_row = 0)
 {
 	LTEN_HIP_REQUIRE(qp != nullptr, "quantized_matmul: qparams is null");
 	if (M == 0 || N == 0) return 0;
@@ -487,6 +488,10 @@ static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const u
 	const bool layer_layout = !tA && tB;
 	if (k_pad == 0 && (!layer_layout || (K & 15) != 0) && scratch == nullptr && (weights_prepared || M * N * K >= (1ull << 16))) {
 		const uint64_t Kp = (K + 15) & ~15ull;
+		if (weights_prepared && layer_layout) {
+			const int rc = qgemm_run(0, 1, M, N, Kp, A, B, C, out_acc, qp, bias, workspace, true, nullptr, weight_sums, (int)(Kp - K), K);
+			if (rc >= 0) return rc;
+		}
 		const bool copy_a = tA || Kp != K, copy_b = !weights_prepared && (!tB || Kp != K);
 		const uint64_t bytes_a = copy_a ? M * Kp : 0, bytes_b = copy_b ? N * Kp : 0;
 		uint8_t* buf = static_cast<uint8_t*>(library_scratch(bytes_a + bytes_b));
@@ -545,7 +550,8 @@ static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const u
 	p.split_partial = nullptr;
 	p.split_counters = nullptr;
 	p.splits = 1;
-	p.vec_ok = ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 && (K & 15) == 0 &&
+	if (a_row != 0) p.a_rs = (int64_t)a_row;
+	p.vec_ok = (((a_row != 0 ? 0 : reinterpret_cast<uintptr_t>(A)) | reinterpret_cast<uintptr_t>(B)) & 15) == 0 && (K & 15) == 0 &&
 	           p.a_ks == 1 && p.b_ks == 1;
 
 	int out = Q_OUT_ACC;
@@ -572,6 +578,12 @@ static int qgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, const u
 		f.coef_a = coef_a;
 		f.coef_b = coef_b;
 		f.konst = (int32_t)((uint32_t)p.konst + (uint32_t)(128 * k_pad) * (uint32_t)coef_b);  // the kept weight sums count no padding
+	}
+	if (a_row != 0) {  // only the one-launch kernel, where it is the one for the padded rows
+		if (!may_stream || get_option(OPT_QSKINNY) != 0 || get_option(OPT_QGEMM_SPLIT) != 0 || (M <= 32 && N * K >= (1ull << 20)) ||
+		    qgemm_wave_choose(f, qdirect_takes(p)) != 0)
+			return -1;
+		return qdirect_ragged_dispatch(p, out, bias, zpA, zpB);
 	}
 	// few tiles: the wavefronts of a workgroup share K (options that name another kernel keep it)
 	if (weights_prepared && (fused || !terms) && may_stream && get_option(OPT_QSKINNY) == 0 && get_option(OPT_QGEMM_SPLIT) == 0) {

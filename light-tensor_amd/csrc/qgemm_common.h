@@ -113,6 +113,7 @@ int qskinny_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 
 // One-launch kernel for small NT products (qdirect.hip); computes its own zero-point sums.  -1 = does not fit.
 int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b);
+int qdirect_ragged_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b);  // A's rows not padded as B's are
 bool qdirect_takes(const QProblem& p);  // whether it will: it fits and is ahead of the 128 x 128 tiles
 
 // Dispatch of the tuned square-ish kernels (qgemm_fast.hip).  Returns -1 when no fast variant fits.

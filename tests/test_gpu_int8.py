@@ -902,3 +902,29 @@ def test_middling_batches_on_prepared_weights(gpu, shape):
         assert "_k4_" in kern or "_k8_" in kern, kern
         mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
         assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])), (shape, zp, kern)
+
+
+@pytest.mark.parametrize("shape,kernel", [((64, 10, 50), "w4"), ((17, 33, 1001), "w4"), ((3, 5, 7), "w4"), ((1, 16, 15), "w4"), ((16, 17, 1007), "w4"),
+                                          ((100, 30, 33), "w4"), ((130, 258, 1020), "w4")])
+def test_ragged_rows_are_read_as_they_lie(gpu, shape, kernel):
+    """Small outputs of prepared weights whose activation rows are no multiple of 16 bytes, on and off a 16-byte boundary: one load, a
+    last chunk of 1 to 15 bytes, nothing but that; every zero-point form."""
+    M, N, K = shape
+    rng = np.random.default_rng(M * 7 + N * 3 + K)
+    X = rng.integers(0, 256, (M, K), dtype=np.uint8)
+    W = rng.integers(0, 256, (N, K), dtype=np.uint8)
+    bias = rng.integers(-20000, 20000, N).astype(np.int32)
+    l, D = gpu.lib(), gpu.DeviceBuffer
+    Kp = (K + 15) // 16 * 16
+    dW, dWp, dS, dB, dY, ws = D.from_numpy(W), D(N * Kp), D(4 * N), D.from_numpy(bias), D(M * N), D(4 * (M + N))
+    gpu.check(l.lten_hip_fcq_prepare_weights(dW.ptr, dWp.ptr, N, K, dS.ptr))
+    for shift in (0, 1):
+        dX = D(M * K + shift)
+        dX.upload(X, offset=shift)
+        for zp in ([128, 128, 128], [17, 125, 100], [255, 0, 3]):
+            for sc in ([0.02, 0.02, 0.02 * np.sqrt(K)], [1.5, 1.0, 1.0]):
+                gpu.check(l.lten_hip_fcq_forward_prepared(1, M, K, N, dX.ptr + shift, dWp.ptr, dS.ptr, dB.ptr, gpu.qparams3(sc, zp), dY.ptr, ws.ptr))
+                assert gpu.last_kernel() == "qdirect_16x16_" + kernel, gpu.last_kernel()
+                mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
+                want = requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])
+                assert np.array_equal(dY.numpy(np.uint8, (M, N)), want), (zp, sc, shift)
