@@ -370,3 +370,15 @@ def test_routes_by_the_gemms_own_estimate(gpu, geo, entry, kernel):
     # a part of the outputs, enough to see a wrong operand: two images, or two input channels
     want = dgrad64((2, *geo[1:]), t, dy[:2]) if entry == "dgrad" else wgrad64((N, 2, *geo[2:]), t[:, :2], dy)
     assert np.array_equal(got[:2] if entry == "dgrad" else got[:, :2], want)
+
+
+@pytest.mark.parametrize("N,Cin,Cout", [(4, 130, 250), (8, 97, 257), (6, 512, 64), (2, 256, 256)])
+def test_weight_gradient_of_wide_layers_on_integers(gpu, N, Cin, Cout):
+    """16 tiles and more, so 16 slices or fewer: channels that are no multiple of 3, 4, 32 or 64; one to 16 slices.  Exact."""
+    geo = (N, Cin, 10, 12, Cout, 3, 3, 1, 1, 1, 1)
+    rng = np.random.default_rng(Cin + Cout)
+    x, dy = rng.integers(-8, 9, (N, Cin, 10, 12)).astype(np.float32), rng.integers(-8, 9, (N, Cout, 10, 12)).astype(np.float32)
+    xp = np.pad(x, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    want = np.stack([dy.transpose(1, 0, 2, 3).reshape(Cout, -1) @ xp[:, :, i:i + 10, j:j + 12].transpose(0, 2, 3, 1).reshape(-1, Cin)
+                     for i in range(3) for j in range(3)], axis=-1)
+    assert np.array_equal(run_wgrad(gpu, geo, x, dy).reshape(Cout, Cin, 9), want)
