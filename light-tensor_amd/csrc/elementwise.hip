@@ -417,6 +417,41 @@ __global__ __launch_bounds__(256) void channel_sum_partial_kernel(const float* _
 	if (tid == 0) partial[c * slices + s] = ((part[0] + part[1]) + part[2]) + part[3];
 }
 
+// One launch where a channel has few values: a workgroup each.  Bound by latency (a launch, the loads of a thread all in flight).
+constexpr int CHANNEL_SUM_ONCE = 65536;
+__global__ __launch_bounds__(1024) void channel_sum_kernel(const float* __restrict__ dy, int N, int C, int HW, float* __restrict__ db, int accumulate)
+{
+	__shared__ float part[16];
+	const int c = blockIdx.x, tid = threadIdx.x, total = N * HW;
+	const int step_n = 1024 / HW, step_hw = 1024 % HW;
+	int n = tid / HW, hw = tid % HW;
+	float sum[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
+	for (int i = tid; i < total; i += 16 * 1024) {
+		float v[16];
+#pragma unroll
+		for (int u = 0; u < 16; u++) {  // (every load is issued, past the end that of the first value)
+			const bool in = i + u * 1024 < total;
+			v[u] = dy[in ? ((int64_t)n * C + c) * HW + hw : 0];
+			if (!in) v[u] = 0.0f;
+			n += step_n;
+			hw += step_hw;
+			if (hw >= HW) { hw -= HW; n++; }
+		}
+#pragma unroll
+		for (int u = 0; u < 16; u++) sum[u & 3] += v[u];
+	}
+	float all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+	for (int off = 32; off > 0; off >>= 1) all += __shfl_down(all, off);
+	if ((tid & 63) == 0) part[tid >> 6] = all;
+	__syncthreads();
+	if (tid >= 16) return;
+	all = part[tid];
+#pragma unroll
+	for (int off = 8; off > 0; off >>= 1) all += __shfl_down(all, off);
+	if (tid == 0) db[c] = accumulate ? db[c] + all : all;
+}
+
 __global__ __launch_bounds__(256) void channel_sum_final_kernel(const float* __restrict__ partial, int C, int slices, float* __restrict__ db, int accumulate)
 {
 	const int c = blockIdx.x * 256 + threadIdx.x;
@@ -607,11 +642,17 @@ int lten_hip_conv2d_bias_grad_f32(uint64_t N, uint64_t C, uint64_t HW, const flo
 	LTEN_HIP_REQUIRE(N * HW == 0 || dy != nullptr, "conv2d_bias_grad: dy is null");
 	LTEN_HIP_REQUIRE(C <= CHANNEL_SUM_SLOTS && N < (1ull << 31) && HW < (1ull << 40), "conv2d_bias_grad: more than %d channels", CHANNEL_SUM_SLOTS);
 	if (N * HW == 0) return accumulate ? 0 : lten_hip_zero(db, C * sizeof(float));  // nothing to sum
+	set_kernel_name("channel_sum");
+	// (32 x 256 x 14 x 14: 5.2 and 4.7 us in two launches, 5.0 in one; 16 x 128 x 29 x 29: 5.5 and 4.5, 4.8)
+	if (HW <= CHANNEL_SUM_ONCE && N * HW <= CHANNEL_SUM_ONCE) {
+		channel_sum_kernel<<<dim3((unsigned)C), dim3(1024), 0, stream()>>>(dy, (int)N, (int)C, (int)HW, db, accumulate);
+		LTEN_HIP_LAUNCH_CHECK();
+		return 0;
+	}
 	const uint64_t runs = ceil_div(N * HW, 256);
 	const int slices = (int)std::max<uint64_t>(1, std::min<uint64_t>(std::min<uint64_t>(CHANNEL_SUM_SLOTS / C, 64), runs));
 	float* partial = nullptr;
 	LTEN_HIP_CHECK(hipGetSymbolAddress(reinterpret_cast<void**>(&partial), HIP_SYMBOL(g_channel_partial)));
-	set_kernel_name("channel_sum");
 	channel_sum_partial_kernel<<<dim3((unsigned)C, (unsigned)slices), dim3(256), 0, stream()>>>(dy, (int)N, (int)C, (int64_t)HW, slices, partial);
 	LTEN_HIP_LAUNCH_CHECK();
 	channel_sum_final_kernel<<<dim3((unsigned)ceil_div(C, 256)), dim3(256), 0, stream()>>>(partial, (int)C, slices, db, accumulate);

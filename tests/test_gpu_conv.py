@@ -690,3 +690,16 @@ def test_conv_bias_gradient(gpu, shape):
     gpu.check(l.lten_hip_conv2d_bias_grad_f32(N, C, HW, dR.ptr, dDB.ptr, 0))
     assert rel_err(dDB.numpy(np.float32, (C,)), r.astype(np.float64).sum(axis=(0, 2))) < TOL
     assert l.lten_hip_conv2d_bias_grad_f32(1, 5000, 4, dR.ptr, dDB.ptr, 0) != 0   # more channels than the library's partial array
+
+
+@pytest.mark.parametrize("N,C,HW", [(1, 3, 65536), (2, 2, 32769), (17, 33, 1000), (1, 1, 1025), (16385, 2, 1), (3, 5, 1023), (64, 4, 1024)])
+def test_conv_bias_gradient_in_one_launch_and_two(gpu, N, C, HW):
+    """The largest channel one workgroup sums and the smallest two launches do, rows on either side of its 1024 threads.  Integers: exact."""
+    rng = np.random.default_rng(N + C + HW)
+    dy = rng.integers(-3, 4, (N, C, HW)).astype(np.float32)
+    db0 = rng.integers(-20, 20, C).astype(np.float32)
+    dDY, dDB = gpu.DeviceBuffer.from_numpy(dy), gpu.DeviceBuffer.from_numpy(db0)
+    gpu.check(gpu.lib().lten_hip_conv2d_bias_grad_f32(N, C, HW, dDY.ptr, dDB.ptr, 1))
+    assert np.array_equal(dDB.numpy(np.float32, (C,)), db0 + dy.sum(axis=(0, 2)))
+    gpu.check(gpu.lib().lten_hip_conv2d_bias_grad_f32(N, C, HW, dDY.ptr, dDB.ptr, 0))
+    assert np.array_equal(dDB.numpy(np.float32, (C,)), dy.sum(axis=(0, 2)))
