@@ -21,6 +21,7 @@
 // call follows l-ten's own decomposition image by image: im2col_u8, then the GEMM with the weights on the left.
 // Layers with more work than launches run as two: pixels of channels, then an implicit GEMM (convq_pixels.hip).
 #include <algorithm>
+#include <type_traits>
 #include "conv_common.h"
 #include "qgemm_common.h"
 
@@ -42,6 +43,147 @@ double conv2dq_band_us(const ConvGeo& g);
 int conv2dq_pixels_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
                             float zp_out, uint8_t* y, void* workspace, uint64_t workspace_bytes, int forced);
 double conv2dq_pixels_us(const ConvGeo& g, const void* workspace, uint64_t workspace_bytes);
+
+// Windows of at most 64 taps in rows of 3 to 8: a thread holds one position's window, a row of a channel in DPR dwords, and takes its
+// dot products with the output channels.  NR = rows it holds, the smallest that covers Cin * kh.
+//
+// Bound by latency, and by its own instructions, which a launch this short fetches for the first time: so a row is one load (25 byte
+// loads and their addresses were two thirds of a 5 x 5 window's kernel; those same loads all in flight at once: 7.6 -> 6.6 us), the
+// weights' byte sums are taken once a workgroup (dot products issue at a quarter of the vector rate), and where the positions leave
+// the chip idle `groups` of threads share them and take a part of the channels each.  64 x 1 x 28 x 28 -> 10 channels 5 x 5:
+// 7.6 -> 4.6 us,
+// 32 x 7 x 57 x 57 -> 24 3 x 3 stride 2 17.0 -> 6.1, 64 x 4 x 112 x 112 -> 47 3 x 3 60 -> 46.  Rows of one or two taps and of more than eight are read byte by byte below.
+template <int OUT, int DPR, int NR>
+__global__ __launch_bounds__(256) void conv2dq_direct_rows_kernel(ConvGeo g, const uint8_t* __restrict__ x, const uint8_t* __restrict__ w,
+                                                                  const int32_t* __restrict__ bias, int zp_in, int zp_w, float mult,
+                                                                  float zp_out, void* __restrict__ y, int groups)
+{
+	constexpr int ND = NR * DPR;
+	using row_bits = std::conditional_t<DPR == 2, uint64_t, uint32_t>;
+	typedef row_bits row_any __attribute__((aligned(1)));
+	__shared__ __attribute__((aligned(16))) uint32_t s_w[CQ_CO][ND];
+	__shared__ uint32_t s_sum[CQ_CO];  // the byte sum of a channel's weights
+	const int tid = threadIdx.x;
+	const int rows = g.Cin * g.kh, K = rows * g.kw, HW = g.Ho * g.Wo;
+	const int co0 = blockIdx.y * CQ_CO, nco = min(CQ_CO, g.Cout - co0);
+	if (tid < CQ_CO) s_sum[tid] = 0;
+	__syncthreads();
+
+	// N * HW < 2^31 (checked by the host): 32-bit divisions
+	const uint32_t share = 256u / (uint32_t)groups;
+	const int group = __builtin_amdgcn_readfirstlane((int)((uint32_t)tid / share));  // (a share is whole wavefronts)
+	const uint32_t gid = blockIdx.x * share + ((uint32_t)tid - (uint32_t)group * share);
+	const bool live = gid < (uint32_t)g.N * (uint32_t)HW;
+	const int n = live ? (int)(gid / (uint32_t)HW) : 0, pos = live ? (int)(gid - (uint32_t)n * (uint32_t)HW) : 0;
+	const int ho = (int)((uint32_t)pos / (uint32_t)g.Wo), wo = pos - ho * g.Wo;
+	const int y0 = ho * g.sh - g.ph, x0 = wo * g.sw - g.pw;
+
+	// Row (ci, i) of the window: the bytes from `base` + (ci H + i) W on (x is 4 DPR to 2^31 - 2^16 bytes, checked by the host), moved
+	// back inside x where they reach past an end of it and shifted into place afterwards.  Rows past the last repeat it.
+	const int base = n * (g.Cin * g.H * g.W) + y0 * g.W + x0, last = g.N * (g.Cin * g.H * g.W) - 4 * DPR;
+	row_bits row[NR];
+	int plane_row[NR];  // ci * H + i
+	{
+		int i = 0, at = 0;
+#pragma unroll
+		for (int r = 0; r < NR; r++) {
+			plane_row[r] = at;
+			row[r] = *reinterpret_cast<const row_any*>(x + (uint32_t)min(max(base + at * g.W, 0), last));
+			const int more = r + 1 < rows ? 1 : 0, next = i + more == g.kh ? 1 : 0;
+			i = next ? 0 : i + more;
+			at += more + (next ? g.H - g.kh : 0);
+			asm volatile("" : "+s"(at));  // (a load for every row: one under a condition is a branch, and waits for those before it)
+		}
+	}
+
+	// weights of this block's output channels, laid out as the rows are, bytes past a row's taps and rows past the last zero
+	for (int idx = tid; idx < nco * ND; idx += 256) {
+		const int co = idx / ND, d = idx % ND, r = d / DPR, j0 = d % DPR * 4;
+		const uint8_t* wr = w + (int64_t)(co0 + co) * K;
+		uint32_t byte[4], v = 0;
+#pragma unroll
+		for (int b = 0; b < 4; b++) byte[b] = wr[min(r * g.kw + j0 + b, K - 1)];
+		asm volatile("" : "+v"(byte[0]), "+v"(byte[1]), "+v"(byte[2]), "+v"(byte[3]));  // (four loads in flight)
+#pragma unroll
+		for (int b = 0; b < 4; b++) v |= (r < rows && j0 + b < g.kw ? byte[b] : 0u) << (8 * b);
+		s_w[co][d] = v;
+		atomicAdd(&s_sum[co], __builtin_amdgcn_udot4(v, 0x01010101u, 0u, false));
+	}
+	__syncthreads();
+
+	if (__any(base < 0 || base + plane_row[NR - 1] * g.W > last)) {
+#pragma unroll
+		for (int r = 0; r < NR; r++) {
+			const int off = base + plane_row[r] * g.W, moved = off - min(max(off, 0), last);
+			row[r] = moved < 0 ? row[r] << (8 * min(-moved, 4 * DPR - 1)) : row[r] >> (8 * min(moved, 4 * DPR - 1));
+		}
+	}
+	if (!live) return;
+
+	// taps outside the image count as 0: columns alike in every row, rows by themselves
+	const int from = max(-x0, 0), to = min(g.kw, g.W - x0);
+	const row_bits below_to = to >= 4 * DPR ? ~(row_bits)0 : ((row_bits)1 << (8 * max(to, 0))) - 1;
+	const row_bits columns = from >= 4 * DPR ? 0 : below_to & (~(row_bits)0 << (8 * from));
+	uint32_t xk[ND], xsum = 0;
+	{
+		int i = 0;
+#pragma unroll
+		for (int r = 0; r < NR; r++) {
+			const row_bits v = r < rows && (unsigned)(y0 + i) < (unsigned)g.H ? row[r] & columns : 0;
+#pragma unroll
+			for (int d = 0; d < DPR; d++) {
+				xk[r * DPR + d] = (uint32_t)(v >> (32 * d * (DPR - 1)));
+				xsum = __builtin_amdgcn_udot4(xk[r * DPR + d], 0x01010101u, xsum, false);
+			}
+			if (++i == g.kh) i = 0;
+		}
+	}
+	// l-ten/math_fns.cpp:1362-1380,1433: row_vector[p] = -zpA * sum_k B[k][p] with A = weights; broadcast = K zpA zpB
+	const int fixed = -zp_w * (int)xsum + K * zp_w * zp_in + (bias ? bias[pos] : 0);
+
+	const int part = (nco + groups - 1) / groups, first_co = group * part, end_co = min(first_co + part, nco);
+	const int64_t out = ((int64_t)n * g.Cout + co0) * HW + pos;
+	for (int co = first_co; co < end_co; co++) {
+		uint32_t dot = 0;
+#pragma unroll
+		for (int d = 0; d < ND; d++) dot = __builtin_amdgcn_udot4(s_w[co][d], xk[d], dot, false);
+		const int v = (int)dot + fixed - zp_in * (int)s_sum[co];
+		const int64_t o = out + (int64_t)co * HW;
+		if (OUT == Q_OUT_ACC) static_cast<int*>(y)[o] = v;
+		else static_cast<uint8_t*>(y)[o] = (uint8_t)requant<OUT>(v, mult, zp_out);
+	}
+}
+
+template <int OUT>
+static bool launch_conv2dq_direct_rows(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w,
+                                       float mult, float zp_out, void* y)
+{
+	const int dpr = g.kw <= 4 ? 1 : 2, rows = g.Cin * g.kh;
+	const int64_t bytes = (int64_t)g.N * g.Cin * g.H * g.W;
+	// (offsets of windows that start above or left of the image, or end below it, stay within 32 bits too)
+	if (g.kw < 3 || g.kw > 8 || rows < 1 || bytes < 4 * dpr || bytes + ((int64_t)g.ph + g.kh + 1) * g.W + g.pw >= (1ll << 31)) return false;
+	// Threads that share positions load the same windows again: only up to two wavefronts a SIMD of them.
+	const uint64_t positions = (uint64_t)g.N * g.Ho * g.Wo;
+	int groups = 1;
+	while (groups < 4 && positions * groups <= 65536 && g.Cout >= 4 * groups) groups *= 2;
+	const dim3 grid((unsigned)ceil_div(positions, (uint64_t)(256 / groups)), (unsigned)ceil_div((uint64_t)g.Cout, CQ_CO));
+	auto launch = [&](auto dpr_c, auto nr_c) {
+		conv2dq_direct_rows_kernel<OUT, decltype(dpr_c)::value, decltype(nr_c)::value><<<grid, dim3(256), 0, stream()>>>(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, groups);
+	};
+	using One = std::integral_constant<int, 1>;
+	using Two = std::integral_constant<int, 2>;
+	if (dpr == 1) {
+		if (rows <= 4) launch(One{}, std::integral_constant<int, 4>{});
+		else if (rows <= 9) launch(One{}, std::integral_constant<int, 9>{});
+		else if (rows <= 15) launch(One{}, std::integral_constant<int, 15>{});
+		else launch(One{}, std::integral_constant<int, 21>{});  // (64 taps in rows of 3)
+	} else {
+		if (rows <= 5) launch(Two{}, std::integral_constant<int, 5>{});
+		else if (rows <= 8) launch(Two{}, std::integral_constant<int, 8>{});
+		else launch(Two{}, std::integral_constant<int, 12>{});  // (64 taps in rows of 5)
+	}
+	return true;
+}
 
 // ND = dwords of packed taps a thread holds (4 taps each): 4, 8, 12 or 16, the smallest that covers K.
 template <int OUT, int ND>
@@ -299,7 +441,7 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	// Windows of at most 64 taps for 48 output channels and more: the band kernel's matrix cores are ahead of the dot
 	// products below, which issue at a quarter of the vector rate (8 x 16 x 56 x 56 -> 64 channels 2 x 2, stride 2: 26.5
 	// -> 6.9 us; 8 x 64 x 56 x 56 -> 256 channels 1 x 1: 30.0 -> 16.6 us; 64 x 3 x 224 x 224 -> 64 channels 3 x 3: 181 ->
-	// 130 us), not for fewer (256 x 3 x 32 x 32 -> 32: 14.5 us below, 19.0 there; l-ten's MNIST conv1, 10 channels: 6.6
+	// 130 us), not for fewer (256 x 3 x 32 x 32 -> 32: 10.4 us below, 19.0 there; l-ten's MNIST conv1, 10 channels: 4.6
 	// and 7.3).  Option "conv_variant" 2 keeps the kernel below.
 	if (K <= CQ_MAXK && Cout >= 48 && (get_option(OPT_CONV_VARIANT) == 0 || get_option(OPT_CONV_VARIANT) == 3)) {
 		const int rc = conv2dq_band_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, out_acc);
@@ -308,8 +450,15 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	if (K <= CQ_MAXK && (uint64_t)N * HW < (1ull << 31) && get_option(OPT_CONV_VARIANT) != 1) {
 		const dim3 grid((unsigned)ceil_div((uint64_t)N * HW, 256), (unsigned)ceil_div(Cout, CQ_CO));
 		set_kernel_name("conv2dq_direct");
+		const bool fast = mult == mult && (mult < 0 ? -mult : mult) <= 0.99f;
+		if (out_acc ? launch_conv2dq_direct_rows<Q_OUT_ACC>(g, x, w, bias, zp_in, zp_w, mult, zp_out, y)
+		    : fast  ? launch_conv2dq_direct_rows<Q_OUT_U8_FAST>(g, x, w, bias, zp_in, zp_w, mult, zp_out, y)
+		            : launch_conv2dq_direct_rows<Q_OUT_U8_EXACT>(g, x, w, bias, zp_in, zp_w, mult, zp_out, y)) {
+			LTEN_HIP_LAUNCH_CHECK();
+			return 0;
+		}
 		if (out_acc) launch_conv2dq_direct<Q_OUT_ACC>(grid, (int)K, g, x, w, bias, zp_in, zp_w, mult, zp_out, y);
-		else if (mult == mult && (mult < 0 ? -mult : mult) <= 0.99f)
+		else if (fast)
 			launch_conv2dq_direct<Q_OUT_U8_FAST>(grid, (int)K, g, x, w, bias, zp_in, zp_w, mult, zp_out, y);
 		else launch_conv2dq_direct<Q_OUT_U8_EXACT>(grid, (int)K, g, x, w, bias, zp_in, zp_w, mult, zp_out, y);
 		LTEN_HIP_LAUNCH_CHECK();

@@ -186,6 +186,54 @@ PIXEL_GEOS = [(1, 16, 8, 8, 32, 3, 3, 1, 1, 1, 1),       # one tile, whole chunk
               (9, 6, 12, 10, 64, 4, 2, 3, 0, 3, 2)]      # borders above and below only, wider than the window reaches
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("geo", [(128, 1, 28, 28, 10, 5, 5, 0, 0, 1, 1),    # 73728 positions: a thread has all channels
+                                 (64, 1, 28, 28, 10, 5, 5, 0, 0, 1, 1),     # two groups of threads, five channels each
+                                 (40, 4, 28, 28, 17, 3, 3, 1, 1, 1, 1),     # two groups of 9 and 8 channels, padded windows of 12 rows
+                                 (3, 1, 9, 11, 16, 2, 3, 0, 0, 1, 1),       # 216 positions: four groups, the last wavefronts past the end
+                                 (1, 3, 7, 9, 15, 4, 4, 3, 2, 1, 2),        # rows whose first taps are outside, all of them or some
+                                 (2, 7, 6, 6, 20, 3, 3, 4, 4, 1, 1),        # 21 rows of 3, windows wholly outside
+                                 (2, 1, 8, 8, 47, 8, 8, 4, 4, 1, 1),        # 8 rows of 8, the last group with 11 of 12 channels
+                                 (1, 2, 5, 5, 3, 6, 5, 1, 0, 1, 1),         # 12 rows of 5, fewer than four channels
+                                 (1, 1, 2, 4, 5, 2, 4, 0, 0, 1, 1),         # the input is one window
+                                 (1, 1, 1, 5, 5, 1, 5, 0, 2, 1, 1),         # an input shorter than a load of 8 bytes
+                                 (2, 1, 4, 12, 6, 3, 9, 0, 1, 1, 1)])       # rows of more than 8 taps
+def test_conv2dq_direct_rows(gpu, ob, geo):
+    """Windows of at most 64 taps, read row by row: loads that reach past the input's ends, the threads that share a position."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo))
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    Ho, Wo = ob.conv_out_hw(H, W, kh, kw, ph, pw, sh, sw)
+    bias = rng.integers(-9999, 9999, Ho * Wo).astype(np.int32)
+    want_y, want_acc = ob.conv2dq_forward(geo, x, w, [0.02, 0.013, 0.9], [17, 250, 100], bias=bias)
+    y, acc = gpu.conv2dq_host(geo, x, w, [0.02, 0.013, 0.9], [17, 250, 100], bias=bias, want_acc=True)
+    assert gpu.last_kernel() == "conv2dq_direct"
+    assert np.array_equal(acc, want_acc) and np.array_equal(y, want_y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("geo", [(128, 1, 28, 28, 10, 5, 5, 0, 0, 1, 1),    # 73728 positions: a thread has all channels
+                                 (64, 1, 28, 28, 10, 5, 5, 0, 0, 1, 1),     # two groups of threads, five channels each
+                                 (40, 4, 28, 28, 17, 3, 3, 1, 1, 1, 1),     # two groups of 9 and 8 channels, padded windows
+                                 (3, 1, 9, 11, 16, 2, 2, 0, 0, 1, 1),       # 240 positions: four groups, the last wavefronts past the end
+                                 (1, 3, 7, 9, 15, 4, 4, 3, 2, 1, 2),        # two groups, windows whose first taps are all outside
+                                 (2, 1, 8, 8, 47, 8, 8, 4, 4, 1, 1),        # 64 taps, four groups, the last with 11 of 12 channels
+                                 (1, 2, 5, 5, 3, 4, 5, 0, 0, 1, 1)])        # 40 taps, fewer than four channels
+def test_conv2dq_direct_groups(gpu, ob, geo):
+    """Short windows: the threads that share a position take their part of the channels, bit-exact."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo))
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    Ho, Wo = ob.conv_out_hw(H, W, kh, kw, ph, pw, sh, sw)
+    bias = rng.integers(-9999, 9999, Ho * Wo).astype(np.int32)
+    want_y, want_acc = ob.conv2dq_forward(geo, x, w, [0.02, 0.013, 0.9], [17, 250, 100], bias=bias)
+    y, acc = gpu.conv2dq_host(geo, x, w, [0.02, 0.013, 0.9], [17, 250, 100], bias=bias, want_acc=True)
+    assert gpu.last_kernel() == "conv2dq_direct"
+    assert np.array_equal(acc, want_acc) and np.array_equal(y, want_y)
+
+
 @pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
 @pytest.mark.parametrize("geo", PIXEL_GEOS)
 def test_conv2dq_pixels_tiles_vs_oracle(gpu, ob, geo, tile):
