@@ -51,8 +51,8 @@ double conv2dq_pixels_us(const ConvGeo& g, const void* workspace, uint64_t works
 // loads and their addresses were two thirds of a 5 x 5 window's kernel; those same loads all in flight at once: 7.6 -> 6.6 us), the
 // weights' byte sums are taken once a workgroup (dot products issue at a quarter of the vector rate), and where the positions leave
 // the chip idle `groups` of threads share them and take a part of the channels each.  64 x 1 x 28 x 28 -> 10 channels 5 x 5:
-// 7.6 -> 4.6 us,
-// 32 x 7 x 57 x 57 -> 24 3 x 3 stride 2 17.0 -> 6.1, 64 x 4 x 112 x 112 -> 47 3 x 3 60 -> 46.  Rows of one or two taps and of more than eight are read byte by byte below.
+// 7.6 -> 4.6 us, 32 x 7 x 57 x 57 -> 24 3 x 3 stride 2 17.0 -> 6.1, 64 x 4 x 112 x 112 -> 47 3 x 3 60 -> 46.  Rows of one or two taps
+// and of more than eight are read byte by byte below.
 template <int OUT, int DPR, int NR>
 __global__ __launch_bounds__(256) void conv2dq_direct_rows_kernel(ConvGeo g, const uint8_t* __restrict__ x, const uint8_t* __restrict__ w,
                                                                   const int32_t* __restrict__ bias, int zp_in, int zp_w, float mult,
