@@ -21,6 +21,7 @@
 // call follows l-ten's own decomposition image by image: im2col_u8, then the GEMM with the weights on the left.
 // Layers with more work than launches run as two: pixels of channels, then an implicit GEMM (convq_pixels.hip).
 #include <algorithm>
+#include <optional>
 #include <type_traits>
 #include "conv_common.h"
 #include "qgemm_common.h"
@@ -41,8 +42,8 @@ double conv2dq_band_estimate_us(const ConvGeo& g);
 double conv2dq_band_us(const ConvGeo& g);
 // two launches, any window: the input as pixels of channels, then an implicit GEMM (convq_pixels.hip); -1 = not a shape for it
 int conv2dq_pixels_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
-                            float zp_out, uint8_t* y, void* workspace, uint64_t workspace_bytes, int forced);
-double conv2dq_pixels_us(const ConvGeo& g, const void* workspace, uint64_t workspace_bytes);
+                            float zp_out, uint8_t* y, void* memory, int forced);
+double conv2dq_pixels_us(const ConvGeo& g, uint64_t& bytes);
 
 // Windows of at most 64 taps in rows of 3 to 8: a thread holds one position's window, a row of a channel in DPR dwords, and takes its
 // dot products with the output channels.  NR = rows it holds, the smallest that covers Cin * kh.
@@ -405,6 +406,8 @@ static BatchedPlan batched_plan(const ConvGeo& g)
 	return b;
 }
 
+constexpr uint64_t LIBRARY_LIMIT = 512ull << 20;  // library memory that a call fills, unless one image takes more
+
 static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_t Cout, int kh, int kw, int ph, int pw, int sh, int sw,
                        const uint8_t* x, const uint8_t* w, const int32_t* bias, const lten_hip_qparams* qp, void* y, bool out_acc,
                        void* workspace)
@@ -420,21 +423,37 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	volatile float ab = qp[1].scale * qp[0].scale;
 	const float mult = ab / qp[2].scale, zp_out = (float)qp[2].zero_point;
 
+	const int variant = get_option(OPT_CONV_VARIANT);
 	const BatchedPlan bp = batched_plan(g);
 	// whether the three launches below are ahead of the band kernel (see there)
-	const bool rows_ahead = get_option(OPT_CONV_VARIANT) == 0 && bp.ok && workspace != nullptr &&
-	                        conv2dq_band_estimate_us(g) > 30.0 + 1.3e-6 * (double)bp.rows * (double)bp.Kp;
+	const bool rows_ahead = variant == 0 && bp.ok && conv2dq_band_estimate_us(g) > 30.0 + 1.3e-6 * (double)bp.rows * (double)bp.Kp;
 	// Bytes out of a layer with some work: pixels of channels and an implicit GEMM (convq_pixels.hip; int32 sums, which only
 	// checks ask for, keep the kernels below).  Ahead of the three launches and of the decomposition image by image wherever
 	// those were taken (1.6 to 5 times over 60 layers); ahead of the band kernel by the two estimates, with a margin for
 	// their errors (8 x 116 x 24 x 24 -> 25 channels 3 x 3: 12.9 -> 8.0 us, 12 x 18 x 56 x 56 -> 144: 28.2 -> 11.2; 11 x 36 x
 	// 14 x 14 -> 32 stays, 7.4 against 8).  Option "conv_variant" 11 to 16 forces a tile.
-	const int variant = get_option(OPT_CONV_VARIANT);
+	// Layers that one of the kernels of one launch could take leave the caller's workspace as it is, whatever they run as: the
+	// header says so.  What they fill is memory of the library's; the others fill the workspace.
 	if (!out_acc && (variant == 0 || variant > 10) && (variant > 10 || (K <= CQ_MAXK ? Cout >= 48 : !conv2dq_image_takes(g, w)))) {
-		const uint64_t bytes = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);
-		const double here = conv2dq_pixels_us(g, workspace, bytes), band = rows_ahead && K > CQ_MAXK ? -1.0 : conv2dq_band_us(g);
-		if (here >= 0.0 && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
-			const int rc = conv2dq_pixels_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), workspace, bytes, variant > 10 ? variant - 10 : 0);
+		uint64_t bytes = 0;
+		const double here = conv2dq_pixels_us(g, bytes), band_us = conv2dq_band_us(g), band = rows_ahead && K > CQ_MAXK ? -1.0 : band_us;
+		const bool one_launch = K <= CQ_MAXK || band_us >= 0.0 || conv2dq_image_takes(g, w);
+		const uint64_t allowed = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);  // (no more than the workspace would hold in any case)
+		if (here >= 0.0 && bytes <= allowed && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
+			// images in groups whose pixels the library's memory holds, one at least
+			ConvGeo part = g;
+			if (one_launch && bytes > LIBRARY_LIMIT) {
+				part.N = (int)std::max<uint64_t>(1, LIBRARY_LIMIT / ceil_div(bytes, N));
+				conv2dq_pixels_us(part, bytes);
+			}
+			void* const memory = one_launch ? library_scratch(bytes) : (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 ? workspace : nullptr;
+			int rc = memory != nullptr ? 0 : -1;
+			for (int n = 0; n < g.N && rc == 0; n += part.N) {
+				ConvGeo now = g;
+				now.N = std::min(part.N, g.N - n);
+				rc = conv2dq_pixels_dispatch(now, x + (int64_t)n * g.Cin * g.H * g.W, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y) + (int64_t)n * g.Cout * HW, memory,
+				                             variant > 10 ? variant - 10 : 0);
+			}
 			if (rc >= 0) return rc;
 		}
 	}
@@ -465,6 +484,7 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 		return 0;
 	}
 
+	void* rows_memory = nullptr;
 	// small images with a longer window (l-ten's quantized MNIST conv2): still one launch, no workspace (convq_image.hip;
 	// option "conv_variant" 2 keeps such shapes on the three launches below, 3 skips the small-image kernel)
 	if (get_option(OPT_CONV_VARIANT) == 0 || get_option(OPT_CONV_VARIANT) == 3) {
@@ -474,13 +494,16 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 		// it needs in LDS -- unless long windows leave a workgroup so few pixels and channels that it stages more than it
 		// computes and the three launches below are ahead, which take 30 us + 1.3 us per MB of patch rows (32 x 1024 x 14
 		// x 14 -> 256 channels 1 x 1: 132 us on bands, 43 below; 32 x 128 x 28 x 28 -> 256 channels 3 x 3 stride 2: 55 and 44)
-		if (!rows_ahead) rc = conv2dq_band_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, out_acc);
+		if (rows_ahead && bp.bytes <= LIBRARY_LIMIT) rows_memory = library_scratch(bp.bytes);
+		if (rows_memory == nullptr) rc = conv2dq_band_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, y, out_acc);
 		if (rc >= 0) return rc;
 	}
 
-	LTEN_HIP_REQUIRE(workspace != nullptr, "conv2dq: workspace is null");
+	LTEN_HIP_REQUIRE(workspace != nullptr || rows_memory != nullptr, "conv2dq: workspace is null");
 	if (bp.ok && get_option(OPT_CONV_VARIANT) != 1) {
-		uint8_t* base = static_cast<uint8_t*>(workspace);
+		std::optional<LibraryScratchHold> hold;  // (the GEMM may ask for memory of its own)
+		if (rows_memory != nullptr) hold.emplace(bp.bytes);
+		uint8_t* base = static_cast<uint8_t*>(rows_memory != nullptr ? rows_memory : workspace);
 		uint8_t* rows = base;
 		uint8_t* wp = base + bp.off_wp;
 		int32_t* sums = reinterpret_cast<int32_t*>(base + bp.off_acc);

@@ -550,11 +550,12 @@ static PixelChoice pixel_tile(const ConvGeo& g, const PixelPlan& pl)
 	return best;
 }
 
-// What the route is expected to take; negative: not a shape for it, or not with this workspace
-double conv2dq_pixels_us(const ConvGeo& g, const void* workspace, uint64_t workspace_bytes)
+// What the route is expected to take, and the bytes of memory it fills; negative: not a shape for it
+double conv2dq_pixels_us(const ConvGeo& g, uint64_t& bytes)
 {
 	PixelPlan pl;
-	if (!pixel_plan(g, pl) || workspace == nullptr || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0 || pl.bytes > workspace_bytes) return -1.0;
+	if (!pixel_plan(g, pl)) return -1.0;
+	bytes = pl.bytes;
 	return pixel_tile(g, pl).us;
 }
 
@@ -584,13 +585,14 @@ static void launch_implicit_wave(const PixelConv& p, bool exact, bool rowsum)
 	}
 }
 
-// 0 = launched; -1 = not a shape for this route.  forced: tile number from 1, 0 the one expected to be quickest.
+// 0 = launched; -1 = not a shape for this route.  memory: the bytes conv2dq_pixels_us names, 16-byte aligned.  forced: tile number from 1,
+// 0 the one expected to be quickest.
 int conv2dq_pixels_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult, float zp_out,
-                            uint8_t* y, void* workspace, uint64_t workspace_bytes, int forced)
+                            uint8_t* y, void* memory, int forced)
 {
 	PixelPlan pl;
-	if (conv2dq_pixels_us(g, workspace, workspace_bytes) < 0.0 || !pixel_plan(g, pl)) return -1;
-	uint8_t* const base = static_cast<uint8_t*>(workspace);
+	if (!pixel_plan(g, pl)) return -1;
+	uint8_t* const base = static_cast<uint8_t*>(memory);
 	uint8_t* const wp = base + pl.off_w;
 	int32_t* const sums = reinterpret_cast<int32_t*>(base + pl.off_sums);
 	PixelConv p;

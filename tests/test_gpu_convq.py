@@ -271,3 +271,49 @@ def test_conv2dq_layers_the_library_sends_to_the_two_launches(gpu, ob, geo):
     got = conv2dq_at(gpu, geo, x, w, sc, zp, None, 0)
     assert gpu.last_kernel() == "conv2dq_pixels", gpu.last_kernel()
     assert np.array_equal(got.reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("geo,kern", [((8, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), "conv2dq_pixels"),        # the band kernel could take it
+                                      ((24, 17, 64, 64, 96, 1, 1, 0, 0, 1, 1), "conv2dq_pixels"),       # 17 taps, 96 channels
+                                      ((16, 1024, 14, 14, 256, 1, 1, 0, 0, 1, 1), "conv2dq_pixels"),    # long windows on small maps
+                                      ((11, 36, 14, 14, 32, 3, 3, 1, 1, 1, 1), "conv2dq_band"),
+                                      ((64, 10, 12, 12, 20, 5, 5, 0, 0, 1, 1), "conv2dq_image"),
+                                      ((40, 4, 28, 28, 17, 3, 3, 1, 1, 1, 1), "conv2dq_direct")])
+def test_conv2dq_leaves_the_workspace_alone(gpu, ob, geo, kern):
+    """Layers that have a kernel of one launch: the workspace keeps its bytes, and may be null, whatever the layer runs as."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo))
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    qp = gpu.qparams3([0.02, 0.013, 0.02 * np.sqrt(Cin * kh * kw)], [17, 125, 100])
+    want, want_acc = ob.conv2dq_forward(geo, x, w, [0.02, 0.013, 0.02 * np.sqrt(Cin * kh * kw)], [17, 125, 100])
+    D, l = gpu.DeviceBuffer, gpu.lib()
+    size = int(l.lten_hip_conv2dq_workspace_bytes(*geo))
+    dx, dw, ws, dy, dacc = D.from_numpy(x), D.from_numpy(w), D(size), D(want.size), D(4 * want.size)
+    gpu.check(l.lten_hip_fill_u8(ws.ptr, size, 0x5A))
+    for memory in (ws.ptr, None):
+        gpu.check(l.lten_hip_fill_u8(dy.ptr, want.size, 0xA5))
+        gpu.check(l.lten_hip_conv2dq_forward(*geo, dx.ptr, dw.ptr, None, qp, dy.ptr, memory))
+        assert gpu.last_kernel() == kern
+        assert np.array_equal(dy.numpy(np.uint8, want.shape), want)
+        gpu.check(l.lten_hip_conv2dq_forward_acc(*geo, dx.ptr, dw.ptr, None, qp, dacc.ptr, memory))
+        assert np.array_equal(dacc.numpy(np.int32, want.shape), want_acc)
+    assert (ws.numpy(np.uint8, (size,)) == 0x5A).all(), "the workspace was written"
+
+
+def test_conv2dq_pixels_in_groups_of_images(gpu, ob):
+    """605 MB of pixels: the library's 512 MB hold seven of the nine images."""
+    geo = (9, 1, 2048, 2048, 2, 3, 3, 1, 1, 1, 1)
+    rng = np.random.default_rng(9)
+    x = rng.integers(0, 256, (9, 1, 2048, 2048), dtype=np.uint8)
+    w = rng.integers(0, 256, (2, 1, 3, 3), dtype=np.uint8)
+    want, _ = ob.conv2dq_forward(geo, x, w, [0.02, 0.013, 0.06], [17, 125, 100])
+    D = gpu.DeviceBuffer
+    dx, dw, dy = D.from_numpy(x), D.from_numpy(w), D(want.size)
+    gpu.set_option("conv_variant", 12)
+    try:
+        gpu.check(gpu.lib().lten_hip_conv2dq_forward(*geo, dx.ptr, dw.ptr, None, gpu.qparams3([0.02, 0.013, 0.06], [17, 125, 100]), dy.ptr, None))
+        assert gpu.last_kernel() == "conv2dq_pixels"
+    finally:
+        gpu.set_option("conv_variant", 0)
+    assert np.array_equal(dy.numpy(np.uint8, want.shape), want)
