@@ -71,3 +71,38 @@ def test_product_does_not_reference_the_oracle(lt):
             if f.endswith((".hip", ".h", ".cpp", ".py")):
                 text = open(os.path.join(root, f), errors="ignore").read()
                 assert "oracle" not in text.lower(), os.path.join(root, f)
+
+
+def _kernel_metadata(path):
+    """What the compiler notes of every kernel in the library's gfx950 code objects, by mangled name."""
+    import msgpack
+    import struct
+    data, kernels, magic = open(path, "rb").read(), {}, b"__CLANG_OFFLOAD_BUNDLE__"
+    at = data.find(magic)
+    while at >= 0:
+        p = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", data, at + len(magic))[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            target, elf = data[p + 24:p + 24 + length], data[at + offset:at + offset + size]
+            p += 24 + length
+            if b"gfx950" not in target:
+                continue
+            sections, = struct.unpack_from("<Q", elf, 0x28)
+            entry, count = struct.unpack_from("<HH", elf, 0x3A)
+            for s in range(sections, sections + entry * count, entry):
+                if struct.unpack_from("<I", elf, s + 4)[0] != 7:  # not a note
+                    continue
+                note, = struct.unpack_from("<Q", elf, s + 0x18)
+                name_bytes, bytes_, kind = struct.unpack_from("<III", elf, note)
+                first = note + 12 + (name_bytes + 3) // 4 * 4
+                if kind == 32:
+                    kernels.update((k[".name"], k) for k in msgpack.unpackb(elf[first:first + bytes_])["amdhsa.kernels"])
+        at = data.find(magic, at + 1)
+    return kernels
+
+
+def test_int8_tiles_keep_everything_in_registers(lt):
+    """No kernel of the int8 products and convolutions spills to scratch memory, the exact-convert forms included."""
+    kernels = {n: k for n, k in _kernel_metadata(lt.LIB_PATH).items() if "qgemm" in n or "qskinny" in n or "qdirect" in n or "conv2dq" in n}
+    assert len(kernels) > 100
+    assert not [n for n, k in kernels.items() if k[".private_segment_fixed_size"] != 0]
