@@ -232,7 +232,7 @@ __global__ __launch_bounds__(NW * 64) void qgemm_wave_kernel(QProblem p)
 		}
 		// The sums as such, in registers: out of the exact form's selects and shifts the compiler otherwise takes them apart element
 		// by element and holds all the partial tiles while it does (244 to 256 registers, of eight wavefronts 448 spilled ones:
-		// 17 x 4096 x 4096 33.5 -> 8.3 us, 100 x 2048 x 2000 32.9 -> EXACT2_US).
+		// 17 x 4096 x 4096 33.4 -> 8.3 us, 100 x 2000 x 2048 32.3 -> 5.6).
 #pragma unroll
 		for (int q = 0; q < 4; q++) asm volatile("" : "+v"(v[q]));
 		unsigned word[4];
@@ -339,9 +339,18 @@ int qgemm_wave_choose(const QProblem& p, bool direct_takes)
 			variant = t.variant;
 		}
 	}
-	// 17 to 32 rows against weights of a megabyte and more, the streaming kernel's: these tiles were ahead on all of 52 such
-	// shapes, by 3 to 38 % (32 x 3392 x 1296: 8.8 -> 8.3 us, 17 x 7221 x 2256: 8.8 -> 5.4, 32 x 8192 x 8192: 16.0 -> 13.2)
-	if (p.M <= 32 && (uint64_t)p.N * p.K >= (1ull << 20)) return variant;
+	// 17 to 32 rows against weights of a megabyte and more, the streaming kernel's.  Up to a K of 8192 and 32768 columns these
+	// tiles were ahead on all of 86 such shapes, by 3 to 69 % (32 x 3392 x 1296: 8.8 -> 8.3 us, 17 x 7221 x 2256: 8.8 -> 5.4, 32 x 8192 x
+	// 8192: 16.0 -> 13.2, 32 x 32768 x 1024: 15.5 -> 12.7), up to 65536 on 65 of 70, by 6 % in the mean (32 x 65536 x 1024: 22.6 -> 19.9;
+	// 17 x 36000 x 1040: 16.5 and 18.2); not where rows of so many outputs start on any byte (17 x 50257 x 768: 17.8 there, 22.3
+	// here), nor with more columns (17 x 131072 x 720: 31.2 and 34.4).  A K above 8192 is cut into chunks there, while a tile here
+	// walks all of it: ahead only with a tile for every other CU (32 x 4096 x 16384: 20.5 there, 17.1 here; 32 x 2048 x 16384: 16.9
+	// and 22.0; 17 x 50 x 25088: 10.1 and 17.0), of rows that start between cache lines from 6000 columns on (32 x 4096 x 8208:
+	// 17.1 and 18.8, 32 x 6000 x 8208: 20.6 and 16.2).
+	if (p.M <= 32 && (uint64_t)p.N * p.K >= (1ull << 20)) {
+		const bool columns = p.N <= 32768 || (p.N <= 65536 && p.N % 4 == 0), length = p.K <= 8192 || p.N >= (p.K % 128 ? 6000 : 4096);
+		return columns && length ? variant : 0;
+	}
 	const double tiles16 = (double)(ceil_div(p.M, 16) * ceil_div(p.N, 16));
 	if (direct_takes) {
 		// the one-launch kernel of qdirect.hip (287 x 960 x 1456: 6.3 -> 4.9 us; 60 x 994 x 6000 stays, 6.3 against 7.4)
