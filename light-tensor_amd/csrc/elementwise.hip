@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void channel_sum_partial_kernel(const float* _
 	if (tid == 0) partial[c * slices + s] = ((part[0] + part[1]) + part[2]) + part[3];
 }
 
-// One launch where a channel has few values: a workgroup each.  Bound by latency (a launch, the loads of a thread all in flight).
+// One launch where a channel has few values (channel_sum_once): a workgroup each.  Bound by latency (a launch, the loads of a thread all in flight).
 constexpr int CHANNEL_SUM_ONCE = 65536;
 __global__ __launch_bounds__(1024) void channel_sum_kernel(const float* __restrict__ dy, int N, int C, int HW, float* __restrict__ db, int accumulate)
 {
@@ -450,6 +450,21 @@ __global__ __launch_bounds__(1024) void channel_sum_kernel(const float* __restri
 #pragma unroll
 	for (int off = 8; off > 0; off >>= 1) all += __shfl_down(all, off);
 	if (tid == 0) db[c] = accumulate ? db[c] + all : all;
+}
+
+// Whether one launch, a workgroup a channel, is ahead of two that spread a channel over up to 64 workgroups; us in one and in
+// two, calls in a recorded row and (both) in a queue that waits for launches, 4.2 and 5.5 us at least:
+//   up to 16384 values a channel, one pass of a workgroup: one (256 channels of 6272 5.2 and 7.6, both 4.3 and 6.1; 16 of 4096
+//   4.8 and 4.4, both 4.2 and 5.5) while the workgroups are on the chip together, 256 channels or 512 whose few values keep four
+//   wavefronts busy; more channels come in rounds, which only values enough make worth it (1024 of 2048 11.1 and 8.0, of 8192
+//   11.8 and 16.7);
+//   beyond, the passes of a workgroup come one behind the other: one only with channels enough to keep the chip as busy (96 of
+//   32768 7.3 and 9.3, of 65536 12.1 and 13.9; 32 of 32768 7.3 and 6.8, 10 of 65536 11.2 and 6.4).
+static bool channel_sum_once(uint64_t C, uint64_t HW, uint64_t values)
+{
+	if (HW > CHANNEL_SUM_ONCE || values > CHANNEL_SUM_ONCE) return false;
+	const bool together = C <= 256 || (C <= 512 && values <= 256) || values >= 8 * C;
+	return together && (values <= 16384 || values <= 700 * C);
 }
 
 __global__ __launch_bounds__(256) void channel_sum_final_kernel(const float* __restrict__ partial, int C, int slices, float* __restrict__ db, int accumulate)
@@ -642,13 +657,13 @@ int lten_hip_conv2d_bias_grad_f32(uint64_t N, uint64_t C, uint64_t HW, const flo
 	LTEN_HIP_REQUIRE(N * HW == 0 || dy != nullptr, "conv2d_bias_grad: dy is null");
 	LTEN_HIP_REQUIRE(C <= CHANNEL_SUM_SLOTS && N < (1ull << 31) && HW < (1ull << 40), "conv2d_bias_grad: more than %d channels", CHANNEL_SUM_SLOTS);
 	if (N * HW == 0) return accumulate ? 0 : lten_hip_zero(db, C * sizeof(float));  // nothing to sum
-	set_kernel_name("channel_sum");
-	// (32 x 256 x 14 x 14: 5.2 and 4.7 us in two launches, 5.0 in one; 16 x 128 x 29 x 29: 5.5 and 4.5, 4.8)
-	if (HW <= CHANNEL_SUM_ONCE && N * HW <= CHANNEL_SUM_ONCE) {
+	if (channel_sum_once(C, HW, N * HW)) {
+		set_kernel_name("channel_sum_once");
 		channel_sum_kernel<<<dim3((unsigned)C), dim3(1024), 0, stream()>>>(dy, (int)N, (int)C, (int)HW, db, accumulate);
 		LTEN_HIP_LAUNCH_CHECK();
 		return 0;
 	}
+	set_kernel_name("channel_sum");
 	const uint64_t runs = ceil_div(N * HW, 256);
 	const int slices = (int)std::max<uint64_t>(1, std::min<uint64_t>(std::min<uint64_t>(CHANNEL_SUM_SLOTS / C, 64), runs));
 	float* partial = nullptr;

@@ -703,3 +703,16 @@ def test_conv_bias_gradient_in_one_launch_and_two(gpu, N, C, HW):
     assert np.array_equal(dDB.numpy(np.float32, (C,)), db0 + dy.sum(axis=(0, 2)))
     gpu.check(gpu.lib().lten_hip_conv2d_bias_grad_f32(N, C, HW, dDY.ptr, dDB.ptr, 0))
     assert np.array_equal(dDB.numpy(np.float32, (C,)), dy.sum(axis=(0, 2)))
+
+
+@pytest.mark.parametrize("N,C,HW,once", [(64, 10, 1024, False), (1, 1, 65536, False), (16, 32, 2048, False), (8, 48, 4096, True), (64, 90, 1024, False),
+                                         (64, 97, 1024, True), (16, 3, 1024, True), (32, 256, 196, True), (8, 1024, 64, False), (128, 1024, 64, True),
+                                         (4, 512, 64, True), (16, 512, 64, False), (1, 4, 65537, False)])
+def test_conv_bias_gradient_route_looks_at_the_channels(gpu, N, C, HW, once):
+    """Few channels of many values are spread over the chip; either route sums integers exactly."""
+    rng = np.random.default_rng(N + C + HW)
+    dy = rng.integers(-3, 4, (N, C, HW)).astype(np.float32)
+    dDY, dDB = gpu.DeviceBuffer.from_numpy(dy), gpu.DeviceBuffer(4 * C)
+    gpu.check(gpu.lib().lten_hip_conv2d_bias_grad_f32(N, C, HW, dDY.ptr, dDB.ptr, 0))
+    assert gpu.last_kernel() == ("channel_sum_once" if once else "channel_sum")
+    assert np.array_equal(dDB.numpy(np.float32, (C,)), dy.sum(axis=(0, 2), dtype=np.float64).astype(np.float32))
