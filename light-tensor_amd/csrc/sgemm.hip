@@ -1086,8 +1086,6 @@ static double fast_plan(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint
 	return us;
 }
 
-constexpr uint64_t pairs_scratch_limit = 2ull << 30;  // library memory that the pieces of a product's operands may take
-
 int sgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, float alpha, const float* A, uint64_t lda,
               int64_t stride_a, const float* B, uint64_t ldb, int64_t stride_b, float beta, float* C, uint64_t ldc,
               int64_t stride_c, uint64_t batch, const float* bias, float* rowsum, bool* rowsum_done, float* relu_out = nullptr,
@@ -1153,20 +1151,7 @@ int sgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, float alpha, c
 		uint64_t slices = 1, kc = K;
 		double below = 0.95 * small_kernels_estimate(tA, tB, M, N, K, batch, operands_vec(p));
 		if (rowsum != nullptr) below -= 5.0 + 4.0 * (double)(K * M) / 3e6;  // the column sums then take a launch of their own
-		double plan_us = 1e30;
-		if (below > 0.0 && (plan_us = fast_plan(tA, tB, M, N, K, batch, variant, slices, kc, below)) < below && variant != 0) {
-			// fp16 pairs (sgemm_pairs.hip): half the matrix products, and two or three launches more.  Only where the sums they take the place of
-			// are longer than 1024: shorter ones lose less to rounding than the pieces do (K = 512: 1.28e-7 against 1.6e-7).
-			if (kc > 1024 * (uint64_t)sgemm_fast_groups(variant) && sgemm_pairs_estimate(tA, tB, M, N, K, batch) < 0.95 * plan_us) {
-				const uint64_t bytes = sgemm_pairs_bytes(M, N, K, batch);
-				const bool relu = relu_done != nullptr && batch == 1 && (relu_out != nullptr || relu_in != nullptr);
-				SProblem pp = p;
-				if (relu) { pp.relu_out = relu_out; pp.relu_in = relu_in; }
-				if (bytes <= pairs_scratch_limit && sgemm_pairs_dispatch(pp, tA, tB, batch, library_scratch(bytes)) == 0) {
-					if (relu) *relu_done = true;
-					return 0;
-				}
-			}
+		if (below > 0.0 && fast_plan(tA, tB, M, N, K, batch, variant, slices, kc, below) < below && variant != 0) {
 			float* partial = slices > 1 ? static_cast<float*>(library_scratch(slices * M * N * sizeof(float))) : nullptr;
 			if (partial != nullptr) {
 				p.C = partial; p.bias = nullptr; p.ldc = (int64_t)N;
@@ -1306,7 +1291,6 @@ int sgemm_run(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, float alpha, c
 	const uint64_t tiles128 = ceil_div(M, 128) * ceil_div(N, 128) * batch;
 	int choice = force;
 	if (choice >= 10) {  // a tile of sgemm_fast.hip by number; falls through to the heuristic when it does not take the problem
-		if (choice == 41 && sgemm_pairs_dispatch(p, tA, tB, batch, library_scratch(sgemm_pairs_bytes(M, N, K, batch))) == 0) return 0;
 		if (sgemm_fast_dispatch(p, tA, tB, batch, choice) == 0) return 0;
 		choice = 0;
 	}

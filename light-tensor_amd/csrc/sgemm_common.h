@@ -29,7 +29,6 @@ struct SProblem {
 	// ldc apart inside it (the output maps of a batch of images, [image][channel][pixel], as one matrix [channel][all pixels])
 	int col_group = 0;
 	int64_t col_group_stride = 0;
-	const uint8_t* marks = nullptr;  // a byte per tile of the batch: 0 is done already (sgemm_pairs.hip)
 	const float* row_bias = nullptr;  // with col_group: added per row m (a convolution's bias per output channel), or null
 };
 
@@ -44,12 +43,6 @@ __device__ __forceinline__ void sgemm_store(const SProblem& p, float* c, float o
 // The tiles of sgemm_fast.hip: one by number (-1 when it does not take the problem), and what the quickest of them is
 // expected to take, in us.
 int sgemm_fast_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, int variant);
-bool sgemm_fast_takes(const SProblem& p, int tA, int tB, int variant);
-int sgemm_fast_groups(int variant);  // groups of wavefronts that a tile cuts K into
-// The tiles on fp16 pairs (sgemm_pairs.hip): -1 when they do not take the problem; what they take in us, and of library memory.
-int sgemm_pairs_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, void* scratch);
-double sgemm_pairs_estimate(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint64_t batch);
-uint64_t sgemm_pairs_bytes(uint64_t M, uint64_t N, uint64_t K, uint64_t batch);
 double sgemm_fast_estimate(int tA, int tB, uint64_t M, uint64_t N, uint64_t K, uint64_t batch, int* variant);
 // What a product of row-major operands on 16-byte boundaries takes on the kernels sgemm_run picks, in us, and the bytes of
 // library memory that the slices of a split reduction want.

@@ -97,8 +97,6 @@ __global__ __launch_bounds__(WM* WN* WK * 64, 2) void sgemm_fast_kernel(SProblem
 	// is read past an edge, and what the tile before already stores is not stored again (m_first, n_first).
 	const int m_first = tm * BM, n_first = tn * BN;
 	const int m0 = p.M >= BM ? min(m_first, p.M - BM) : 0, n0 = p.N >= BN ? min(n_first, p.N - BN) : 0;
-	// (behind the tiles of sgemm_pairs.hip: only what those left)
-	if (p.marks != nullptr && p.marks[((int64_t)bz * tiles_m + tm) * tiles_n + tn] == 0) return;
 	const float* A = p.A + (int64_t)bz * p.stride_a + (A_KC ? (int64_t)m0 * p.lda : m0);
 	const float* B = p.B + (int64_t)bz * p.stride_b + (B_KC ? (int64_t)n0 * p.ldb : n0);
 	float* C = p.C + (int64_t)bz * p.stride_c;
@@ -582,29 +580,13 @@ static int launch_fast(const SProblem& q, int tA, int tB, uint64_t batch)
 	return 0;
 }
 
-static const FastTile* find_tile(int variant)
-{
-	for (const FastTile& t : fast_tiles)
-		if (t.number == variant) return &t;
-	return nullptr;
-}
-
-bool sgemm_fast_takes(const SProblem& p, int tA, int tB, int variant)
-{
-	const FastTile* tile = find_tile(variant);
-	return tile != nullptr && tile_takes(*tile, tA, tB, (uint64_t)p.M, (uint64_t)p.N) && p.K >= 1 && fast_takes(tA, tB, p);
-}
-
-int sgemm_fast_groups(int variant)
-{
-	const FastTile* tile = find_tile(variant);
-	return tile != nullptr ? tile->WK : 1;
-}
-
 int sgemm_fast_dispatch(const SProblem& p, int tA, int tB, uint64_t batch, int variant)
 {
-	if (!sgemm_fast_takes(p, tA, tB, variant)) return -1;
-	set_kernel_name(find_tile(variant)->name);
+	const FastTile* tile = nullptr;
+	for (const FastTile& t : fast_tiles)
+		if (t.number == variant) tile = &t;
+	if (tile == nullptr || !tile_takes(*tile, tA, tB, (uint64_t)p.M, (uint64_t)p.N) || p.K < 1 || !fast_takes(tA, tB, p)) return -1;
+	set_kernel_name(tile->name);
 	switch (variant) {
 	case 12: return launch_fast<256, 256, 4, 2, 1>(p, tA, tB, batch);
 	case 13: return launch_fast<256, 128, 4, 2, 1>(p, tA, tB, batch);

@@ -201,3 +201,15 @@ def test_leading_dimensions_of_millions(gpu, tA, tB):
             gpu.set_option("sgemm_tile", 0)
         assert gpu.last_kernel().startswith("sgemm_fast"), gpu.last_kernel()
         assert np.array_equal(C.numpy(np.float32, (M, N)), A @ B)
+
+
+@pytest.mark.parametrize("M,N,K,tA,tB", [(2048, 2048, 2048, 0, 1), (1500, 1700, 2060, 1, 0), (1100, 3001, 1301, 0, 0)])
+def test_values_keep_all_their_bits_in_long_sums(gpu, M, N, K, tA, tB):
+    """What the library itself picks for a product with a long reduction: values of 24 significand bits against a selection with
+    signs come back bit for bit."""
+    rng = np.random.default_rng(M + N + K)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    first, sign = rng.integers(0, K, N), rng.choice(np.float32([-1, 1]), N)
+    B = np.zeros((K, N), np.float32)
+    B[first, np.arange(N)] = sign
+    assert np.array_equal(sgemm(gpu, tA, tB, A, B), A[:, first] * sign)
