@@ -16,6 +16,18 @@ namespace lten_hip {
 
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
 
+// The bytes of v from number `count` on (0 to 15, the same in every lane), the zero of the signed domain behind them.
+__device__ __forceinline__ v4i drop_bytes(v4i v, int count)
+{
+	const uint32_t none = 0x80808080u;
+	uint32_t w[5] = { (uint32_t)v.x, (uint32_t)v.y, (uint32_t)v.z, (uint32_t)v.w, none };
+	if (count & 8) { w[0] = w[2]; w[1] = w[3]; w[2] = w[3] = none; }
+	if (count & 4) { w[0] = w[1]; w[1] = w[2]; w[2] = w[3]; w[3] = none; }
+#pragma unroll
+	for (int d = 0; d < 4; d++) w[d] = __builtin_amdgcn_alignbyte(w[d + 1], w[d], (uint32_t)count);
+	return v4i{ (int)w[0], (int)w[1], (int)w[2], (int)w[3] };
+}
+
 // RAGGED: the rows of A as they lie, p.K - p.k_pad bytes long and one behind the other, where those of B are padded to p.K.
 template <int WAVES, int OUT, bool RAGGED = false>
 __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const int32_t* bias, int coef_a, int coef_b)
@@ -31,7 +43,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 	const bool a_ok = m0 + lrow < p.M, b_ok = n0 + lrow < p.N;
 	const uint8_t* arow = p.A + (int64_t)(m0 + lrow) * p.a_rs + lgrp * 16;
 	const uint8_t* brow = p.B + (int64_t)(n0 + lrow) * p.b_rs + lgrp * 16;
-	const int steps = (p.K + 63) / 64;
+	const int steps = (p.K + 63) / 64, real = p.K - p.k_pad;
 	const v4i zero = { (int)0x80808080, (int)0x80808080, (int)0x80808080, (int)0x80808080 };
 	const v4i zero_b = { (int)p.b_flip, (int)p.b_flip, (int)p.b_flip, (int)p.b_flip };  // prepared weights: int8 zeros
 
@@ -47,14 +59,23 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 			if (k < p.K) {
 				const uint8_t* a = arow + (int64_t)(s0 + u * WAVES) * 64;
 				if (RAGGED && a_ok) {
-					if (k + 16 <= p.K - p.k_pad) fa[u] = *reinterpret_cast<const v4i_any*>(a);
-					else {  // the row's last chunk, which nothing may be read behind
+					// nothing may be read behind the last row: a row's last chunk is the 16 bytes up to its end, shifted below
+					if (real >= 16) fa[u] = *reinterpret_cast<const v4i_any*>(k + 16 <= real ? a : a - p.k_pad);
+					else if ((m0 + lrow) * real + 16 <= p.M * real) {  // rows shorter than that: some of the next ones too, masked
+						fa[u] = *reinterpret_cast<const v4i_any*>(a);
+#pragma unroll
+						for (int d = 0; d < 4; d++) {
+							const int live = min(max(real - 4 * d, 0), 4);
+							const uint32_t past = live == 4 ? 0u : ~0u << (8 * live);
+							fa[u][d] = (int)(((uint32_t)fa[u][d] & ~past) | (0x80808080u & past));
+						}
+					} else {
 #pragma unroll
 						for (int d = 0; d < 4; d++) {
 							uint32_t word = 0x80808080u;
 #pragma unroll
 							for (int e = 0; e < 4; e++)
-								if (k + 4 * d + e < p.K - p.k_pad) word = (word & ~(0xffu << (8 * e))) | (uint32_t)a[4 * d + e] << (8 * e);
+								if (4 * d + e < real) word = (word & ~(0xffu << (8 * e))) | (uint32_t)a[4 * d + e] << (8 * e);
 							fa[u][d] = (int)word;
 						}
 					}
@@ -64,6 +85,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 		}
 #pragma unroll
 		for (int u = 0; u < U; u++) {
+			if (RAGGED && real >= 16 && (s0 + u * WAVES) * 64 + lgrp * 16 == p.K - 16) fa[u] = drop_bytes(fa[u], p.k_pad);
 			const v4i a = flip_sign_bits(fa[u]), b = flip_bits(fb[u], p.b_flip);
 			sa = __builtin_amdgcn_sdot4(a.x, 0x01010101, sa, false);
 			sa = __builtin_amdgcn_sdot4(a.y, 0x01010101, sa, false);
@@ -163,7 +185,10 @@ int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 }
 
 // A with rows of K - k_pad bytes (RAGGED) where the padded problem would come here with at most four wavefronts: the copy that
-// pads A is a launch of its own (64 x 10 x 50 7.0 -> 4.0 us, 96 x 512 x 1000 7.1 -> 4.1).
+// pads A is a launch of its own (64 x 10 x 50 7.0 -> 4.0 us, 96 x 512 x 1000 7.1 -> 4.1; with a row's last chunk loaded byte by byte
+// large outputs were slower than with the copy, 64 x 8991 x 607 13.3 us and 9.6 where the shifted load takes 10.0, 300 x 1999 x 607
+// 13.0, 9.7 and 10.4, 448 x 832 x 607 8.5, 7.7 and 7.3; over 180 shapes it is ahead of the copy by 28 % in the mean, 7 % behind at
+// most.  Rows shorter than a chunk: 959 x 1568 x 12 11.2 us byte by byte, 9.6 masked, 9.2 with the copy; 500 x 500 x 12 4.2 and 5.2).
 int qdirect_ragged_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, int zp_b)
 {
 	if (p.K > 1024 || !qdirect_takes(p)) return -1;

@@ -943,3 +943,16 @@ def test_ragged_rows_are_read_as_they_lie(gpu, shape, kernel):
                 mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
                 want = requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])
                 assert np.array_equal(dY.numpy(np.uint8, (M, N)), want), (zp, sc, shift)
+
+
+@pytest.mark.parametrize("K", [*range(1, 16), *range(17, 32), *range(593, 608)])
+def test_ragged_rows_last_chunk_of_every_length(gpu, K):
+    """Rows of 1 to 15 bytes, and a last chunk of as many in the first k-step and behind several; 70 rows, the last at the end of the buffer."""
+    M, N = 70, 20
+    rng = np.random.default_rng(K)
+    X, W = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(0, 256, (N, K), dtype=np.uint8)
+    bias, sc, zp = rng.integers(-20000, 20000, N).astype(np.int32), [0.02, 0.02, 0.02 * np.sqrt(K)], [17, 125, 100]
+    got, kern = fcq(gpu, gpu.lib().lten_hip_fcq_forward_prepared, X, W, sc, zp, bias, prepared=True)
+    assert kern == "qdirect_16x16_w4"
+    mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
+    assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2]))
