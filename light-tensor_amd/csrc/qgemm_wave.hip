@@ -339,23 +339,27 @@ int qgemm_wave_choose(const QProblem& p, bool direct_takes)
 			variant = t.variant;
 		}
 	}
-	// 17 to 32 rows against weights of a megabyte and more, the streaming kernel's.  Up to a K of 8192 and 32768 columns these
-	// tiles were ahead on all of 86 such shapes, by 3 to 69 % (32 x 3392 x 1296: 8.8 -> 8.3 us, 17 x 7221 x 2256: 8.8 -> 5.4, 32 x 8192 x
-	// 8192: 16.0 -> 13.2, 32 x 32768 x 1024: 15.5 -> 12.7), up to 65536 on 65 of 70, by 6 % in the mean (32 x 65536 x 1024: 22.6 -> 19.9;
-	// 17 x 36000 x 1040: 16.5 and 18.2); not where rows of so many outputs start on any byte (17 x 50257 x 768: 17.8 there, 22.3
-	// here), nor with more columns (17 x 131072 x 720: 31.2 and 34.4).  A K above 8192 is cut into chunks there, while a tile here
-	// walks all of it: ahead only with a tile for every other CU (32 x 4096 x 16384: 20.5 there, 17.1 here; 32 x 2048 x 16384: 16.9
-	// and 22.0; 17 x 50 x 25088: 10.1 and 17.0), of rows that start between cache lines from 6000 columns on (32 x 4096 x 8208:
-	// 17.1 and 18.8, 32 x 6000 x 8208: 20.6 and 16.2).
+	// 17 to 32 rows against weights of a megabyte and more, the streaming kernel's; pairs are its time and the one here, the weights in
+	// the last-level cache / out of HBM.  Up to a K of 8192 in whole cache lines and 32768 columns these tiles are ahead (32 x 2048 x
+	// 512 7.7 and 4.8; 17 x 1815 x 1024 1.33 / 1.19 times, 32 x 8192 x 8192 1.24 / 1.17, 32 x 1815 x 8192 1.34 / 0.89), up to 65536
+	// on 65 of 70 shapes, by 6 % in the mean (32 x 65536 x 1024: 22.6 and 19.9); not where rows of so many outputs start on any byte
+	// (17 x 50257 x 768: 17.8 and 22.3), nor with more columns (17 x 131072 x 720: 31.2 and 34.4).
+	// A tile walks all of a K on one CU, and rows that start between cache lines take two lines a piece: from HBM that is slower from
+	// a K of about 4608 on (17 x 1000 x 4112 1.64 / 1.11 times, 32 x 1000 x 4112 1.65 / 0.96, x 5008 1.57 / 0.85, x 7504 1.49 /
+	// 0.70) unless there are tiles for most CUs (32 x 6000 x 6000 1.40 / 0.98, 17 x 6000 x 9232 1.54 / 1.29).  A K above 8192 is cut
+	// into chunks there: in whole lines ahead here from about a tile for every third CU on (32 x 3173 x 16384 1.34 / 1.10, 32 x 1500 x 12288 1.38 / 0.85; 17 x 50 x 25088: 10.1 and 17.0 us).
 	if (p.M <= 32 && (uint64_t)p.N * p.K >= (1ull << 20)) {
-		const bool columns = p.N <= 32768 || (p.N <= 65536 && p.N % 4 == 0), length = p.K <= 8192 || p.N >= (p.K % 128 ? 6000 : 4096);
+		const bool columns = p.N <= 32768 || (p.N <= 65536 && p.N % 4 == 0);
+		const bool length = p.K % 128 == 0 ? p.K <= 8192 || p.N >= 3000 : p.K <= 4608 || p.N >= 6000;
 		return columns && length ? variant : 0;
 	}
 	const double tiles16 = (double)(ceil_div(p.M, 16) * ceil_div(p.N, 16));
 	if (direct_takes) {
-		// the one-launch kernel of qdirect.hip (287 x 960 x 1456: 6.3 -> 4.9 us; 60 x 994 x 6000 stays, 6.3 against 7.4)
+		// the one-launch kernel of qdirect.hip (287 x 960 x 1456: 6.3 -> 4.9 us; 60 x 994 x 6000 stays, 6.3 against 7.4).  Its small
+		// tiles hide the way to HBM better, which shows on a long K (64 x 1000 x 7504, weights from there: 10.3 and 14.6, by the
+		// estimates 0.80; 128 x 490 x 6016 8.6 and 10.4; 128 x 1000 x 6000, 0.66, 1.2 times ahead)
 		const double direct = 1.5 + 2.1e-6 * tiles16 * p.K + 0.59 * kk + 0.55 * tiles16 / 1024;
-		return best < 0.85 * direct ? variant : 0;
+		return best < (p.K > 6000 ? 0.79 : 0.85) * direct ? variant : 0;
 	}
 	// the 128 x 128 tiles of qgemm_fast.hip, K split where qgemm_dispatch splits it; outputs that give the chip 256-row tiles
 	// are theirs (256 x 4096 x 4096: 18.4 -> 9.9 us, 64 x 4096 x 4096: 15.2 -> 6.1, 432 x 920 x 6416: 42 -> 11;

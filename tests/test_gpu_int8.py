@@ -904,19 +904,20 @@ def test_middling_batches_on_prepared_weights(gpu, shape):
         assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])), (shape, zp, kern)
 
 
-@pytest.mark.parametrize("shape,streamed", [((17, 42, 25088), True), ((32, 50, 25088), True), ((20, 130, 8208), True), ((32, 64, 16384), True), ((17, 33009, 512), True), ((17, 65552, 512), True),
-                                            ((17, 128, 8192), False), ((32, 4096, 8320), False), ((32, 2048, 512), False), ((17, 33008, 512), False)])
-def test_17_to_32_rows_long_reductions_and_many_columns_are_streamed(gpu, shape, streamed):
-    """Where a tile would walk all of a K above 8192 on a few CUs, or the columns are many, the streaming kernel keeps the layer."""
-    M, N, K = shape
-    rng = np.random.default_rng(sum(shape))
-    X = rng.integers(0, 256, (M, K), dtype=np.uint8)
-    W = rng.integers(0, 256, (N, K), dtype=np.uint8)
-    bias, sc, zp = rng.integers(-20000, 20000, N).astype(np.int32), [0.02, 0.02, 0.02 * np.sqrt(K)], [17, 125, 100]
-    got, kern = fcq(gpu, gpu.lib().lten_hip_fcq_forward_prepared, X, W, sc, zp, bias, prepared=True)
-    assert kern.startswith("qskinny") == streamed and ("_k4_" in kern or "_k8_" in kern) != streamed, kern
-    mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
-    assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])), kern
+@pytest.mark.parametrize("kernel,shapes", [("qskinny", [(17, 42, 25088), (32, 50, 25088), (20, 130, 8208), (32, 64, 16384), (20, 500, 4624), (17, 33009, 512), (17, 65552, 512)]),
+                                           ("qgemm_fast_32", [(17, 128, 8192), (20, 500, 4592), (32, 3072, 8320), (32, 2048, 512), (17, 33008, 512)]),
+                                           ("qdirect", [(64, 1000, 7504), (128, 490, 6016)])])
+def test_long_reductions_and_many_columns_stay_off_the_tiles_that_share_k(gpu, kernel, shapes):
+    """Where a tile would walk a long K on a few CUs, or the columns are many, the kernels that had the layer before keep it."""
+    for M, N, K in shapes:
+        rng = np.random.default_rng(M + N + K)
+        X = rng.integers(0, 256, (M, K), dtype=np.uint8)
+        W = rng.integers(0, 256, (N, K), dtype=np.uint8)
+        bias, sc, zp = rng.integers(-20000, 20000, N).astype(np.int32), [0.02, 0.02, 0.02 * np.sqrt(K)], [17, 125, 100]
+        got, kern = fcq(gpu, gpu.lib().lten_hip_fcq_forward_prepared, X, W, sc, zp, bias, prepared=True)
+        assert kern.startswith(kernel), (M, N, K, kern)
+        mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
+        assert np.array_equal(got, requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])), kern
 
 
 @pytest.mark.parametrize("shape,kernel", [((64, 10, 50), "w4"), ((17, 33, 1001), "w4"), ((3, 5, 7), "w4"), ((1, 16, 15), "w4"), ((16, 17, 1007), "w4"),
