@@ -265,9 +265,10 @@ uint64_t lten_hip_conv2d_dgrad_workspace_bytes(uint64_t N, uint64_t Cin, uint64_
  * bytes, 16-byte aligned.  Windows of at most 64 taps, and longer windows whose weights (of 32 output channels at
  * least) and a few input rows fit 64 KB of LDS, leave it untouched (it may be null): they run in one launch or, where
  * that is quicker, in two, an image's channels first laid out pixel by pixel (in three for the int32 sums of long windows
- * on small maps), in memory the library owns: at most 512 MB, or what one image takes (inside a graph recording only if that
- * memory exists already, otherwise in one launch; the bytes are the same).  Other windows use it: the input laid out pixel
- * by pixel beside the weights or, where that does not fit, the patches of all output positions of the batch as rows
+ * on small maps), in memory the library owns: at most 512 MB, or what one image takes (4 to 24 MB in one of three places
+ * that calls take in turn).  Inside a graph recording they do so only if that memory exists already, otherwise they run in
+ * one launch; the bytes are the same.  Other windows use the workspace: the input laid out pixel by pixel
+ * beside the weights or, where that does not fit, the patches of all output positions of the batch as rows
  * of a matrix, the padded weights, the int32 sums of one int8 GEMM over the whole batch and its zero-point terms;
  * where that would exceed 2 GiB, the column buffer of one image (l-ten's decomposition, image by image). */
 uint64_t lten_hip_conv2dq_workspace_bytes(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_t Cout,

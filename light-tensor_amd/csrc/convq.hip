@@ -408,6 +408,22 @@ static BatchedPlan batched_plan(const ConvGeo& g)
 
 constexpr uint64_t LIBRARY_LIMIT = 512ull << 20;  // library memory that a call fills, unless one image takes more
 
+// Library memory for the pixels of a call.  Where they about fill the L2s (4 MB in each of the eight XCDs, which all read some of
+// the same lines) writing what the call before has read is slow: three places take turns then (call after call, 3 x 3, 32 x 64 x 56 x
+// 56 -> 64 channels, 6.9 MB: 16.0 us in one place, 15.4 in two, 14.5 in three or more; 32 x 64 x 80 x 80 -> 64, 13.8 MB: 26.8 and
+// 23.2; 1 x 1, 64 x 64 x 64 x 64 -> 96, 16.8 MB: 26.4 and 23.0; of 3.8 MB and less and of 28 MB all the same).
+static void* pixels_memory(uint64_t bytes)
+{
+	constexpr unsigned places = 3;
+	static unsigned turn = 0;
+	const uint64_t place = align256(bytes);
+	if (bytes > (4ull << 20) && bytes <= (24ull << 20)) {
+		uint8_t* const all = static_cast<uint8_t*>(library_scratch(places * place));
+		if (all != nullptr) return all + turn++ % places * place;
+	}
+	return library_scratch(bytes);
+}
+
 static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_t Cout, int kh, int kw, int ph, int pw, int sh, int sw,
                        const uint8_t* x, const uint8_t* w, const int32_t* bias, const lten_hip_qparams* qp, void* y, bool out_acc,
                        void* workspace)
@@ -446,7 +462,7 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 				part.N = (int)std::max<uint64_t>(1, LIBRARY_LIMIT / ceil_div(bytes, N));
 				conv2dq_pixels_us(part, bytes);
 			}
-			void* const memory = one_launch ? library_scratch(bytes) : (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 ? workspace : nullptr;
+			void* const memory = one_launch ? pixels_memory(bytes) : (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 ? workspace : nullptr;
 			int rc = memory != nullptr ? 0 : -1;
 			for (int n = 0; n < g.N && rc == 0; n += part.N) {
 				ConvGeo now = g;

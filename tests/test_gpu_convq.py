@@ -295,3 +295,34 @@ def test_conv2dq_pixels_in_groups_of_images(gpu, ob):
     finally:
         gpu.set_option("conv_variant", 0)
     assert np.array_equal(dy.numpy(np.uint8, want.shape), want)
+
+
+def test_conv2dq_pixels_take_turns(gpu, ob):
+    """4 to 24 MB of pixels have three places that calls take in turn: calls one behind the other on inputs of their own, and two
+    recorded ones replayed between them."""
+    geo = (34, 16, 90, 90, 48, 1, 1, 0, 0, 1, 1)
+    rng = np.random.default_rng(34)
+    sc, zp = [0.02, 0.013, 0.06], [17, 125, 100]
+    w = rng.integers(0, 256, (48, 16, 1, 1), dtype=np.uint8)
+    xs = [rng.integers(0, 256, geo[:4], dtype=np.uint8) for _ in range(4)]
+    want = [ob.conv2dq_forward(geo, x, w, sc, zp)[0] for x in xs]
+    D, l, qp = gpu.DeviceBuffer, gpu.lib(), gpu.qparams3(sc, zp)
+    dw, dxs, dys = D.from_numpy(w), [D.from_numpy(x) for x in xs], [D(want[0].size) for _ in xs]
+    call = lambda i: gpu.check(l.lten_hip_conv2dq_forward(*geo, dxs[i].ptr, dw.ptr, None, qp, dys[i].ptr, None))
+    gpu.set_option("conv_variant", 12)
+    try:
+        call(0)
+        with gpu.Graph() as g:
+            call(0)
+            call(1)
+        assert gpu.last_kernel() == "conv2dq_pixels"
+        for rep in range(4):
+            for dy in dys:
+                gpu.check(l.lten_hip_fill_u8(dy.ptr, want[0].size, rep))
+            call(2)
+            g.launch()
+            call(3)
+            for i in range(4):
+                assert np.array_equal(dys[i].numpy(np.uint8, want[i].shape), want[i]), (rep, i)
+    finally:
+        gpu.set_option("conv_variant", 0)
