@@ -312,7 +312,8 @@ int qgemm_wave_dispatch(const QProblem& p, int out, int variant)
 
 // What each tile is expected to take (us): a start and an end, a k-step's share of the loads (a CU's vector L1 hands over
 // 40-odd bytes a clock; rows that start between cache lines take two lines a piece), more so the fuller the chip is, and
-// what each further round of workgroups adds.  Fitted to 240 shapes of 17 to 2048 rows, K and N of 512 to 8192 (10 % rms).
+// what each further round of workgroups adds.  Fitted to 240 shapes of 17 to 2048 rows, K and N of 512 to 8192, the weights in the
+// last-level cache (10 % rms).
 struct WaveTile {
 	int variant, bm, bn;
 	double start, per_k1024, lone, unaligned, round;
