@@ -6,8 +6,12 @@
 // inside a chunk over the taps of the window, one k-step of 16 channels each:
 //   LDS holds, for one chunk, every input position the tile's windows touch (the rows with their padding), as
 //   [octet of channels][piece][position][8 channels]: a matrix operand is the 16 bytes of (octet, piece) at a lane's own
-//   position, and another tap is another position, a constant further on.  So a value is loaded and converted once per
-//   tile and used under all taps (a column matrix holds it once per tap), whatever the window, the stride and the map.
+//   position, and another tap is another position.  So a value is loaded and converted once per tile and used under all taps
+//   (a column matrix holds it once per tap), whatever the window, the stride and the map.
+//   The rows of the patch are whole quads of positions: a staging thread loads 16 bytes, four positions of a row, for four
+//   channels (one position of eight channels took four times the load instructions, which cost 16 clocks each whatever their
+//   width).  Position 4 q + e lies in slot e Q + q of its plane, Q = 2 modulo 8: the writes of neighbouring quads are next to each
+//   other, and any eight consecutive positions, or eight that are two apart, fall on different banks.
 //   The weights are packed into pieces in operand order by a small launch before, [32 channels][chunk][tap][piece][lane][8],
 //   and go from the cache straight into registers, D k-steps ahead.
 // Half of the eight wavefronts of a workgroup (one per SIMD) only multiply, the other half only loads, converts and fills the
@@ -16,11 +20,14 @@
 // per CU walks over tiles, the chunks of the next tile staged under the last of this one.
 //
 // Measured (forward; fp32 matrix instructions or column matrices -> here): 32 x 32 x 128 x 128 -> 64 channels 3 x 3
-// 155 -> 108 us (180 TFLOP/s), 32 x 256 x 14 x 14 -> 256 81 -> 51, 16 x 64 x 57 x 57 -> 128 at stride 2 40 -> 25, 17 x 352 x
-// 50 x 50 -> 48 427 -> 99, 30 x 176 x 14 x 14 -> 320 5 x 5 205 -> 95.  Bound by the matrix cores at the clock the power
-// limit leaves (1.6 to 1.8 GHz, 70 % of the clocks in matrix instructions); then the stores at the end of a tile, which
-// all CUs reach together (32 KB to 128 KB a CU: 2 to 6 us), and the first chunk (1 to 5 us).  The weights one to three
-// k-steps ahead or five, and with half the traffic, made no difference.
+// 155 -> 111 us (174 TFLOP/s), 32 x 256 x 14 x 14 -> 256 81 -> 50, 16 x 64 x 57 x 57 -> 128 at stride 2 40 -> 22, 17 x 352 x
+// 50 x 50 -> 48 427 -> 90, 30 x 176 x 14 x 14 -> 320 5 x 5 205 -> 88.  One wavefront to a SIMD multiplies, so what stands
+// between two of its matrix instructions is lost: a k-step of the small tiles took 560 clocks of which 384 are matrix
+// instructions while the taps were counted between k-steps and operands read one block ahead, and takes 430 with the nine
+// taps of a 3 x 3 window written out, loads and reads each behind a matrix instruction and operands read two blocks ahead
+// (32 x 256 x 14 x 14 -> 256: 60 -> 50 us; 40 x 50 x 28 x 28 -> 150 46 -> 40, 64 x 256 x 7 x 7 -> 512 58 -> 51).
+// Bound by the matrix cores (clocks in matrix instructions: 75 to 85 % of the main loop, 2.1 to 2.3 GHz); then the stores at the
+// end of a tile, which all CUs reach together (32 KB to 128 KB a CU: 2 to 8 us at 4.2 TB/s), and the first chunk (3 to 4.5 us).
 //
 // 2-norm error against float64 over 22 layers each way, the routes before -> here: 0.31 to 0.5 of it in the tiles of four or
 // fewer blocks of 32 x 32, whose registers leave room for sums of their own (below), 0.8 to 0.9 in the tiles of eight; up to
@@ -40,6 +47,8 @@
 
 namespace lten_hip {
 
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));  // quads need not start on 16-byte boundaries
+
 namespace {
 
 constexpr int MAX_CLASSES = 4;
@@ -48,8 +57,9 @@ constexpr int MAX_CLASSES = 4;
 struct SplitClass {
 	int kh, kw, ph, pw, Ho, Wo;
 	int strip_w, strips;   // the columns of the map in strips, a tile lies in one
-	int patch_w;           // positions in a row of the patch
+	int patch_q;           // quads of positions in a row of the patch
 	int pixels, tiles_n;   // output pixels of a strip of the batch, their tiles
+	int step;              // pixels of a tile, at most BN
 	int first_tile;        // of the launch
 	int out_y, out_x;      // output pixel (oy, ox) is stored at (oy out_s + out_y, ox out_s + out_x)
 	int w0, wa, wb;        // tap (a, b) is weight w0 + a wa + b wb of its channels
@@ -59,6 +69,8 @@ struct SplitClass {
 struct SplitConv {
 	const float* x;
 	const float* w;
+	const float* src;   // what is staged: x, or a copy whose planes have four values
+	int plane;          // of src
 	const uint8_t* wp;
 	const float* bias;
 	float* y;
@@ -96,14 +108,25 @@ __global__ __launch_bounds__(256) void conv_split_pack_kernel(SplitConv p, uint8
 	for (int q = 0; q < 3; q++) *reinterpret_cast<uint4*>(out + q * 1024) = piece[q];
 }
 
-// U: 128 positions per octet that a staging thread can take, the patch holds up to PMAX positions.
-template <int BM, int BN, int WM, int WN, int U>
+// Planes of fewer than four values, a quad each (the last values repeat).
+__global__ __launch_bounds__(256) void pad_planes_kernel(const float* x, float* out, int planes, int hw)
+{
+	const int i = blockIdx.x * 256 + threadIdx.x;
+	if (i >= planes) return;
+#pragma unroll
+	for (int e = 0; e < 4; e++) out[4 * (int64_t)i + e] = x[(int64_t)i * hw + min(e, hw - 1)];
+}
+
+// Q: quads of positions that the patch holds (2 modulo 8, see the header).
+// T3: every class has 3 x 3 taps.
+template <int BM, int BN, int WM, int WN, int Q, bool T3>
 __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 {
-	constexpr int PMAX = U == 7 ? 832 : U * 128, PLANE = PMAX * 16, STAGE = 6 * PLANE;
+	constexpr int PLANE = 4 * Q * 16, STAGE = 6 * PLANE, U = (Q + 63) / 64;  // U: quads of a staging thread
 	constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
 	static_assert(WM * WN == 4 && FN % 2 == 0, "four multiplying wavefronts, column blocks in pairs");
-	constexpr int D = FM * FN == 8 ? 1 : FM * FN == 4 ? 2 : 3;  // k-steps the weights are loaded ahead
+	static_assert(Q % 8 == 2, "the four groups of quads lie 32 bytes apart modulo 128");
+	constexpr int D = FM * FN == 8 ? 1 : T3 || FM * FN == 4 ? 2 : 3;  // k-steps the weights are loaded ahead
 	__shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
 
 	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -125,7 +148,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 		t.m0 = (int)(r % (unsigned)p.tiles_m) * BM;
 		r /= (unsigned)p.tiles_m;
 		t.strip = (int)(r / (unsigned)c.tiles_n);
-		t.p0 = (int)(r - (unsigned)t.strip * c.tiles_n) * BN;
+		t.p0 = (int)(r - (unsigned)t.strip * c.tiles_n) * c.step;
 		const unsigned row = (unsigned)t.p0 / (unsigned)c.strip_w;
 		t.n0 = (int)(row / (unsigned)c.Ho);
 		t.ho0 = (int)row - t.n0 * c.Ho;
@@ -133,69 +156,95 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 	};
 
 	if (wave >= 4) {
-		// ---- the staging half: thread -> octet of channels, positions (threadIdx.x & 127) + 128 u
-		const int oct = wave >> 1 & 1, pos0 = threadIdx.x & 127;
-		const int64_t plane = (int64_t)p.H * p.W;
-		uint32_t off[U];           // of the item being loaded: byte offset of the position in channel 0
-		float raw[U][8];
-		unsigned inside = 0, inside_next = 0;
-		int count = 0, count_next = 0;  // positions of the tile
+		// ---- the staging half: wavefront -> octet of channels; thread -> four channels of it, quads quad0 + 64 u of positions
+		const int oct = wave >> 1 & 1, half = lane & 1, quad0 = (wave & 1) * 32 + (lane >> 1), ch0 = oct * 8 + half * 4;
+		uint32_t off[U];           // of the item being loaded: byte offset of the quad in channel 0
+		float raw[U][4][4];        // [channel][position]
+		unsigned inside = 0, inside_next = 0, turn = 0, turn_next = 0;
+		int quads = 0, quads_next = 0;  // of the tile's patch
 		auto place_loads = [&](int tile) {
 			const Place t = place_of(tile);
 			const SplitClass& c = p.cls[t.cls];
-			const int last = min(t.p0 + BN, c.pixels) - 1;
+			const int last = min(t.p0 + c.step, c.pixels) - 1;
 			const int row_l = last / c.strip_w, n_l = row_l / c.Ho, ho_l = row_l - n_l * c.Ho;
 			const int first_rows = (c.Ho - 1 - t.ho0) * p.sh + c.kh, full_rows = (c.Ho - 1) * p.sh + c.kh;
 			const int rows = n_l == t.n0 ? (ho_l - t.ho0) * p.sh + c.kh : first_rows + (n_l - t.n0 - 1) * full_rows + ho_l * p.sh + c.kh;
-			count_next = rows * c.patch_w;
-			inside_next = 0;
+			quads_next = rows * c.patch_q;
+			inside_next = turn_next = 0;
 			const int x0 = t.strip * c.strip_w * p.sw - c.pw, y0 = t.ho0 * p.sh - c.ph;
 #pragma unroll
 			for (int u = 0; u < U; u++) {
-				const unsigned pos = (unsigned)pos0 + 128 * u;
-				const unsigned r = pos / (unsigned)c.patch_w, q = pos - r * c.patch_w;
+				const unsigned quad = (unsigned)quad0 + 64 * u;
+				const unsigned r = quad / (unsigned)c.patch_q, q = quad - r * c.patch_q;
 				int n = t.n0, yy = y0 + (int)r;
 				if ((int)r >= first_rows) {
 					const unsigned k = (r - (unsigned)first_rows) / (unsigned)full_rows;
 					n += 1 + (int)k;
 					yy = (int)(r - first_rows - k * full_rows) - c.ph;
 				}
-				const int xx = x0 + (int)q;
-				const bool in = (int)pos < count_next && (unsigned)yy < (unsigned)p.H && (unsigned)xx < (unsigned)p.W && n < p.N;
-				off[u] = in ? (uint32_t)(((unsigned)n * p.C * (unsigned)p.H + (unsigned)yy) * (unsigned)p.W + (unsigned)xx) * 4u : 0u;
-				inside_next |= (unsigned)in << u;
+				const int xx = x0 + 4 * (int)q;
+				unsigned in = 0;
+				if ((int)quad < quads_next && (unsigned)yy < (unsigned)p.H && n < p.N) {
+#pragma unroll
+					for (int e = 0; e < 4; e++) in |= (unsigned)((unsigned)(xx + e) < (unsigned)p.W) << e;
+				}
+				// a quad that reaches past the ends of the map's plane is loaded from the plane's first or last four values and
+				// turned in registers
+				const int at = yy * p.W + xx, clamped = min(max(at, 0), p.plane - 4);
+				off[u] = in ? ((unsigned)n * p.C * (unsigned)p.plane + (unsigned)clamped) * 4u : 0u;
+				inside_next |= in << (4 * u);
+				turn_next |= (in ? (unsigned)(at - clamped) & 3u : 0u) << (2 * u);
 			}
 		};
 		// (every load is issued whatever the position: a load under a condition would make each wait one for all)
 		auto load = [&](int u, int chunk) {
 #pragma unroll
-			for (int e = 0; e < 8; e++) {
-				const char* base = reinterpret_cast<const char*>(p.x + (int64_t)min(chunk * 16 + oct * 8 + e, p.C - 1) * plane);
-				raw[u][e] = *reinterpret_cast<const float*>(base + off[u]);
+			for (int e = 0; e < 4; e++) {
+				const char* base = reinterpret_cast<const char*>(p.src + (int64_t)min(chunk * 16 + ch0 + e, p.C - 1) * p.plane);
+				const f4_any v = *reinterpret_cast<const f4_any*>(base + off[u]);
+				raw[u][e][0] = v.x; raw[u][e][1] = v.y; raw[u][e][2] = v.z; raw[u][e][3] = v.w;
 			}
 		};
-		auto convert = [&](int u, int chunk, int stage) {
-			const int pos = pos0 + 128 * u;
-			if (pos >= count) return;
-			float v[8];
-			const bool in = inside >> u & 1;
+		// (channels past the end repeat the last one: their weights are zero)
+		auto convert = [&](int u, int stage) {
+			const int quad = quad0 + 64 * u;
+			if (quad >= quads) return;
+			if (__any(turn >> (2 * u) & 3u)) {
+				const bool by1 = turn >> (2 * u) & 1u, by2 = turn >> (2 * u) & 2u;
 #pragma unroll
-			for (int e = 0; e < 8; e++) v[e] = in && chunk * 16 + oct * 8 + e < p.C ? raw[u][e] : 0.0f;
-			uint4 piece[3];
-			split8(v, piece);
-			uint8_t* d = smem + stage * STAGE + oct * 3 * PLANE + pos * 16;
+				for (int e = 0; e < 4; e++) {
+					float(&r)[4] = raw[u][e];
+					const float a0 = by1 ? r[1] : r[0], a1 = by1 ? r[2] : r[1], a2 = by1 ? r[3] : r[2], a3 = by1 ? r[0] : r[3];
+					r[0] = by2 ? a2 : a0; r[1] = by2 ? a3 : a1; r[2] = by2 ? a0 : a2; r[3] = by2 ? a1 : a3;
+				}
+			}
+			uint8_t* d = smem + stage * STAGE + oct * 3 * PLANE + quad * 16 + half * 8;
 #pragma unroll
-			for (int q = 0; q < 3; q++) *reinterpret_cast<uint4*>(d + q * PLANE) = piece[q];
+			for (int e = 0; e < 4; e++) {
+				// a position outside the map counts as zeros: the scale is zero there (an infinity times it is a NaN, and the tile
+				// is computed again on the values themselves)
+				const float scale = __builtin_bit_cast(float, (uint32_t)((int)(inside << (31 - 4 * u - e)) >> 31) & __builtin_bit_cast(uint32_t, pieces_scale));
+				float v[4];
+#pragma unroll
+				for (int k = 0; k < 4; k++) v[k] = raw[u][k][e] * scale;
+				uint2 piece[3];
+				piece[0].x = split_off(v[0], v[1]); piece[0].y = split_off(v[2], v[3]);
+				piece[1].x = split_off(v[0], v[1]); piece[1].y = split_off(v[2], v[3]);
+				piece[2].x = split_last(v[0], v[1]); piece[2].y = split_last(v[2], v[3]);
+#pragma unroll
+				for (int k = 0; k < 3; k++) *reinterpret_cast<uint2*>(d + k * PLANE + e * Q * 16) = piece[k];
+			}
 		};
-		int ld_tile = tile0, ld_chunk = 0, cv_chunk = 0;
+		int ld_tile = tile0, ld_chunk = 0;
 		place_loads(tile0);
 #pragma unroll
 		for (int u = 0; u < U; u++) load(u, 0);
 		for (int it = -1; it < items; it++) {
 			// convert item it + 1, load item it + 2 (past the last one: loaded again, not converted)
 			const bool have = it + 1 < items;
-			count = have ? count_next : 0;
+			quads = have ? quads_next : 0;
 			inside = inside_next;
+			turn = turn_next;
 			if (it + 2 < items) {
 				if (++ld_chunk == p.chunks) {
 					ld_chunk = 0;
@@ -206,10 +255,9 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 			const int stage = (it + 1) & 1;
 #pragma unroll
 			for (int u = 0; u < U; u++) {
-				convert(u, cv_chunk, stage);
+				convert(u, stage);
 				load(u, ld_chunk);
 			}
-			if (++cv_chunk == p.chunks) cv_chunk = 0;
 			__syncthreads();
 		}
 		return;
@@ -218,7 +266,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 	// ---- the multiplying half
 	__builtin_amdgcn_s_setprio(1);
 	const int wm = wave / WN, wn = wave % WN, lrow = lane & 31, lk = lane >> 5;
-	const uint32_t lane16 = lane * 16;
+	const uint32_t lane16 = lane * 16, lk3 = lk * 3 * PLANE;
 	__syncthreads();  // stage 0 holds the first chunk
 
 	int stage = 0;
@@ -227,28 +275,30 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 		const SplitClass& c = p.cls[t.cls];
 		// (through readfirstlane: kept in registers instead of loaded again in the loop)
 		const int kh = __builtin_amdgcn_readfirstlane(c.kh), kw = __builtin_amdgcn_readfirstlane(c.kw);
-		const int row_step = __builtin_amdgcn_readfirstlane((c.patch_w - c.kw) * 16);
+		const int row_step = __builtin_amdgcn_readfirstlane((4 * c.patch_q - c.kw) * 4);
 		const int total = p.chunks * kh * kw;
 		const int first_rows = (c.Ho - 1 - t.ho0) * p.sh + c.kh, full_rows = (c.Ho - 1) * p.sh + c.kh;
-		// the lane's column of each block: position in the patch, place in the output (-1: none)
+		// the lane's column of each block: four times its position in the patch, place in the output (-1: none)
 		uint32_t vb[FN];
 		int out[FN];
 #pragma unroll
 		for (int j = 0; j < FN; j++) {
 			const int px = t.p0 + wn * TN + j * 32 + lrow;
-			const unsigned pc = (unsigned)min(px, c.pixels - 1), row = pc / (unsigned)c.strip_w, wo = pc - row * c.strip_w;
+			const int end = min(t.p0 + c.step, c.pixels);
+			const unsigned pc = (unsigned)min(px, end - 1), row = pc / (unsigned)c.strip_w, wo = pc - row * c.strip_w;
 			const unsigned n = row / (unsigned)c.Ho, ho = row - n * c.Ho;
 			const int r = (int)n == t.n0 ? ((int)ho - t.ho0) * p.sh : first_rows + ((int)n - t.n0 - 1) * full_rows + (int)ho * p.sh;
-			vb[j] = (uint32_t)((r * c.patch_w + (int)wo * p.sw) * 16 + lk * 3 * PLANE);
+			vb[j] = (uint32_t)((r * 4 * c.patch_q + (int)wo * p.sw) * 4);
 			const int ox = t.strip * c.strip_w + (int)wo;
-			out[j] = px < c.pixels && ox < c.Wo ? (int)(((int64_t)n * p.M + t.m0 + wm * TM) * p.out_plane) + ((int)ho * p.out_s + c.out_y) * p.out_w + ox * p.out_s + c.out_x : -1;
+			out[j] = px < end && ox < c.Wo ? (int)(((int64_t)n * p.M + t.m0 + wm * TM) * p.out_plane) + ((int)ho * p.out_s + c.out_y) * p.out_w + ox * p.out_s + c.out_x : -1;
 		}
 		const uint8_t* wb[FM];
+		const int64_t packed = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)c.packed) | (uint64_t)__builtin_amdgcn_readfirstlane((int)(c.packed >> 32)) << 32);
 #pragma unroll
 		for (int i = 0; i < FM; i++) {
 			// (blocks of 32 channels past the last one: read the last one again, never stored)
-			const int block = min(t.m0 / 32 + wm * FM + i, (p.M + 31) / 32 - 1);
-			wb[i] = p.wp + c.packed + (int64_t)block * total * 3072;
+			const int block = __builtin_amdgcn_readfirstlane(min(t.m0 / 32 + wm * FM + i, (p.M + 31) / 32 - 1));
+			wb[i] = p.wp + packed + (int64_t)block * total * 3072;
 		}
 
 		// register 4q + e of block (i, j) of lane (lrow, lk): channel i * 32 + 8q + 4 lk + e, column j * 32 + lrow of the
@@ -267,70 +317,173 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 #pragma unroll
 				for (int r = 0; r < 16; r++) acc[i][j][r] = low[APART ? i : 0][APART ? j : 0][r] = 0.0f;
 
-		bf16x8 fa[D + 1][FM][3], fb[2][3];
-		auto load_a = [&](int set, int s) {
-			const int at = min(s, total - 1) * 3072;
+		// Operands of column blocks are read DB blocks ahead: with one row block to a column block its six matrix instructions are
+		// over before an LDS read that queues behind the staging half's writes has come back.
+		constexpr int DB = FM == 1 ? 2 : 1, SETS = FM == 2 ? 2 : D == 2 ? 3 : 4;
+		static_assert((T3 ? 9 : D + 1) * FN % SETS == 0 && SETS > DB, "a block's operand set is the same in every round of k-steps");
+		bf16x8 fa[D + 1][FM][3], fb[SETS][3];
+		// (the loads run up to D k-steps past a block: into the next one, or what the buffer has behind the last one)
+		uint32_t a_at = 0;
+		auto load_a = [&](int set, int i, int v) { fa[set][i][v] = *reinterpret_cast<const bf16x8*>(wb[i] + (uint32_t)(lane16 + a_at) + v * 1024); };
+		auto next_a = [&]() {
+			a_at += 3072;
+			asm volatile("" : "+s"(a_at));  // (a scalar, not a pointer of every lane)
+		};
+		// position 4 q + e lies in slot e Q + q of its plane; tap4: four times the tap's place in the patch, at: the stage
+		auto slot_of = [&](int j, uint32_t tap4, uint32_t at) {
+			const uint32_t t = vb[j] + tap4;
+			uint32_t slot = __umul24(t & 12u, 4 * Q - 1) + t + at + lk3;
+			asm volatile("" : "+v"(slot));  // (a multiple of 16, which its parts are not)
+			return slot;
+		};
+		auto read_b = [&](int set, uint32_t slot, int v) { fb[set][v] = *reinterpret_cast<const bf16x8*>(smem + slot + v * PLANE); };
+#pragma unroll
+		for (int d = 0; d < D; d++) {
 #pragma unroll
 			for (int i = 0; i < FM; i++)
 #pragma unroll
-				for (int v = 0; v < 3; v++) fa[set][i][v] = *reinterpret_cast<const bf16x8*>(wb[i] + at + lane16 + v * 1024);
-		};
-		auto read_b = [&](int set, int j, uint32_t at, int v) { fb[set][v] = *reinterpret_cast<const bf16x8*>(smem + vb[j] + at + v * PLANE); };
-#pragma unroll
-		for (int d = 0; d < D; d++) load_a(d, d);
-		uint32_t at = stage * STAGE;  // of the tap in the stage
-#pragma unroll
-		for (int v = 0; v < 3; v++) read_b(0, 0, at, v);
-		int tb = 0, ta = 0, s = 0;
-		// One k-step: the matrix instructions of every column block, the operands of the next block read under them; the last
-		// block's run while the operands of the next k-step arrive, behind a barrier where that is the next chunk's.
-		auto k_step = [&](auto par_c) {
-			constexpr int PAR = decltype(par_c)::value;
-			uint32_t next_at = at + 16;
-			bool chunk_end = false;
-			if (++tb == kw) {
-				tb = 0;
-				next_at += row_step;
-				if (++ta == kh) {
-					ta = 0;
-					chunk_end = true;
-				}
-			}
-#pragma unroll
-			for (int j = 0; j < FN; j++) {
-				const bool last = j == FN - 1;
-				if (last && chunk_end) {
-					__syncthreads();
-					stage ^= 1;
-					next_at = stage * STAGE;
-				}
-#pragma unroll
-				for (int q = 0; q < 6 * FM; q++) {
-					const int i = q % FM, qq = q / FM;
-					v16f& sum = APART && qq < 5 ? low[APART ? i : 0][APART ? j : 0] : acc[i][j];
-					sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[PAR][i][piece_a[qq]], fb[j & 1][piece_b[qq]], sum, 0, 0, 0);
-					if (j == 0 && q == 0) load_a((PAR + D) % (D + 1), s + D);
-					if (q < 3) read_b((j + 1) & 1, last ? 0 : j + 1, last ? next_at : at, q);
-					__builtin_amdgcn_sched_barrier(0);
-				}
-			}
-			at = next_at;
-		};
-		using S0 = std::integral_constant<int, 0>;
-		using S1 = std::integral_constant<int, 1>;
-		using S2 = std::integral_constant<int, D >= 2 ? 2 : 0>;
-		using S3 = std::integral_constant<int, D >= 3 ? 3 : 0>;
-		while (s + D < total) {
-			k_step(S0{}); s++;
-			k_step(S1{}); s++;
-			if (D >= 2) { k_step(S2{}); s++; }
-			if (D >= 3) { k_step(S3{}); s++; }
+				for (int v = 0; v < 3; v++) load_a(d, i, v);
+			next_a();
 		}
-		if (s < total) {
-			k_step(S0{});
-			if (D >= 2 && ++s < total) {
+		if constexpr (T3) {
+			// Nine k-steps to a chunk, written out.  (With the taps counted at run time the scalar instructions between two k-steps
+			// took the pipe 60 to 110 clocks of 384.)  Where registers are left, the addresses of a row's taps are kept.
+			constexpr bool KEPT = FM * FN == 2;
+			uint32_t slot3[KEPT ? FN : 1][3];
+			if (KEPT) {
+#pragma unroll
+				for (int j = 0; j < FN; j++)
+#pragma unroll
+					for (int b = 0; b < 3; b++) {
+						slot3[KEPT ? j : 0][b] = slot_of(j, 4 * b, 0);
+						asm volatile("" : "+v"(slot3[KEPT ? j : 0][b]));
+					}
+			}
+			const uint32_t row_bytes = 16 * (uint32_t)__builtin_amdgcn_readfirstlane(c.patch_q);
+			auto opaque = [](uint32_t v) {  // (what hangs on it is worked out where it is used, not kept in registers)
+				asm volatile("" : "+s"(v));
+				return v;
+			};
+			auto slot_at = [&](int j, int tap, uint32_t at) { return KEPT ? slot3[KEPT ? j : 0][tap % 3] + (at + tap / 3 * row_bytes) : slot_of(j, opaque(4 * (tap % 3)), at + tap / 3 * row_bytes); };
+			uint32_t stage_at = stage * STAGE;
+#pragma unroll
+			for (int b = 0; b < DB; b++)
+#pragma unroll
+				for (int v = 0; v < 3; v++) read_b(b, slot_at(b, 0, stage_at), v);
+			auto k_step = [&](auto phase_c, auto tap_c) {
+				constexpr int TAP = decltype(tap_c)::value, NEXT = (TAP + 1) % 9, SET = (TAP + decltype(phase_c)::value) % (D + 1), FIRST = TAP * FN;
+#pragma unroll
+				for (int j = 0; j < FN; j++) {
+					const bool ahead = j >= FN - DB;  // the block that is read is of the next k-step
+					uint32_t slot = 0;
+#pragma unroll
+					for (int q = 0; q < 6 * FM; q++) {
+						const int i = q % FM, qq = q / FM;
+						v16f& sum = APART && qq < 5 ? low[APART ? i : 0][APART ? j : 0] : acc[i][j];
+						sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[SET][i][piece_a[qq]], fb[(FIRST + j) % SETS][piece_b[qq]], sum, 0, 0, 0);
+						__builtin_amdgcn_sched_barrier(0);
+						if (q == 0) {
+							if (TAP == 8 && j == FN - DB) {  // the next k-step is the next chunk's
+								__syncthreads();
+								stage_at = STAGE - stage_at;
+							}
+							slot = slot_at(ahead ? j + DB - FN : j + DB, ahead ? NEXT : TAP, stage_at);
+						}
+						if (q >= 1 && q < 4) read_b((FIRST + j + DB) % SETS, slot, q - 1);
+						if (j < FM && q >= 3 && q < 6) load_a((SET + D) % (D + 1), j, q - 3);
+						if (j == FN - 1 && q == 6 * FM - 2) next_a();
+						__builtin_amdgcn_sched_barrier(0);
+					}
+				}
+			};
+			auto chunk = [&](auto phase_c) {
+				k_step(phase_c, std::integral_constant<int, 0>{});
+				k_step(phase_c, std::integral_constant<int, 1>{});
+				k_step(phase_c, std::integral_constant<int, 2>{});
+				k_step(phase_c, std::integral_constant<int, 3>{});
+				k_step(phase_c, std::integral_constant<int, 4>{});
+				k_step(phase_c, std::integral_constant<int, 5>{});
+				k_step(phase_c, std::integral_constant<int, 6>{});
+				k_step(phase_c, std::integral_constant<int, 7>{});
+				k_step(phase_c, std::integral_constant<int, 8>{});
+			};
+			for (int left = p.chunks;;) {
+				chunk(std::integral_constant<int, 0>{});
+				if (--left == 0) break;
+				if (9 % (D + 1) != 0) {
+					chunk(std::integral_constant<int, 9 % (D + 1)>{});
+					if (--left == 0) break;
+				}
+			}
+			stage = stage_at != 0;
+		} else {
+#pragma unroll
+			for (int b = 0; b < DB; b++)
+#pragma unroll
+				for (int v = 0; v < 3; v++) read_b(b, slot_of(b, 0, stage * STAGE), v);
+			// The tap of this k-step and of the next one, and whether that is the next chunk's: worked out under the matrix
+			// instructions of the k-step before.
+			int tb = 0, ta = 0, s = 0;
+			uint32_t tap4 = 0, next_tap4 = 0;
+			bool chunk_end = false;
+			auto advance = [&]() {
+				const bool row_end = tb == kw - 1;
+				chunk_end = row_end & (ta == kh - 1);
+				next_tap4 = chunk_end ? 0u : tap4 + 4 + (row_end ? (uint32_t)row_step : 0u);
+				ta = chunk_end ? 0 : ta + (int)row_end;
+				tb = row_end ? 0 : tb + 1;
+			};
+			advance();
+			// One k-step: the matrix instructions of every column block, the operands of a later block read under them, those of the
+			// next k-step's first blocks behind a barrier where that is the next chunk's.  Everything else stands behind a matrix
+			// instruction too: between two k-steps it left the pipe empty for 110 clocks.
+			auto k_step = [&](auto par_c) {
+				constexpr int PAR = decltype(par_c)::value, FIRST = PAR * FN;
+#pragma unroll
+				for (int j = 0; j < FN; j++) {
+					const bool ahead = j >= FN - DB;  // the block that is read is of the next k-step
+					uint32_t slot = 0;
+#pragma unroll
+					for (int q = 0; q < 6 * FM; q++) {
+						const int i = q % FM, qq = q / FM;
+						v16f& sum = APART && qq < 5 ? low[APART ? i : 0][APART ? j : 0] : acc[i][j];
+						sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[PAR][i][piece_a[qq]], fb[(FIRST + j) % SETS][piece_b[qq]], sum, 0, 0, 0);
+						__builtin_amdgcn_sched_barrier(0);
+						if (q == 0) {
+							if (j == FN - DB && chunk_end) {
+								__syncthreads();
+								stage ^= 1;
+							}
+							slot = slot_of(ahead ? j + DB - FN : j + DB, ahead ? next_tap4 : tap4, stage * STAGE);
+						}
+						if (q >= 1 && q < 4) read_b((FIRST + j + DB) % SETS, slot, q - 1);
+						if (j < FM && q >= 3 && q < 6) load_a((PAR + D) % (D + 1), j, q - 3);
+						if (j == FN - 1 && q == 6 * FM - 2) {
+							next_a();
+							tap4 = next_tap4;
+							advance();
+							s++;
+						}
+						__builtin_amdgcn_sched_barrier(0);
+					}
+				}
+			};
+			using S0 = std::integral_constant<int, 0>;
+			using S1 = std::integral_constant<int, 1>;
+			using S2 = std::integral_constant<int, D >= 2 ? 2 : 0>;
+			using S3 = std::integral_constant<int, D >= 3 ? 3 : 0>;
+			while (s + D < total) {
+				k_step(S0{});
 				k_step(S1{});
-				if (D >= 3 && ++s < total) k_step(S2{});
+				if (D >= 2) k_step(S2{});
+				if (D >= 3) k_step(S3{});
+			}
+			if (s < total) {
+				k_step(S0{});
+				if (D >= 2 && s < total) {
+					k_step(S1{});
+					if (D >= 3 && s < total) k_step(S2{});
+				}
 			}
 		}
 
@@ -355,7 +508,8 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 #pragma unroll 1
 			for (int ij = 0; ij < FM * FN; ij++) {
 				const int i = ij / FN, j = ij % FN, px = t.p0 + wn * TN + j * 32 + lrow;
-				const unsigned pc = (unsigned)min(px, c.pixels - 1), row = pc / (unsigned)c.strip_w, n = row / (unsigned)c.Ho;
+				const int end = min(t.p0 + c.step, c.pixels);
+				const unsigned pc = (unsigned)min(px, end - 1), row = pc / (unsigned)c.strip_w, n = row / (unsigned)c.Ho;
 				const int oy = (int)(row - n * c.Ho), ox = t.strip * c.strip_w + (int)(pc - row * c.strip_w);
 				const int yy = oy * p.sh - c.ph, xx = ox * p.sw - c.pw, co = t.m0 + wm * TM + i * 32;
 				const float* wr = p.w + c.w0 + (int64_t)min(co + lrow, p.M - 1) * p.w_co;
@@ -385,7 +539,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 #pragma unroll
 				for (int r = 0; r < 16; r++) {
 					const int m = co + (r >> 2) * 8 + 4 * lk + (r & 3);
-					if (m < p.M && px < c.pixels && ox < c.Wo)
+					if (m < p.M && px < end && ox < c.Wo)
 						p.y[((int64_t)n * p.M + m) * p.out_plane + (oy * p.out_s + c.out_y) * p.out_w + ox * p.out_s + c.out_x] = sum[r] + (p.bias ? p.bias[m] : 0.0f);
 				}
 			}
@@ -418,21 +572,26 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 
 namespace {
 
-// The tiles, with what a k-step of a wavefront multiplies (blocks of 32 x 32) and the positions a patch may have.
+// The tiles, with what a k-step of a wavefront multiplies (blocks of 32 x 32), the quads of positions a patch may have, and what
+// a matrix instruction and the rest of a round of tiles take (fitted to 28 convolutions each, which it meets within 15 %).
 struct SplitTile {
-	int BM, BN, blocks, U, pmax;
+	int BM, BN, blocks, quads;
+	double mfma_ns, round_us;
 };
 const SplitTile split_tiles[] = {
-	{ 64, 512, 8, 7, 832 }, { 32, 512, 4, 7, 832 }, { 128, 256, 8, 5, 640 }, { 64, 256, 4, 5, 640 },
-	{ 32, 256, 2, 5, 640 }, { 64, 128, 2, 3, 384 }, { 64, 128, 2, 7, 832 },
+	{ 64, 512, 8, 210, 15.1, 16.0 }, { 32, 512, 4, 210, 15.8, 7.5 }, { 128, 256, 8, 162, 15.0, 12.0 }, { 64, 256, 4, 162, 17.9, 8.2 },
+	{ 32, 256, 2, 162, 20.7, 2.7 }, { 64, 128, 2, 98, 19.2, 3.3 }, { 64, 128, 2, 210, 20.3, 3.3 },
 };
 constexpr int SPLIT_TILES = sizeof(split_tiles) / sizeof(split_tiles[0]);
 
-template <int BM, int BN, int WM, int WN, int U>
-void launch_split(const SplitConv& p)
+template <int BM, int BN, int WM, int WN, int Q>
+void launch_split(const SplitConv& p, bool t3)
 {
 	const unsigned per_xcd = (unsigned)((p.tiles + 7) / 8);
-	conv_split_kernel<BM, BN, WM, WN, U><<<dim3(8 * std::min(32u, per_xcd)), dim3(512), 0, stream()>>>(p);
+	const dim3 grid(8 * std::min(32u, per_xcd));
+	constexpr bool T3 = BM / WM / 32 * (BN / WN / 32) < 8;  // (with eight blocks the registers do not hold out)
+	if (T3 && t3) conv_split_kernel<BM, BN, WM, WN, Q, T3><<<grid, dim3(512), 0, stream()>>>(p);
+	else conv_split_kernel<BM, BN, WM, WN, Q, false><<<grid, dim3(512), 0, stream()>>>(p);
 }
 
 // Lays the classes out in strips and tiles of the given kind; false when a patch would not fit.
@@ -442,25 +601,27 @@ bool split_layout(SplitConv& p, const SplitTile& t)
 	uint64_t tiles = 0;
 	for (int k = 0; k < p.classes; k++) {
 		SplitClass& c = p.cls[k];
-		// strips of at most 128 columns, more and narrower ones where a patch would not fit
+		// strips of at most 128 columns, more and narrower ones where a patch would not fit; where none does, tiles of fewer pixels
 		const int first = (int)ceil_div((uint64_t)c.Wo, 128);
 		int64_t pixels = 0;
 		bool fits = false;
-		for (int strips = first; strips < first + 4 && !fits; strips++) {
-			c.strips = strips;
-			c.strip_w = (int)ceil_div((uint64_t)c.Wo, (uint64_t)strips);
-			c.patch_w = (c.strip_w - 1) * p.sw + c.kw;
-			pixels = (int64_t)p.N * c.Ho * c.strip_w;
-			if (pixels >= (1ll << 30)) return false;
-			// the most rows and images that BN consecutive pixels touch (tiles start at multiples of BN)
-			const int64_t w = c.strip_w, all_rows = (int64_t)p.N * c.Ho;
-			const int64_t rows = std::min(all_rows, t.BN % w == 0 ? t.BN / w : w % t.BN == 0 ? 1 : (t.BN - 2) / w + 2);
-			const int64_t images = std::min<int64_t>(p.N, t.BN % w == 0 && c.Ho % rows == 0 ? 1 : t.BN % w == 0 && rows % c.Ho == 0 ? rows / c.Ho : (rows - 2 + c.Ho) / c.Ho + 1);
-			fits = ((rows - images) * p.sh + images * std::max(c.kh, p.sh)) * c.patch_w <= t.pmax;
-		}
+		for (c.step = t.BN; c.step >= t.BN / 2 && !fits; c.step -= 16)
+			for (int strips = first; strips < first + 4 && !fits; strips++) {
+				c.strips = strips;
+				c.strip_w = (int)ceil_div((uint64_t)c.Wo, (uint64_t)strips);
+				c.patch_q = ((c.strip_w - 1) * p.sw + c.kw + 3) / 4;
+				pixels = (int64_t)p.N * c.Ho * c.strip_w;
+				if (pixels >= (1ll << 30)) return false;
+				// the most rows and images that `step` consecutive pixels touch (tiles start at multiples of it)
+				const int64_t w = c.strip_w, all_rows = (int64_t)p.N * c.Ho, step = c.step;
+				const int64_t rows = std::min(all_rows, step % w == 0 ? step / w : w % step == 0 ? 1 : (step - 2) / w + 2);
+				const int64_t images = std::min<int64_t>(p.N, step % w == 0 && c.Ho % rows == 0 ? 1 : step % w == 0 && rows % c.Ho == 0 ? rows / c.Ho : (rows - 2 + c.Ho) / c.Ho + 1);
+				fits = ((rows - images) * p.sh + images * std::max(c.kh, p.sh)) * c.patch_q <= t.quads;
+			}
+		c.step += 16;  // (as the loop left it)
 		if (!fits) return false;
 		c.pixels = (int)pixels;
-		c.tiles_n = (int)ceil_div((uint64_t)pixels, (uint64_t)t.BN);
+		c.tiles_n = (int)ceil_div((uint64_t)pixels, (uint64_t)c.step);
 		if (tiles > (1ull << 28)) return false;
 		c.first_tile = (int)tiles;
 		tiles += (uint64_t)c.tiles_n * c.strips * p.tiles_m;
@@ -470,15 +631,23 @@ bool split_layout(SplitConv& p, const SplitTile& t)
 	return true;
 }
 
-// What a launch takes, in us: rounds of tiles on 256 CUs, a chunk as long as its matrix instructions (32 clocks each, 46
-// with the waits between) or its staging, a tile's start and store, the two launches; at the clock the chip holds.
+bool split_t3(const SplitConv& p)
+{
+	for (int k = 0; k < p.classes; k++)
+		if (p.cls[k].kh != 3 || p.cls[k].kw != 3) return false;
+	return true;
+}
+
+// What a launch takes, in us: the two launches, rounds of tiles on 256 CUs; a chunk as long as its matrix instructions (taps that
+// are counted at run time cost 10 % more) or its staging (9.5 ns a quad); the start and the store of a tile.  Classes of one to four
+// taps switch between the two limits and store every other pixel.
 double split_us(const SplitConv& p, const SplitTile& t)
 {
-	double taps = 0;
-	for (int k = 0; k < p.classes; k++) taps += (double)p.cls[k].kh * p.cls[k].kw / p.classes;
-	const double rounds = (double)ceil_div(ceil_div((uint64_t)p.tiles, 8), 32);
-	const double chunk = std::max(taps * 6 * t.blocks * 46.0, t.U * 900.0);
-	return 8.0 + rounds * (p.chunks * chunk + 3000.0 + t.blocks * 2500.0) / 1750.0;
+	const double rounds = (double)ceil_div(ceil_div((uint64_t)p.tiles, 8), 32), slower = split_t3(p) ? 1.0 : 1.1;
+	double chunk_us = 0;
+	for (int k = 0; k < p.classes; k++) chunk_us += std::max(p.cls[k].kh * p.cls[k].kw * 6e-3 * t.blocks * t.mfma_ns * slower, t.quads * 9.5e-3) / p.classes;
+	if (p.classes > 1) return 9.0 + rounds * (p.chunks * chunk_us * (t.blocks == 8 ? 1.6 : 1.25) + t.round_us * 1.4);
+	return 9.0 + rounds * (p.chunks * chunk_us + t.round_us);
 }
 
 // Fills in the sizes that are common to all classes, packs the weights and launches; -1 when no tile takes the shape, the
@@ -511,19 +680,30 @@ int split_run(SplitConv& p, double limit_us, int forced)
 	}
 	int tap_groups = 1;
 	for (int k = 0; k < p.classes; k++) tap_groups = std::max(tap_groups, (p.cls[k].kh * p.cls[k].kw + 3) / 4);
-	uint8_t* scratch = static_cast<uint8_t*>(library_scratch((uint64_t)packed));
+	packed += 3 * 3072;  // (read, not used, where the last block's loads run ahead)
+	const int hw = p.H * p.W;
+	p.src = p.x;
+	p.plane = std::max(hw, 4);
+	uint8_t* scratch = static_cast<uint8_t*>(library_scratch((uint64_t)packed + (hw < 4 ? 16ull * p.N * p.C : 0)));
 	if (scratch == nullptr) return -1;
+	if (hw < 4) {  // planes of less than a quad: one each in a copy
+		float* copy = reinterpret_cast<float*>(scratch + packed);
+		pad_planes_kernel<<<dim3((unsigned)ceil_div((uint64_t)p.N * p.C, 256)), dim3(256), 0, stream()>>>(p.x, copy, p.N * p.C, hw);
+		LTEN_HIP_LAUNCH_CHECK();
+		p.src = copy;
+	}
 	conv_split_pack_kernel<<<dim3((unsigned)p.chunks, (unsigned)cobs, (unsigned)(p.classes * tap_groups)), dim3(256), 0, stream()>>>(p, scratch);
 	LTEN_HIP_LAUNCH_CHECK();
 	p.wp = scratch;
+	const bool t3 = split_t3(p);
 	switch (best) {
-	case 0: launch_split<64, 512, 1, 4, 7>(p); break;
-	case 1: launch_split<32, 512, 1, 4, 7>(p); break;
-	case 2: launch_split<128, 256, 2, 2, 5>(p); break;
-	case 3: launch_split<64, 256, 1, 4, 5>(p); break;
-	case 4: launch_split<32, 256, 1, 4, 5>(p); break;
-	case 5: launch_split<64, 128, 2, 2, 3>(p); break;
-	default: launch_split<64, 128, 2, 2, 7>(p); break;
+	case 0: launch_split<64, 512, 1, 4, 210>(p, t3); break;
+	case 1: launch_split<32, 512, 1, 4, 210>(p, t3); break;
+	case 2: launch_split<128, 256, 2, 2, 162>(p, t3); break;
+	case 3: launch_split<64, 256, 1, 4, 162>(p, t3); break;
+	case 4: launch_split<32, 256, 1, 4, 162>(p, t3); break;
+	case 5: launch_split<64, 128, 2, 2, 98>(p, t3); break;
+	default: launch_split<64, 128, 2, 2, 210>(p, t3); break;
 	}
 	LTEN_HIP_LAUNCH_CHECK();
 	return 0;

@@ -382,3 +382,27 @@ def test_weight_gradient_of_wide_layers_on_integers(gpu, N, Cin, Cout):
     want = np.stack([dy.transpose(1, 0, 2, 3).reshape(Cout, -1) @ xp[:, :, i:i + 10, j:j + 12].transpose(0, 2, 3, 1).reshape(-1, Cin)
                      for i in range(3) for j in range(3)], axis=-1)
     assert np.array_equal(run_wgrad(gpu, geo, x, dy).reshape(Cout, Cin, 9), want)
+
+
+@pytest.mark.parametrize("geo", [
+    (5, 16, 1, 3, 32, 3, 3, 1, 1, 1, 1),       # planes of fewer values than a quad: staged from a copy
+    (2, 48, 2, 2, 40, 3, 3, 1, 1, 1, 1),       # every quad of a plane reaches past one of its ends; an odd number of chunks
+    (2, 64, 5, 6, 33, 3, 3, 2, 2, 1, 1),       # quads turned by two and more; rows and their padding no multiple of 4
+    (12, 90, 7, 7, 70, 3, 3, 1, 1, 1, 1),      # narrow maps: more positions to a tile than pixels, tiles of fewer than 256 pixels
+    (20, 20, 33, 33, 40, 5, 5, 2, 2, 2, 2),    # a window and stride that fit with narrow strips or small tiles only
+    (3, 16, 31, 43, 64, 3, 3, 0, 0, 2, 2),     # 3 x 3 at stride 2, one chunk, no padding
+])
+def test_patches_of_quads_on_integers(gpu, geo):
+    """The quads at the ends of a plane, patches that do not fit at a full tile, one chunk to six.  Exact in any order."""
+    rng = np.random.default_rng(sum(geo))
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    mk = lambda *s: rng.integers(-8, 9, s).astype(np.float32)
+    x, w, bias, dy = mk(N, Cin, H, W), mk(Cout, Cin, kh, kw), mk(Cout), mk(N, Cout, *out_hw(geo))
+    want_y, want_dx = forward64(geo, x, w, bias), dgrad64(geo, w, dy)
+    taken = 0
+    for variant in [10] + [11 + k for k in range(TILES)]:
+        y, dx = run(gpu, geo, x, w, bias, dy, variant)
+        taken += (y is not None) + (dx is not None)
+        assert y is None or np.array_equal(y, want_y), (geo, variant)
+        assert dx is None or np.array_equal(dx, want_dx), (geo, variant)
+    assert taken >= 8
