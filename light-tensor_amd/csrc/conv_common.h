@@ -53,7 +53,22 @@ int conv_reduce_partials(const float* partial, int parts, int64_t count, float* 
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Quotients of numbers below 2^31 by a divisor that a whole launch shares: n / d = (n ceil(2^(31 + s) / d)) >> (31 + s) for
+// 2^(s - 1) < d <= 2^s (Granlund and Montgomery, "Division by invariant integers using multiplication", PLDI 1994).
+struct Divisor {
+	uint32_t mul, shift;
+};
+inline Divisor make_divisor(uint32_t d)
+{
+	Divisor r = { 0, 0 };
+	while ((1ull << r.shift) < d) r.shift++;
+	r.mul = (uint32_t)(((1ull << (31 + r.shift)) + d - 1) / d);
+	return r;
+}
+
 #if defined(__HIPCC__)
+__device__ __forceinline__ int quotient(int n, Divisor d) { return (int)(__umulhi((uint32_t)n << 1, d.mul) >> d.shift); }
+
 // Four consecutive floats of a row starting at column gx; columns outside [0, limit) read as 0.  With VEC
 // (limit % 4 == 0, gx % 4 == 0, 16-byte aligned row) the four are inside or outside together.
 template <bool VEC>

@@ -220,19 +220,21 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 			}
 			uint8_t* d = smem + stage * STAGE + oct * 3 * PLANE + quad * 16 + half * 8;
 #pragma unroll
-			for (int e = 0; e < 4; e++) {
-				// a position outside the map counts as zeros: the scale is zero there (an infinity times it is a NaN, and the tile
-				// is computed again on the values themselves)
-				const float scale = __builtin_bit_cast(float, (uint32_t)((int)(inside << (31 - 4 * u - e)) >> 31) & __builtin_bit_cast(uint32_t, pieces_scale));
-				float v[4];
+			for (int e = 0; e < 4; e += 2) {
+				const float scale0 = scale_where(inside, 4 * u + e), scale1 = scale_where(inside, 4 * u + e + 1);  // (a position outside the map counts as zeros)
+				float v[8];
 #pragma unroll
-				for (int k = 0; k < 4; k++) v[k] = raw[u][k][e] * scale;
-				uint2 piece[3];
-				piece[0].x = split_off(v[0], v[1]); piece[0].y = split_off(v[2], v[3]);
-				piece[1].x = split_off(v[0], v[1]); piece[1].y = split_off(v[2], v[3]);
-				piece[2].x = split_last(v[0], v[1]); piece[2].y = split_last(v[2], v[3]);
+				for (int k = 0; k < 4; k++) {
+					v[k] = raw[u][k][e] * scale0;
+					v[4 + k] = raw[u][k][e + 1] * scale1;
+				}
+				uint4 piece[3];
+				split8_scaled(v, piece);
 #pragma unroll
-				for (int k = 0; k < 3; k++) *reinterpret_cast<uint2*>(d + k * PLANE + e * Q * 16) = piece[k];
+				for (int k = 0; k < 3; k++) {
+					*reinterpret_cast<uint2*>(d + k * PLANE + e * Q * 16) = make_uint2(piece[k].x, piece[k].y);
+					*reinterpret_cast<uint2*>(d + k * PLANE + (e + 1) * Q * 16) = make_uint2(piece[k].z, piece[k].w);
+				}
 			}
 		};
 		int ld_tile = tile0, ld_chunk = 0;

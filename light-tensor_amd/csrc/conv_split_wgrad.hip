@@ -10,13 +10,14 @@
 // A tap row's operands for all three tap columns are the 16 bytes of a slot and the first four of the next: the shift by
 // one column is four vector instructions a piece, and a value is converted once however many taps use it.
 //
-// Half of the eight wavefronts load, convert and fill the stage of the next chunk (a thread stages one channel of every
-// eighth slot, as many as the chunk has; loads are a chunk further ahead), the other half multiplies: two blocks of 32 channels x two
-// halves of the chunk's k-steps of 16 pixels, nine accumulators each, added at the end.  Measured (patch kernels, column
-// matrices -> here): 32 x 32 x 128 x 128 -> 64 channels 171 -> 123 us (157 TFLOP/s), 32 x 256 x 14 x 14 -> 256 120 -> 60,
-// 27 x 124 x 35 x 35 -> 32 86 -> 43, 31 x 16 x 36 x 91 -> 32 64 -> 33; at stride two a chunk's staging is the longer half (16
-// x 64 x 57 x 57 -> 128: 34.5 us against the implicit GEMM's 44; with one slot per thread for four channels, which left the
-// threads of slots 15 to 31 idle where a chunk has 15: 40.8, and 31 x 128 x 28 x 28 -> 256 59 against 49).  Shifting the operands of the next tap
+// Half of the eight wavefronts load, convert and fill the stage of the next chunk (loads are a chunk further ahead), the other
+// half multiplies: two blocks of 32 channels x two halves of the chunk's k-steps of 16 pixels, nine accumulators each, added at
+// the end.  Measured (patch kernels, column matrices -> here): 32 x 32 x 128 x 128 -> 64 channels 171 -> 107 us (180 TFLOP/s),
+// 32 x 256 x 14 x 14 -> 256 120 -> 51, 27 x 124 x 35 x 35 -> 32 86 -> 38; at stride two a chunk's staging is the longer half (16
+// x 64 x 57 x 57 -> 128: 32.3 us against the implicit GEMM's 44).  What staging a chunk takes had bound stride one too, 5800
+// clocks to the 4000 of its products: loads that touched 64 cache lines each (3500 clocks of them), divisions, conversions of two
+// values at a time, in which every instruction waits for the one before.  Now it is 4300 (3800 at stride two, was 5100), and
+// the chip is at its power limit on long runs (1.7 GHz; 120 -> 107, 59 -> 51, 97 -> 86 us at 64 x 128 x 28 x 28).  Shifting the operands of the next tap
 // between the products of this one instead of ahead of them made no difference.  The sums of the slices go to memory
 // of the library as [slice][tap][co][ci] and are added in order by a second launch.
 // 2-norm error against float64 over 16 layers, the routes before -> here: 0.07 to 0.95 of it on uniform values, 0.24 to 1.3 on
@@ -46,15 +47,17 @@ struct SplitWgrad {
 	int rows;                          // output rows of the batch
 	int row_chunks, chunks;            // chunks of a strip, of all strips
 	int tiles_m, tiles, slices, per_slice;
-	unsigned x_last4, dy_last4;        // the last element four values can be read from
+	int x_last4, dy_last4;             // the last element four values can be read from
+	Divisor by_Ho, by_full_rows, by_row_chunks;
 };
 
 template <int S>
 struct WgradTile {
 	static constexpr int OCT = S == 1 ? 8 : 4, SLOTS = S == 1 ? 32 : 20;
-	static constexpr int X_PIECE = SLOTS * 512, X_PLANE = 3 * X_PIECE, X_BYTES = S * X_PLANE;
-	static constexpr int DY_PIECE = OCT * 1024, DY_BYTES = 3 * DY_PIECE, STAGE = X_BYTES + DY_BYTES;
-	static constexpr int X_UNITS = (SLOTS + 7) / 8, DY_UNITS = OCT / 4;  // of a staging thread
+	// (slots and octets set apart so that the 8-byte writes of 32 lanes, two to a slot or octet, fall on different banks)
+	static constexpr int X_SLOT = 512 + 16, X_PIECE = SLOTS * X_SLOT, X_PLANE = 3 * X_PIECE, X_BYTES = S * X_PLANE;
+	static constexpr int DY_OCT = 1024 + (OCT == 8 ? 32 : 64), DY_PIECE = OCT * DY_OCT, DY_BYTES = 3 * DY_PIECE, STAGE = X_BYTES + DY_BYTES;
+	static constexpr int X_UNITS = S == 1 ? 8 : 5, DY_LANES = 32 / OCT, DY_UNITS = 16 / DY_LANES;  // of a staging thread; channels of dy to a wavefront
 	static constexpr int STEPS = OCT / 4;     // k-steps of a wavefront in a chunk
 	static_assert(2 * STAGE + 64 <= 160 * 1024 && 2 * STAGE >= 2 * 9 * 16 * 64 * 4, "two stages fit LDS, and the halves' sums fit them");
 };
@@ -85,138 +88,150 @@ __global__ __launch_bounds__(512, 2) void conv_split_wgrad_kernel(SplitWgrad p)
 
 	if (wave >= 4) {
 		// ---- the staging half
-		const int t = threadIdx.x & 255;
-		// unit u: a wavefront takes 16 channels of four slots, the whole half 32 channels of the slots 8 u .. 8 u + 7
-		const int ch = (lane & 15) | (t >> 6 & 1) << 4, slot = (lane >> 4) + (t >> 7) * 4;
-		int slot_row[T::X_UNITS], slot_oct[T::X_UNITS];
+		// x: two lanes to a slot.  A wavefront takes eight channels: all 32 slots of one at a time, at stride two 16 slots of two at a
+		// time and then the other four slots of all eight.  dy: two lanes to an octet, all octets of DY_LANES channels at a time.  So the
+		// lanes of a load read rows that lie next to each other (with 16 channels of four slots to a wavefront every lane had a cache
+		// line of its own, and the loads of a chunk took 3500 clocks).
+		const int w = wave & 3, h = lane & 1;
+		constexpr int COLS = 4 * S, KINDS = S;    // columns of a lane; kinds of slots it takes: its first, its second
+		constexpr int DY_STEP = 4 * T::DY_LANES;  // channels from one unit to the next
+		int slot_row[KINDS], slot_oct[KINDS], x_lds[KINDS], x_channel[T::X_UNITS], dy_channel[T::DY_UNITS];
+		const int x_plane = p.H * p.W, x_image = p.C * x_plane, dy_plane = p.Ho * p.Wo, dy_image = p.M * dy_plane;
 #pragma unroll
-		for (int u = 0; u < T::X_UNITS; u++) {
-			slot_row[u] = (slot + 8 * u) / XO;
-			slot_oct[u] = slot + 8 * u - slot_row[u] * XO;
+		for (int k = 0; k < KINDS; k++) {
+			const int slot = S == 1 ? lane >> 1 : k == 0 ? lane >> 1 & 15 : 16 + (lane >> 1 & 3);
+			slot_row[k] = slot / XO;
+			slot_oct[k] = slot - slot_row[k] * XO;
+			x_lds[k] = slot * T::X_SLOT + (8 * w + (S == 1 ? 0 : k == 0 ? lane >> 5 : lane >> 3)) * 16 + h * 8;
 		}
-		const int dy_oct = (t >> 3) & (T::OCT - 1), dy_co = (t & 7) + 8 * (t / (8 * T::OCT));
-		constexpr int DY_CO_STEP = 8 * 256 / (8 * T::OCT);  // channels from one unit to the next
-		float rx[T::X_UNITS][8 * S], rd[T::DY_UNITS][8];
-		// what lies in the registers: of x, the slots of the chunk, how many columns from a slot's first on exist, whether that
-		// is the padding, by how much the last loads were moved back into the tensor (of one unit at most: two are eight
-		// columns or more than three rows apart); of dy likewise
-		struct Held { int slots, x_valid[T::X_UNITS], x_back, dy_valid, dy_back; bool left[T::X_UNITS]; };
+		// (channels past the end repeat the last one, and what they add up to is not read)
+#pragma unroll
+		for (int u = 0; u < T::X_UNITS; u++) x_channel[u] = min(c0 + 8 * w + (S == 1 ? u : u < 4 ? 2 * u + (lane >> 5) : lane >> 3), p.C - 1) * x_plane;
+		const int dy_oct = (lane >> 1) & (T::OCT - 1), dy_co = w * T::DY_LANES + (lane >> 1) / T::OCT;
+#pragma unroll
+		for (int u = 0; u < T::DY_UNITS; u++) dy_channel[u] = min(m0 + dy_co + DY_STEP * u, p.M - 1) * dy_plane;
+		float rx[T::X_UNITS][COLS], rd[T::DY_UNITS][4];
+		// of a lane's loads: where they start in channel 0, which columns exist, whether a load could leave the tensor
+		struct Held { int x_at[KINDS], dy_at; unsigned x_bits[KINDS], dy_bits; bool edge; };
 		Held held = {}, next = {};
-		auto load = [&](int chunk) {
-			const int strip = chunk / p.row_chunks, g0 = (chunk - strip * p.row_chunks) * chunk_rows;
-			const int n0 = g0 / p.Ho, ho0 = g0 - n0 * p.Ho, g_last = min(g0 + chunk_rows, p.rows) - 1;
+		auto place_loads = [&](int chunk) {
+			const int strip = quotient(chunk, p.by_row_chunks), g0 = (chunk - strip * p.row_chunks) * chunk_rows;
+			const int n0 = quotient(g0, p.by_Ho), ho0 = g0 - n0 * p.Ho, g_last = min(g0 + chunk_rows, p.rows) - 1;
 			const int first_rows = (p.Ho - 1 - ho0) * S + 3;
-			const int n_last = g_last / p.Ho, ho_last = g_last - n_last * p.Ho;
+			const int n_last = quotient(g_last, p.by_Ho), ho_last = g_last - n_last * p.Ho;
 			const int rows = n_last == n0 ? (ho_last - ho0) * S + 3 : first_rows + (n_last - n0 - 1) * full_rows + ho_last * S + 3;
-			next.slots = rows * XO;
-			next.x_back = 0;
+			next.edge = false;
 #pragma unroll
-			for (int u = 0; u < T::X_UNITS; u++) {
-				if (8 * u >= next.slots) continue;
-				int n = n0, yy = ho0 * S - p.ph + slot_row[u];
-				if (slot_row[u] >= first_rows) {
-					const unsigned k = (unsigned)(slot_row[u] - first_rows) / (unsigned)full_rows;
-					n += 1 + (int)k;
-					yy = slot_row[u] - first_rows - (int)k * full_rows - p.ph;
+			for (int k = 0; k < KINDS; k++) {
+				int image = n0 * x_image, yy = ho0 * S - p.ph + slot_row[k];
+				if (slot_row[k] >= first_rows) {
+					const int i = quotient(slot_row[k] - first_rows, p.by_full_rows);
+					image += (1 + i) * x_image;
+					yy = slot_row[k] - first_rows - i * full_rows - p.ph;
 				}
-				const int col = (strip * OC + slot_oct[u]) * 8 * S - PW;
-				next.left[u] = PW != 0 && col < 0;
-				next.x_valid[u] = slot + 8 * u < next.slots && c0 + ch < p.C && (unsigned)yy < (unsigned)p.H ? p.W - col : 0;
-				const unsigned at = next.x_valid[u] > 0 ? (((unsigned)n * p.C + (unsigned)(c0 + ch)) * (unsigned)p.H + (unsigned)yy) * (unsigned)p.W + (unsigned)max(col, 0) : 0u;
-#pragma unroll
-				for (int q = 0; q < 2 * S; q++) {
-					const unsigned want = at + 4 * q, got = min(want, p.x_last4);
-					if (want != got && 4 * q < next.x_valid[u]) next.x_back = (int)(want - got) | (q << 4) | (u << 8);
-					const f4_any v = *reinterpret_cast<const f4_any*>(p.x + got);
-					rx[u][4 * q] = v.x; rx[u][4 * q + 1] = v.y; rx[u][4 * q + 2] = v.z; rx[u][4 * q + 3] = v.w;
-				}
+				// (the column left of a row is the value before it, which does not count)
+				const int col = (strip * OC + slot_oct[k]) * 8 * S - PW + h * COLS;
+				const bool there = slot_row[k] < rows && (unsigned)yy < (unsigned)p.H;
+				next.x_bits[k] = there ? ((1u << min(max(p.W - col, 0), COLS)) - 1) & ~(unsigned)(PW != 0 && col < 0) : 0u;
+				next.x_at[k] = next.x_bits[k] != 0 ? image + yy * p.W + col : 0;
+				next.edge |= next.x_at[k] < 0 || next.x_at[k] + (p.C - 1) * x_plane + COLS - 4 > p.x_last4;
 			}
-			const int g = g0 + (dy_oct >> p.oc_log2), dcol = (strip * OC + (dy_oct & (OC - 1))) * 8;
-			next.dy_valid = g < p.rows ? p.Wo - dcol : 0;
-			next.dy_back = 0;
-			const int dn = g / p.Ho, dho = g - dn * p.Ho;
-			const unsigned d_at = next.dy_valid > 0 ? ((unsigned)dn * p.M * (unsigned)p.Ho + (unsigned)dho) * (unsigned)p.Wo + (unsigned)dcol : 0u;
-#pragma unroll
-			for (int u = 0; u < T::DY_UNITS; u++) {
-				const unsigned c_at = d_at + (unsigned)(min(m0 + dy_co + DY_CO_STEP * u, p.M - 1) * p.Ho) * (unsigned)p.Wo;
-#pragma unroll
-				for (int q = 0; q < 2; q++) {
-					const unsigned want = c_at + 4 * q, got = min(want, p.dy_last4);
-					if (want != got && 4 * q < next.dy_valid && m0 + dy_co + DY_CO_STEP * u < p.M) next.dy_back = max(next.dy_back, (int)(want - got) | (q << 4) | (u << 8));
-					const f4_any v = *reinterpret_cast<const f4_any*>(p.dy + got);
-					rd[u][4 * q] = v.x; rd[u][4 * q + 1] = v.y; rd[u][4 * q + 2] = v.z; rd[u][4 * q + 3] = v.w;
-				}
-			}
+			const int g = g0 + (dy_oct >> p.oc_log2), dcol = (strip * OC + (dy_oct & (OC - 1))) * 8 + 4 * h;
+			const int dn = quotient(g, p.by_Ho), dho = g - dn * p.Ho;
+			next.dy_bits = g < p.rows ? (1u << min(max(p.Wo - dcol, 0), 4)) - 1 : 0u;
+			next.dy_at = next.dy_bits != 0 ? dn * dy_image + dho * p.Wo + dcol : 0;
+			next.edge |= next.dy_at + (p.M - 1) * dy_plane > p.dy_last4;
 		};
-		// value e of four that were read `back` elements early because the tensor ends behind them
-		auto moved = [&](float v0, float v1, float v2, float v3, int e, int back) {
-			const float s0 = e == 0 ? v0 : e == 1 ? v1 : e == 2 ? v2 : v3, s1 = e == 0 ? v1 : e == 1 ? v2 : v3, s2 = e == 0 ? v2 : v3;
-			return back == 0 ? s0 : back == 1 ? s1 : back == 2 ? s2 : v3;
+		auto kind = [](int u) { return S == 2 && u == 4 ? 1 : 0; };
+		auto load4 = [&](const float* from, int at, float* r) {
+			const f4_any v = *reinterpret_cast<const f4_any*>(reinterpret_cast<const char*>(from) + (uint32_t)at * 4u);
+			r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
 		};
-		auto convert = [&](int stage) {
-			uint8_t* sx = smem + stage * T::STAGE + slot * 512 + ch * 16;
+		// (loads under no condition: each wait is for all behind one)
+		auto load_x = [&](int u) {
 #pragma unroll
-			for (int u = 0; u < T::X_UNITS; u++) {
-				if (8 * u >= held.slots) continue;
-				if (__any(held.x_back != 0)) {
+			for (int q = 0; q < S; q++) load4(p.x, min(max(next.x_at[kind(u) < KINDS ? kind(u) : 0] + x_channel[u] + 4 * q, 0), p.x_last4), &rx[u][4 * q]);
+		};
+		auto load_dy = [&](int u) { load4(p.dy, min(next.dy_at + dy_channel[u], p.dy_last4), rd[u]); };
+		// four values that were read `by` elements early because the tensor ends behind them, or one late because it starts with the second
+		auto move = [&](float* r, int by) {
+			const float v0 = r[0], v1 = r[1], v2 = r[2], v3 = r[3];
+			r[0] = by == 1 ? v1 : by == 2 ? v2 : by == 3 ? v3 : v0;
+			r[1] = by == -1 ? v0 : by == 1 ? v2 : by == 2 ? v3 : v1;
+			r[2] = by == -1 ? v1 : by == 1 ? v3 : v2;
+			r[3] = by == -1 ? v2 : v3;
+		};
+		// eight values, the first four for `a`, the others for `b`
+		auto put = [&](float (&v)[8], uint8_t* a, uint8_t* b, int step) {
+			uint4 piece[3];
+			split8_scaled(v, piece);
 #pragma unroll
-					for (int q = 0; q < 2 * S; q++)
-						{
-							const int back = held.x_back >> 4 == (q | u << 4) ? held.x_back & 15 : 0;
-							const float v0 = rx[u][4 * q], v1 = rx[u][4 * q + 1], v2 = rx[u][4 * q + 2], v3 = rx[u][4 * q + 3];
+			for (int q = 0; q < 3; q++) *reinterpret_cast<uint2*>(a + q * step) = make_uint2(piece[q].x, piece[q].y);
 #pragma unroll
-							for (int e = 0; e < 4; e++) rx[u][4 * q + e] = moved(v0, v1, v2, v3, e, back);
+			for (int q = 0; q < 3; q++) *reinterpret_cast<uint2*>(b + q * step) = make_uint2(piece[q].z, piece[q].w);
+		};
+		place_loads(begin);
+#pragma unroll
+		for (int u = 0; u < T::X_UNITS; u++) load_x(u);
+#pragma unroll
+		for (int u = 0; u < T::DY_UNITS; u++) load_dy(u);
+		for (int chunk = begin - 1; chunk < end; chunk++) {  // converts chunk + 1, loads chunk + 2 (the last one again past the end)
+			if (chunk + 1 < end) {
+				held = next;
+				place_loads(min(chunk + 2, end - 1));
+				if (__any(held.edge)) {
+#pragma unroll
+					for (int u = 0; u < T::X_UNITS; u++)
+#pragma unroll
+						for (int q = 0; q < S; q++) {
+							const int want = held.x_at[kind(u) < KINDS ? kind(u) : 0] + x_channel[u] + 4 * q;
+							move(&rx[u][4 * q], want - min(max(want, 0), p.x_last4));
 						}
-				}
-				float v[8 * S], before = 0.0f;
 #pragma unroll
-				for (int e = 0; e < 8 * S; e++) {
-					const uint32_t here_bits = __builtin_bit_cast(uint32_t, rx[u][e]), before_bits = __builtin_bit_cast(uint32_t, before);
-					const uint32_t bits = PW != 0 && held.left[u] ? before_bits : here_bits;
-					v[e] = e < held.x_valid[u] ? __builtin_bit_cast(float, bits) : 0.0f;
-					before = rx[u][e];
-				}
-				if (slot + 8 * u < held.slots) {
-#pragma unroll
-					for (int s = 0; s < S; s++) {
-						float w[8];
-#pragma unroll
-						for (int e = 0; e < 8; e++) w[e] = v[S * e + s];
-						uint4 piece[3];
-						split8(w, piece);
-#pragma unroll
-						for (int q = 0; q < 3; q++) *reinterpret_cast<uint4*>(sx + s * T::X_PLANE + q * T::X_PIECE + u * 4096) = piece[q];
+					for (int u = 0; u < T::DY_UNITS; u++) {
+						const int want = held.dy_at + dy_channel[u];
+						move(rd[u], want - min(want, p.dy_last4));
 					}
 				}
-			}
-			uint8_t* sd = smem + stage * T::STAGE + T::X_BYTES + dy_oct * 1024 + dy_co * 16;
+				uint8_t* const st = smem + ((chunk + 1 - begin) & 1) * T::STAGE;
+				float scale[COLS], v[8];
 #pragma unroll
-			for (int u = 0; u < T::DY_UNITS; u++) {
-				if (__any(held.dy_back != 0)) {
+				for (int e = 0; e < COLS; e++) scale[e] = scale_where(held.x_bits[0], e);
+				if constexpr (S == 1) {
+					uint8_t* const sx = st + x_lds[0];
 #pragma unroll
-					for (int q = 0; q < 2; q++)
-						{
-							const int back = held.dy_back >> 4 == (q | u << 4) ? held.dy_back & 15 : 0;
-							const float v0 = rd[u][4 * q], v1 = rd[u][4 * q + 1], v2 = rd[u][4 * q + 2], v3 = rd[u][4 * q + 3];
+					for (int u = 0; u < T::X_UNITS; u += 2) {
 #pragma unroll
-							for (int e = 0; e < 4; e++) rd[u][4 * q + e] = moved(v0, v1, v2, v3, e, back);
+						for (int e = 0; e < 8; e++) v[e] = rx[u + e / 4][e % 4] * scale[e % 4];
+						load_x(u);
+						load_x(u + 1);
+						put(v, sx + u * 16, sx + u * 16 + 16, T::X_PIECE);
+					}
+				} else {
+#pragma unroll
+					for (int u = 0; u < T::X_UNITS; u++) {
+						if (u == 4) {
+#pragma unroll
+							for (int e = 0; e < COLS; e++) scale[e] = scale_where(held.x_bits[KINDS - 1], e);
 						}
+#pragma unroll
+						for (int e = 0; e < 8; e++) v[e] = rx[u][e < 4 ? 2 * e : 2 * e - 7] * scale[e < 4 ? 2 * e : 2 * e - 7];  // the even ones, the odd ones
+						load_x(u);
+						uint8_t* const sx = st + x_lds[u == 4 ? KINDS - 1 : 0] + (u < 4 ? u * 32 : 0);
+						put(v, sx, sx + T::X_PLANE, T::X_PIECE);
+					}
 				}
-				float v[8];
 #pragma unroll
-				for (int e = 0; e < 8; e++) v[e] = e < held.dy_valid ? rd[u][e] : 0.0f;
-				uint4 piece[3];
-				split8(v, piece);
+				for (int e = 0; e < 4; e++) scale[e] = scale_where(held.dy_bits, e);
+				uint8_t* const sd = st + T::X_BYTES + dy_oct * T::DY_OCT + dy_co * 16 + h * 8;
 #pragma unroll
-				for (int q = 0; q < 3; q++) *reinterpret_cast<uint4*>(sd + q * T::DY_PIECE + u * DY_CO_STEP * 16) = piece[q];
-			}
-		};
-		load(begin);
-		for (int chunk = begin - 1; chunk < end; chunk++) {  // converts chunk + 1, loads chunk + 2 (the last one again past the end)
-			held = next;
-			if (chunk + 1 < end) {
-				convert((chunk + 1 - begin) & 1);
-				load(min(chunk + 2, end - 1));
+				for (int u = 0; u < T::DY_UNITS; u += 2) {
+#pragma unroll
+					for (int e = 0; e < 8; e++) v[e] = rd[u + e / 4][e % 4] * scale[e % 4];
+					load_dy(u);
+					load_dy(u + 1);
+					put(v, sd + u * DY_STEP * 16, sd + (u + 1) * DY_STEP * 16, T::DY_PIECE);
+				}
 			}
 			__syncthreads();
 		}
@@ -236,17 +251,17 @@ __global__ __launch_bounds__(512, 2) void conv_split_wgrad_kernel(SplitWgrad p)
 	// k-step t of this wavefront: octets 2 (khalf + 2 t) + lk of the chunk; where they lie in the stage
 	uint32_t xb[T::STEPS], db[T::STEPS];
 #pragma unroll
-	for (int t = 0; t < T::STEPS; t++) db[t] = (uint32_t)(T::X_BYTES + (2 * (khalf + 2 * t) + lk) * 1024 + (mt * 32 + lrow) * 16);
+	for (int t = 0; t < T::STEPS; t++) db[t] = (uint32_t)(T::X_BYTES + (2 * (khalf + 2 * t) + lk) * T::DY_OCT + (mt * 32 + lrow) * 16);
 	auto place = [&](int chunk) {
-		const int strip = chunk / p.row_chunks, g0 = (chunk - strip * p.row_chunks) * chunk_rows;
-		const int n0 = g0 / p.Ho, ho0 = g0 - n0 * p.Ho, first_rows = (p.Ho - 1 - ho0) * S + 3;
+		const int strip = quotient(chunk, p.by_row_chunks), g0 = (chunk - strip * p.row_chunks) * chunk_rows;
+		const int n0 = quotient(g0, p.by_Ho), ho0 = g0 - n0 * p.Ho, first_rows = (p.Ho - 1 - ho0) * S + 3;
 #pragma unroll
 		for (int t = 0; t < T::STEPS; t++) {
 			const int oct = 2 * (khalf + 2 * t) + lk;
 			const int g = min(g0 + (oct >> p.oc_log2), p.rows - 1);  // (rows past the last: their dy is zero)
-			const int n = g / p.Ho, ho = g - n * p.Ho;
+			const int n = quotient(g, p.by_Ho), ho = g - n * p.Ho;
 			const int r = n == n0 ? (ho - ho0) * S : first_rows + (n - n0 - 1) * full_rows + ho * S;
-			xb[t] = (uint32_t)((r * XO + (oct & (OC - 1))) * 512 + lrow * 16);
+			xb[t] = (uint32_t)((r * XO + (oct & (OC - 1))) * T::X_SLOT + lrow * 16);
 		}
 	};
 	// a window: eight columns in four words and two more in the fifth; at stride two the eight odd ones behind them
@@ -256,10 +271,10 @@ __global__ __launch_bounds__(512, 2) void conv_split_wgrad_kernel(SplitWgrad p)
 	auto read_window = [&](int set, uint32_t base, int i) {
 #pragma unroll
 		for (int v = 0; v < 3; v++) {
-			const uint8_t* at = smem + base + i * XO * 512 + v * T::X_PIECE;
+			const uint8_t* at = smem + base + i * XO * T::X_SLOT + v * T::X_PIECE;
 			const uint4 a = *reinterpret_cast<const uint4*>(at);
 			win[set][v][0] = a.x; win[set][v][1] = a.y; win[set][v][2] = a.z; win[set][v][3] = a.w;
-			win[set][v][4] = *reinterpret_cast<const uint32_t*>(at + 512);
+			win[set][v][4] = *reinterpret_cast<const uint32_t*>(at + T::X_SLOT);
 			if (S == 2) {
 				const uint4 o = *reinterpret_cast<const uint4*>(at + T::X_PLANE);
 				win[set][v][WORDS - 4] = o.x; win[set][v][WORDS - 3] = o.y; win[set][v][WORDS - 2] = o.z; win[set][v][WORDS - 1] = o.w;
@@ -467,15 +482,15 @@ int conv_split_wgrad(const ConvGeo& g, const float* x, const float* dy, float* d
 	const uint64_t in_elems = (uint64_t)g.N * g.Cin * g.H * g.W, out_elems = (uint64_t)g.N * g.Cout * g.Ho * g.Wo;
 	if (g.kh != 3 || g.kw != 3 || g.dh != 1 || g.dw != 1 || g.sh != g.sw || g.sh > 2 || g.pw > 1 || g.ph > 2 || in_elems >= (1ull << 30) || out_elems >= (1ull << 30) ||
 	    in_elems < 4 || out_elems < 4 || (uint64_t)g.Cout >= 65536) return -1;
-	// x of up to four images of one or two columns: two slots of a thread could both end behind x_last4 (walked through for all
-	// sizes up to 9 images of 9 x 19: none from 16 values or three columns on)
-	if (in_elems < 16 && g.W < 3) return -1;
+	if (in_elems < 16 && g.W < 3) return -1;  // (a handful of values: the other routes')
 	const int S = g.sh, oct = S == 1 ? 8 : 4, slots = S == 1 ? 32 : 20;
 	SplitWgrad p = {};
 	p.x = x; p.dy = dy;
 	p.N = g.N; p.C = g.Cin; p.H = g.H; p.W = g.W; p.M = g.Cout; p.Ho = g.Ho; p.Wo = g.Wo; p.ph = g.ph;
-	p.x_last4 = (unsigned)in_elems - 4; p.dy_last4 = (unsigned)out_elems - 4;
+	p.x_last4 = (int)in_elems - 4; p.dy_last4 = (int)out_elems - 4;
 	p.rows = g.N * g.Ho;
+	p.by_Ho = make_divisor((uint32_t)g.Ho);
+	p.by_full_rows = make_divisor((uint32_t)((g.Ho - 1) * S + 3));
 	p.tiles_m = (int)ceil_div((uint64_t)g.Cout, 64);
 	p.tiles = p.tiles_m * (int)ceil_div((uint64_t)g.Cin, 32);
 	// Strips of OC octets: the fewest chunks, then the fewest slots staged (a chunk's rows with their halo, of every image they
@@ -498,16 +513,16 @@ int conv_split_wgrad(const ConvGeo& g, const float* x, const float* dy, float* d
 	p.oc_log2 = best_log2;
 	p.row_chunks = (int)ceil_div((uint64_t)p.rows, (uint64_t)(oct >> best_log2));
 	p.chunks = p.row_chunks * (int)ceil_div((uint64_t)g.Wo, (uint64_t)(8 << best_log2));
+	p.by_row_chunks = make_divisor((uint32_t)p.row_chunks);
 	// slices that give every CU a workgroup
 	const uint64_t want = std::max<uint64_t>(1, 256 / (uint64_t)p.tiles);
 	p.per_slice = (int)ceil_div((uint64_t)p.chunks, want);
 	p.slices = (int)ceil_div((uint64_t)p.chunks, (uint64_t)p.per_slice);
 	const uint64_t Mp = (uint64_t)p.tiles_m * 64, Cp = (uint64_t)(p.tiles / p.tiles_m) * 32, bytes = (uint64_t)p.slices * 9 * Mp * Cp * 4;
 	if (bytes > (1ull << 29) || (uint64_t)p.tiles * p.slices >= (1u << 24)) return -1;
-	// a chunk: two k-steps of 54 products (32 clocks each, 46 with what comes between), at stride two its staging (measured:
-	// 3050 to 3900 clocks with up to 16 slots, two units a thread, 4000 to 4700 with more); a start and an end; the launches and
-	// the sums
-	const double rounds = (double)ceil_div((uint64_t)p.tiles * p.slices, 256), chunk_clocks = S == 1 ? 2 * 54 * 46.0 : 3900.0 + 200.0 * (double)std::max<int64_t>(0, best_used - 16);
+	// a chunk: two k-steps of 54 products (32 clocks each, 41 with what comes between), at stride two its staging (3900 clocks
+	// with 15 slots); a start and an end; the launches and the sums
+	const double rounds = (double)ceil_div((uint64_t)p.tiles * p.slices, 256), chunk_clocks = S == 1 ? 2 * 54 * 41.0 : 3900.0 + 200.0 * (double)std::max<int64_t>(0, best_used - 16);
 	if (10.0 + rounds * (p.per_slice * chunk_clocks + 8000.0) / 1850.0 + 1.2 * (double)bytes / 4e6 >= limit_us) return -1;
 	p.partial = static_cast<float*>(library_scratch(bytes));
 	if (p.partial == nullptr) return -1;

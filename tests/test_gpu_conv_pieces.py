@@ -406,3 +406,17 @@ def test_patches_of_quads_on_integers(gpu, geo):
         assert y is None or np.array_equal(y, want_y), (geo, variant)
         assert dx is None or np.array_equal(dx, want_dx), (geo, variant)
     assert taken >= 8
+
+
+@pytest.mark.parametrize("geo", [
+    (3, 6, 1, 1, 4, 3, 3, 1, 1, 1, 1), (2, 11, 1, 2, 70, 3, 3, 1, 1, 1, 1),  # quads that reach over the planes behind, at the end of either tensor
+    (5, 2, 3, 1, 3, 3, 3, 1, 1, 2, 2), (2, 9, 2, 5, 5, 3, 3, 1, 1, 2, 2),
+    (6, 4, 17, 17, 33, 3, 3, 1, 1, 1, 1), (6, 1, 17, 18, 33, 3, 3, 1, 1, 2, 2),  # few channels: the others repeat the last
+    (7, 37, 4, 40, 66, 3, 3, 1, 1, 2, 2), (9, 40, 5, 13, 20, 3, 3, 1, 0, 2, 2),  # up to 20 slots: the second kind of a lane
+])
+def test_weight_gradient_staging_on_integers(gpu, geo):
+    """Loads that leave a plane, a row or the tensor, both strides.  Exact in any order."""
+    rng = np.random.default_rng(sum(geo))
+    x = rng.integers(-8, 9, geo[:4]).astype(np.float32)
+    dy = rng.integers(-8, 9, (geo[0], geo[4], *out_hw(geo))).astype(np.float32)
+    assert np.array_equal(run_wgrad(gpu, geo, x, dy), wgrad64(geo, x, dy))
