@@ -3,10 +3,14 @@
 // At these sizes (e.g. l-ten's 64 x 784 MNIST batch against a 512 x 784 weight matrix) the run time is launch
 // and memory latency, not arithmetic, so the kernel is one dependent chain as short as possible: a workgroup
 // owns one 16 x 16 output tile, its wavefronts split K in 64-byte steps (wavefront w takes steps w, w + WAVES,
-// ...), every lane loads the 16 bytes the 16x16x64 int8 MFMA wants from it (row lane % 16, k-group lane / 16)
-// for all its steps at once, and the zero-point byte sums come from the same registers with dot4 instructions
-// — no separate row-sum launch.  The partial tiles and sums meet in LDS and wavefront 0 applies the identity
-// of qgemm.hip and the requantize of l-ten/math_fns.cpp:1469-1474.
+// ...), the loads of U of its steps at once, and the zero-point byte sums come from the same registers with dot4
+// instructions — no separate row-sum launch.  What bounds it is a CU's loads: with 16 bytes of 16 different rows on
+// neighbouring lanes, as the 16x16x64 int8 MFMA wants its operands (row lane % 16, k-group lane / 16), every lane was an
+// access of its own and a load took 67 clocks; four lanes of a row next to each other are one access, and a pass through
+// two KB of LDS brings the bytes into the operand layout.  64 x 50 x 5760: 7.4 -> 5.4 us, 128 x 48 x 12288 12.9 -> 8.2, 300 x
+// 1000 x 1024 7.0 -> 5.1, 400 x 400 x 2048 7.8 -> 5.3, 4096 x 50 x 5760 22.7 -> 18.1 (a launch that does nothing: 3 to 4).
+// The partial tiles and sums meet in LDS and wavefront 0 applies the identity of qgemm.hip and the requantize of
+// l-ten/math_fns.cpp:1469-1474.
 //
 // K only has to be a multiple of 16 (k-groups past K read as the zero of the signed domain).
 #include "common.h"
@@ -29,20 +33,26 @@ __device__ __forceinline__ v4i drop_bytes(v4i v, int count)
 }
 
 // RAGGED: the rows of A as they lie, p.K - p.k_pad bytes long and one behind the other, where those of B are padded to p.K.
-template <int WAVES, int OUT, bool RAGGED = false>
+// U: steps in flight per wavefront and pass.
+template <int WAVES, int U, int OUT, bool RAGGED = false>
 __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const int32_t* bias, int coef_a, int coef_b)
 {
-	constexpr int U = 4;  // steps in flight per wavefront and pass
-	__shared__ __attribute__((aligned(16))) int partial[WAVES][64 * 4];
+	__shared__ __attribute__((aligned(16))) uint8_t slabs[WAVES][2048];  // a step of A and of B; a wavefront's sums at the end
 	__shared__ int sums_a[WAVES][16], sums_b[WAVES][16];
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int lrow = lane & 15, lgrp = lane >> 4;
 	const int tiles_n = (p.N + 15) / 16;
 	const int m0 = (blockIdx.x / tiles_n) * 16, n0 = (blockIdx.x % tiles_n) * 16;
-	const bool a_ok = m0 + lrow < p.M, b_ok = n0 + lrow < p.N;
-	const uint8_t* arow = p.A + (int64_t)(m0 + lrow) * p.a_rs + lgrp * 16;
-	const uint8_t* brow = p.B + (int64_t)(n0 + lrow) * p.b_rs + lgrp * 16;
+	// loads: four lanes to a row, 64 bytes next to each other (with 16 rows on neighbouring lanes, as the matrix instruction
+	// wants them, the memory pipeline takes every lane for an access of its own: 67 clocks a load)
+	const int ldrow = lane >> 2, ldgrp = lane & 3;
+	const bool a_ok = m0 + ldrow < p.M, b_ok = n0 + ldrow < p.N;
+	const uint8_t* arow = p.A + (int64_t)(m0 + ldrow) * p.a_rs + ldgrp * 16;
+	const uint8_t* brow = p.B + (int64_t)(n0 + ldrow) * p.b_rs + ldgrp * 16;
+	// through LDS into the operand layout, the four chunks of a row turned so that neither side meets a bank twice
+	uint8_t* const to = slabs[wave] + (ldrow * 4 + (ldgrp ^ (ldrow >> 2))) * 16;
+	const uint8_t* const from = slabs[wave] + (lrow * 4 + (lgrp ^ (lrow >> 2))) * 16;
 	const int steps = (p.K + 63) / 64, real = p.K - p.k_pad;
 	const v4i zero = { (int)0x80808080, (int)0x80808080, (int)0x80808080, (int)0x80808080 };
 	const v4i zero_b = { (int)p.b_flip, (int)p.b_flip, (int)p.b_flip, (int)p.b_flip };  // prepared weights: int8 zeros
@@ -53,7 +63,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 		v4i fa[U], fb[U];
 #pragma unroll
 		for (int u = 0; u < U; u++) {
-			const int k = (s0 + u * WAVES) * 64 + lgrp * 16;
+			const int k = (s0 + u * WAVES) * 64 + ldgrp * 16;
 			fa[u] = zero;
 			fb[u] = zero_b;
 			if (k < p.K) {
@@ -61,7 +71,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 				if (RAGGED && a_ok) {
 					// nothing may be read behind the last row: a row's last chunk is the 16 bytes up to its end, shifted below
 					if (real >= 16) fa[u] = *reinterpret_cast<const v4i_any*>(k + 16 <= real ? a : a - p.k_pad);
-					else if ((m0 + lrow) * real + 16 <= p.M * real) {  // rows shorter than that: some of the next ones too, masked
+					else if ((m0 + ldrow) * real + 16 <= p.M * real) {  // rows shorter than that: some of the next ones too, masked
 						fa[u] = *reinterpret_cast<const v4i_any*>(a);
 #pragma unroll
 						for (int d = 0; d < 4; d++) {
@@ -85,7 +95,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 		}
 #pragma unroll
 		for (int u = 0; u < U; u++) {
-			if (RAGGED && real >= 16 && (s0 + u * WAVES) * 64 + lgrp * 16 == p.K - 16) fa[u] = drop_bytes(fa[u], p.k_pad);
+			if (RAGGED && real >= 16 && (s0 + u * WAVES) * 64 + ldgrp * 16 == p.K - 16) fa[u] = drop_bytes(fa[u], p.k_pad);
 			const v4i a = flip_sign_bits(fa[u]), b = flip_bits(fb[u], p.b_flip);
 			sa = __builtin_amdgcn_sdot4(a.x, 0x01010101, sa, false);
 			sa = __builtin_amdgcn_sdot4(a.y, 0x01010101, sa, false);
@@ -95,15 +105,19 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 			sb = __builtin_amdgcn_sdot4(b.y, 0x01010101, sb, false);
 			sb = __builtin_amdgcn_sdot4(b.z, 0x01010101, sb, false);
 			sb = __builtin_amdgcn_sdot4(b.w, 0x01010101, sb, false);
+			*reinterpret_cast<v4i*>(to) = a;
+			*reinterpret_cast<v4i*>(to + 1024) = b;
+			__builtin_amdgcn_wave_barrier();
+			const v4i ma = *reinterpret_cast<const v4i*>(from), mb = *reinterpret_cast<const v4i*>(from + 1024);
 			// lane (lrow, lgrp), register e holds out[m = 4*lgrp + e][n = lrow]
-			acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, acc, 0, 0, 0);
+			acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ma, mb, acc, 0, 0, 0);
 		}
 	}
-	// a lane holds the byte sums of its 16-byte k-groups only: fold the four k-groups (lanes l, l+16, l+32, l+48)
-	sa += __shfl_xor(sa, 16, 64); sa += __shfl_xor(sa, 32, 64);
-	sb += __shfl_xor(sb, 16, 64); sb += __shfl_xor(sb, 32, 64);
-	if (lane < 16) { sums_a[wave][lane] = sa; sums_b[wave][lane] = sb; }
-	*reinterpret_cast<v4i*>(&partial[wave][lane * 4]) = acc;
+	// a lane holds the byte sums of its 16-byte k-groups only: fold the four lanes of a row
+	sa += __shfl_xor(sa, 1, 64); sa += __shfl_xor(sa, 2, 64);
+	sb += __shfl_xor(sb, 1, 64); sb += __shfl_xor(sb, 2, 64);
+	if (ldgrp == 0) { sums_a[wave][ldrow] = sa; sums_b[wave][ldrow] = sb; }
+	*reinterpret_cast<v4i*>(slabs[wave] + lane * 16) = acc;
 	__syncthreads();
 	if (wave != 0) return;
 
@@ -111,7 +125,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 	int tsa[4] = { 0, 0, 0, 0 }, tsb = 0;
 #pragma unroll
 	for (int w = 0; w < WAVES; w++) {
-		tot += *reinterpret_cast<const v4i*>(&partial[w][lane * 4]);
+		tot += *reinterpret_cast<const v4i*>(slabs[w] + lane * 16);
 		tsb += sums_b[w][lrow];
 #pragma unroll
 		for (int e = 0; e < 4; e++) tsa[e] += sums_a[w][lgrp * 4 + e];
@@ -137,14 +151,15 @@ bool qdirect_takes(const QProblem& p)
 	if (!(p.a_ks == 1 && p.b_ks == 1 && p.vec_ok && p.K % 16 == 0 && p.M >= 1 && p.N >= 1 && p.K >= 1)) return false;
 	const int64_t tiles = (int64_t)ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16);
 	// Up to 8192 tiles, as long as this kernel is ahead of the 128 x 128 direct-to-LDS tiles where those apply (at least
-	// 64 output columns, K >= 512 or at least 64 such tiles: qgemm_dispatch).  It takes about 2.3 us + 4.1 us per million
-	// (tiles x K), they about 5.4 us + 0.33 us per k-step of 128 bytes of a workgroup's share of K while they run in one
+	// 64 output columns, K >= 512 or at least 64 such tiles: qgemm_dispatch).  It takes at most 2.3 us + 3 us per million
+	// (tiles x K) up to a K of 1024 and 3.5 above (4 us and 1.8 in the mean of 40 layers), they about 5.4 us + 0.33 us per k-step of 128 bytes of a workgroup's share of K while they run in one
 	// round, 4 us more when workgroups share tiles (split K, as qgemm_dispatch picks it), 2 us more when N is no multiple
-	// of 4 (rows of the output that start on any byte), 2.5 us more with a partial last k-step.  300 x 1000 x 512: 4.8 us here, 6.9 there; 400 x 400 x 2048: 7.7
-	// and 10.8; 256 x 512 x 4096: 9.4 and 13.8; 200 x 2000 x 256: 4.3 (13.8 on the guarded kernel, which took it before);
-	// 1024 x 1000 x 1024: 16.8 and 8.6; 128 x 4096 x 1024: 9.6 and 7.4; 128 x 1024 x 16384: 30.3 and 23.3.  A few output
+	// of 4 (rows of the output that start on any byte), 2.5 us more with a partial last k-step.  Raw weights, here and there: 851 x
+	// 736 x 896 6.8 and 11.3 us, 393 x 1859 x 1040 12.9 and 16.3, 318 x 1338 x 2192 11.0 and 23.1, 463 x 440 x 5296 12.2 and
+	// 39.1, 1135 x 191 x 6864 21.7 and 52.0, 45 x 2247 x 14160 24.4 and 97.2; 200 x 2000 x 256 4.3 (13.8 on the guarded kernel,
+	// which took it before).  Prepared weights come here only where qgemm_wave_choose leaves them.  A few output
 	// columns make poor use of 128-column tiles and stay here (4096 x 50 x 5760, l-ten's quantized MNIST layer at a large
-	// batch: 22.5 us).
+	// batch: 18.1 us).
 	if (tiles > 8192 || p.K > 16384) return false;
 	const uint64_t tiles128 = ceil_div((uint64_t)p.M, 128) * ceil_div((uint64_t)p.N, 128);
 	// (from 64 output columns on: half-empty 128-column tiles still beat this kernel on long or many rows, 4096 x 100 x 9216 58 -> 25
@@ -153,20 +168,20 @@ bool qdirect_takes(const QProblem& p)
 	                         (uint64_t)p.M * p.K < (1ull << 32) && (uint64_t)p.N * p.K < (1ull << 32);
 	if (tiles_apply) {
 		const int splits = (tiles128 <= 64 && p.K >= 8192) ? (tiles128 <= 32 ? 4 : 2) : (tiles128 <= 32 && p.K >= 4096) ? 2 : 1;
-		const double here = 2.3 + 4.1e-6 * (double)tiles * p.K;
+		const double here = 2.3 + (p.K <= 1024 ? 3.0e-6 : 3.5e-6) * (double)tiles * p.K;
 		const double there = 5.4 + 0.0026 * p.K / splits + (splits > 1 ? 4.0 : 0.0) + (p.N % 4 != 0 ? 2.0 : 0.0) + (p.K % 128 != 0 ? 2.5 : 0.0);
 		if (here >= there) return false;
 	}
 	return true;
 }
 
-template <int WAVES, bool RAGGED = false>
+template <int WAVES, int U, bool RAGGED = false>
 static int launch_qdirect(const QProblem& p, int out, const int32_t* bias, int coef_a, int coef_b)
 {
 	const dim3 grid((unsigned)(ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16))), block(WAVES * 64);
-	if (out == Q_OUT_U8_FAST) qdirect_kernel<WAVES, Q_OUT_U8_FAST, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
-	else if (out == Q_OUT_U8_EXACT) qdirect_kernel<WAVES, Q_OUT_U8_EXACT, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
-	else qdirect_kernel<WAVES, Q_OUT_ACC, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	if (out == Q_OUT_U8_FAST) qdirect_kernel<WAVES, U, Q_OUT_U8_FAST, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	else if (out == Q_OUT_U8_EXACT) qdirect_kernel<WAVES, U, Q_OUT_U8_EXACT, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	else qdirect_kernel<WAVES, U, Q_OUT_ACC, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
 	LTEN_HIP_LAUNCH_CHECK();
 	return 0;
 }
@@ -176,12 +191,24 @@ int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 {
 	if (!qdirect_takes(p)) return -1;
 	const int coef_a = 128 - zp_b, coef_b = 128 - zp_a;
+	// A wavefront alone up to four steps: 2000 x 200 x 256 4.7 -> 4.0 us, 500 x 500 x 256 4.6 -> 4.1; above, the loads of one
+	// wavefront are the longer way (300 x 1000 x 1024: 6.3 with one, 5.0 with four).
+	if (p.K <= 256) {
+		set_kernel_name("qdirect_16x16_w1");
+		return launch_qdirect<1, 4>(p, out, bias, coef_a, coef_b);
+	}
+	// Steps in flight: as many as a wavefront has (2000 x 200 x 256 in four places of which one is used: 5.3 us, in one or two
+	// 4.5), on a longer K the number of the two that leaves fewer places empty (400 x 400 x 2048: 5.3 with four, 5.9 with six; 64 x
+	// 50 x 5760 5.7 and 5.4; 600 x 60 x 8192 6.7 and 6.9; 40 x 40 x 9216 7.4 and 7.0; twelve in flight, or sixteen wavefronts, are behind).
 	if (p.K <= 1024) {
 		set_kernel_name("qdirect_16x16_w4");
-		return launch_qdirect<4>(p, out, bias, coef_a, coef_b);
+		if (p.K <= 512) return launch_qdirect<4, 2>(p, out, bias, coef_a, coef_b);
+		return launch_qdirect<4, 4>(p, out, bias, coef_a, coef_b);
 	}
 	set_kernel_name("qdirect_16x16_w8");
-	return launch_qdirect<8>(p, out, bias, coef_a, coef_b);
+	const int each = (int)ceil_div((uint64_t)p.K, 8 * 64);
+	if ((each + 5) / 6 * 6 <= (each + 3) / 4 * 4) return launch_qdirect<8, 6>(p, out, bias, coef_a, coef_b);
+	return launch_qdirect<8, 4>(p, out, bias, coef_a, coef_b);
 }
 
 // A with rows of K - k_pad bytes (RAGGED) where the padded problem would come here with at most four wavefronts: the copy that
@@ -193,7 +220,8 @@ int qdirect_ragged_dispatch(const QProblem& p, int out, const int32_t* bias, int
 {
 	if (p.K > 1024 || !qdirect_takes(p)) return -1;
 	set_kernel_name("qdirect_16x16_w4");
-	return launch_qdirect<4, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
+	if (p.K <= 256) return launch_qdirect<4, 1, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
+	return launch_qdirect<4, 4, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
 }
 
 }  // namespace lten_hip

@@ -946,6 +946,25 @@ def test_ragged_rows_are_read_as_they_lie(gpu, shape, kernel):
                 assert np.array_equal(dY.numpy(np.uint8, (M, N)), want), (zp, sc, shift)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 16), (15, 17, 240), (16, 16, 256), (33, 20, 272), (17, 31, 512), (31, 18, 528), (16, 48, 1024), (50, 15, 1040),
+                                   (17, 33, 2048), (20, 21, 2576), (64, 50, 5760), (19, 17, 6144), (18, 30, 16384)])
+def test_one_launch_kernel_at_the_edges_of_its_steps(gpu, shape):
+    """One, four and eight wavefronts a tile with one, two, four or six steps of 64 in flight each: the smallest and largest K of each, steps that
+    wavefronts have more or fewer of, a last step of 16 bytes; ragged rows and columns, raw and prepared weights.  Exact."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + 31 * N + K)
+    X, W = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(0, 256, (N, K), dtype=np.uint8)
+    bias, sc, zp = rng.integers(-20000, 20000, N).astype(np.int32), [0.02, 0.02, 0.02 * np.sqrt(K)], [17, 125, 100]
+    mult = np.float32(np.float32(sc[0]) * np.float32(sc[1])) / np.float32(sc[2])
+    want = requant_numpy(exact_acc(X, W, zp[0], zp[1]) + bias[None, :], mult, zp[2])
+    for prepared in (False, True):
+        entry = gpu.lib().lten_hip_fcq_forward_prepared if prepared else gpu.lib().lten_hip_fcq_forward
+        got, kern = fcq(gpu, entry, X, W, sc, zp, bias, prepared=prepared)
+        assert np.array_equal(got, want), (shape, prepared, kern)
+        if N * K < 1 << 19:
+            assert kern == "qdirect_16x16_w" + ("1" if K <= 256 else "4" if K <= 1024 else "8"), kern
+
+
 @pytest.mark.parametrize("K", [*range(1, 16), *range(17, 32), *range(593, 608)])
 def test_ragged_rows_last_chunk_of_every_length(gpu, K):
     """Rows of 1 to 15 bytes, and a last chunk of as many in the first k-step and behind several; 70 rows, the last at the end of the buffer."""
