@@ -44,6 +44,8 @@ double conv2dq_band_us(const ConvGeo& g);
 int conv2dq_pixels_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult,
                             float zp_out, uint8_t* y, void* memory, int forced);
 double conv2dq_pixels_us(const ConvGeo& g, uint64_t& bytes);
+int conv2dq_region_dispatch(const ConvGeo& g, const uint8_t* x, const uint8_t* w, const int32_t* bias, int zp_in, int zp_w, float mult, float zp_out,
+                            uint8_t* y, double limit_us);
 
 // Windows of at most 64 taps in rows of 3 to 8: a thread holds one position's window, a row of a channel in DPR dwords, and takes its
 // dot products with the output channels.  NR = rows it holds, the smallest that covers Cin * kh.
@@ -450,12 +452,21 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	// 14 x 14 -> 32 stays, 7.4 against 8).  Option "conv_variant" 11 to 16 forces a tile.
 	// Layers that one of the kernels of one launch could take leave the caller's workspace as it is, whatever they run as: the
 	// header says so.  What they fill is memory of the library's; the others fill the workspace.
+	// Before that the kernel that has a band of the input and its weights in LDS (convq_region.hip), one launch without memory of
+	// its own, where it is ahead of both by the estimates with the same margin: 32 x 64 x 56 x 56 -> 64 channels 3 x 3 15.7 ->
+	// 11.1 us (two launches), 4 x 8 x 52 x 52 -> 149 9.9 -> 6.2 (bands); 59 x 37 x 16 x 16 -> 39 5 x 5 stays, 9.5 against 12.9, and
+	// 18 x 4 x 12 x 12 -> 61, 5.6 against 5.8.  Option "conv_variant" 20 forces it.
 	if (!out_acc && (variant == 0 || variant > 10) && (variant > 10 || (K <= CQ_MAXK ? Cout >= 48 : !conv2dq_image_takes(g, w)))) {
 		uint64_t bytes = 0;
 		const double here = conv2dq_pixels_us(g, bytes), band_us = conv2dq_band_us(g), band = rows_ahead && K > CQ_MAXK ? -1.0 : band_us;
+		if (variant == 0 || variant == 20) {
+			const double other = std::min(here < 0.0 ? 1e30 : here, band_us < 0.0 ? 1e30 : band_us);
+			const int rc = conv2dq_region_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), variant == 20 ? 1e30 : 0.85 * other);
+			if (rc >= 0) return rc;
+		}
 		const bool one_launch = K <= CQ_MAXK || band_us >= 0.0 || conv2dq_image_takes(g, w);
 		const uint64_t allowed = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);  // (no more than the workspace would hold in any case)
-		if (here >= 0.0 && bytes <= allowed && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
+		if (variant != 20 && here >= 0.0 && bytes <= allowed && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
 			// images in groups whose pixels the library's memory holds, one at least
 			ConvGeo part = g;
 			if (one_launch && bytes > LIBRARY_LIMIT) {

@@ -237,6 +237,40 @@ def test_conv2dq_pixels_tiles_vs_oracle(gpu, ob, geo, tile):
         gpu.set_option("conv_variant", 0)
 
 
+REGION_GEOS = [(1, 16, 8, 16, 32, 3, 3, 1, 1, 1, 1),      # whole chunks, one block of channels
+               (3, 17, 5, 7, 33, 3, 3, 1, 1, 1, 1),       # a channel past a chunk, one past a block; rows shorter than a load
+               (2, 1, 9, 21, 10, 5, 5, 0, 0, 1, 1),       # one channel, an odd number of chunks
+               (2, 20, 19, 11, 65, 5, 5, 2, 2, 2, 2),     # stride 2, a second group with one channel
+               (1, 70, 13, 9, 100, 3, 5, 0, 2, 2, 1),     # five chunks, oblong window, columns the windows do not reach
+               (3, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),     # several blocks of positions, bands that end inside one
+               (2, 250, 6, 6, 40, 1, 1, 0, 0, 1, 1),      # 1 x 1, no border
+               (1, 33, 40, 37, 64, 3, 3, 1, 1, 1, 1),     # odd rows, three chunks
+               (5, 6, 12, 10, 64, 4, 2, 3, 0, 3, 2),      # rows above and below the image, wider than the window reaches
+               (2, 12, 64, 100, 48, 5, 5, 2, 2, 1, 1)]    # more weights in a row than in a chunk, bands of few rows
+
+
+@pytest.mark.parametrize("geo", REGION_GEOS)
+def test_conv2dq_region_vs_oracle(gpu, ob, geo):
+    """The band in LDS, forced: remainders of positions, channels, chunks and k-steps, bands that end early, tensors on and off their
+    alignment, all zero-point forms and both epilogues; the workspace is not touched."""
+    N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw = geo
+    rng = np.random.default_rng(sum(geo) + 3)
+    x = rng.integers(0, 256, (N, Cin, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (Cout, Cin, kh, kw), dtype=np.uint8)
+    Ho, Wo = ob.conv_out_hw(H, W, kh, kw, ph, pw, sh, sw)
+    gpu.set_option("conv_variant", 20)
+    try:
+        for i, (sc, zp, with_bias) in enumerate((([1 / 255, 0.01, 0.05], [0, 128, 128], False), ([0.02, 0.013, 0.9], [17, 250, 100], True),
+                                                 ([1.5, 1.0, 1.0], [200, 3, 9], True), ([1.5, 1.0, 1.0], [7, 128, 9], True))):
+            bias = rng.integers(-9999, 9999, Ho * Wo).astype(np.int32) if with_bias else None
+            want, _ = ob.conv2dq_forward(geo, x, w, sc, zp, bias=bias)
+            got = conv2dq_at(gpu, geo, x, w, sc, zp, bias, i)
+            assert gpu.last_kernel() == "conv2dq_region", (geo, zp, gpu.last_kernel())
+            assert np.array_equal(got.reshape(want.shape), want), (geo, zp)
+    finally:
+        gpu.set_option("conv_variant", 0)
+
+
 @pytest.mark.parametrize("geo", [(8, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), (8, 116, 24, 24, 25, 3, 3, 1, 1, 1, 1), (3, 134, 30, 31, 70, 5, 5, 2, 2, 1, 1),
                                  (6, 100, 33, 35, 60, 3, 3, 1, 1, 2, 2), (24, 17, 64, 64, 96, 1, 1, 0, 0, 1, 1)])
 def test_conv2dq_layers_the_library_sends_to_the_two_launches(gpu, ob, geo):
