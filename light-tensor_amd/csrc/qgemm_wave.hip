@@ -358,7 +358,9 @@ int qgemm_wave_choose(const QProblem& p, bool direct_takes)
 	if (direct_takes) {
 		// the one-launch kernel of qdirect.hip (287 x 960 x 1456: 6.3 -> 4.9 us; 60 x 994 x 6000 stays, 6.3 against 7.4).  Its small
 		// tiles hide the way to HBM better, which shows on a long K (64 x 1000 x 7504, weights from there: 10.3 and 14.6, by the
-		// estimates 0.80; 128 x 490 x 6016 8.6 and 10.4; 128 x 1000 x 6000, 0.66, 1.2 times ahead)
+		// estimates 0.80; 128 x 490 x 6016 8.6 and 10.4; 128 x 1000 x 6000, 0.66, 1.2 times ahead).  The pairs are from before that
+		// kernel's loads took four lanes a row; since then the line holds over 50 layers (95 x 1972 x 4976 7.0 here and 10.6 there, 467 x
+		// 557 x 4880 9.2 and 16.3, 1368 x 194 x 2176 7.2 and 8.4; short K: 392 x 1825 x 704 7.7 and 7.4)
 		const double direct = 1.5 + 2.1e-6 * tiles16 * p.K + 0.59 * kk + 0.55 * tiles16 / 1024;
 		return best < (p.K > 6000 ? 0.79 : 0.85) * direct ? variant : 0;
 	}
