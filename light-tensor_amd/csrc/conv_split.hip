@@ -673,7 +673,6 @@ int split_run(SplitConv& p, double limit_us, int forced)
 		}
 	}
 	if (best < 0) return -1;
-	split_layout(p, split_tiles[best]);
 	int64_t packed = 0;
 	for (int k = 0; k < p.classes; k++) {
 		p.cls[k].packed = packed;
@@ -683,31 +682,41 @@ int split_run(SplitConv& p, double limit_us, int forced)
 	int tap_groups = 1;
 	for (int k = 0; k < p.classes; k++) tap_groups = std::max(tap_groups, (p.cls[k].kh * p.cls[k].kw + 3) / 4);
 	packed += 3 * 3072;  // (read, not used, where the last block's loads run ahead)
+	// Planes of less than a quad are staged from a copy with a quad each, of as many images at a time as 512 MB hold: a load's offset
+	// is a 32-bit number of bytes, in the copy as in the tensor.
 	const int hw = p.H * p.W;
-	p.src = p.x;
+	const int group = hw < 4 ? (int)std::min<uint64_t>((uint64_t)p.N, std::max<uint64_t>(1, (512ull << 20) / (16ull * p.C))) : p.N;
 	p.plane = std::max(hw, 4);
-	uint8_t* scratch = static_cast<uint8_t*>(library_scratch((uint64_t)packed + (hw < 4 ? 16ull * p.N * p.C : 0)));
+	uint8_t* scratch = static_cast<uint8_t*>(library_scratch((uint64_t)packed + (hw < 4 ? 16ull * group * p.C : 0)));
 	if (scratch == nullptr) return -1;
-	if (hw < 4) {  // planes of less than a quad: one each in a copy
-		float* copy = reinterpret_cast<float*>(scratch + packed);
-		pad_planes_kernel<<<dim3((unsigned)ceil_div((uint64_t)p.N * p.C, 256)), dim3(256), 0, stream()>>>(p.x, copy, p.N * p.C, hw);
-		LTEN_HIP_LAUNCH_CHECK();
-		p.src = copy;
-	}
 	conv_split_pack_kernel<<<dim3((unsigned)p.chunks, (unsigned)cobs, (unsigned)(p.classes * tap_groups)), dim3(256), 0, stream()>>>(p, scratch);
 	LTEN_HIP_LAUNCH_CHECK();
 	p.wp = scratch;
 	const bool t3 = split_t3(p);
-	switch (best) {
-	case 0: launch_split<64, 512, 1, 4, 210>(p, t3); break;
-	case 1: launch_split<32, 512, 1, 4, 210>(p, t3); break;
-	case 2: launch_split<128, 256, 2, 2, 162>(p, t3); break;
-	case 3: launch_split<64, 256, 1, 4, 162>(p, t3); break;
-	case 4: launch_split<32, 256, 1, 4, 162>(p, t3); break;
-	case 5: launch_split<64, 128, 2, 2, 98>(p, t3); break;
-	default: launch_split<64, 128, 2, 2, 210>(p, t3); break;
+	const float* const x = p.x;
+	float* const y = p.y;
+	for (int n = 0, N = p.N; n < N; n += group) {
+		p.N = std::min(group, N - n);
+		p.x = p.src = x + (int64_t)n * p.C * hw;
+		p.y = y + (int64_t)n * p.M * p.out_plane;
+		split_layout(p, split_tiles[best]);
+		if (hw < 4) {
+			float* copy = reinterpret_cast<float*>(scratch + packed);
+			pad_planes_kernel<<<dim3((unsigned)ceil_div((uint64_t)p.N * p.C, 256)), dim3(256), 0, stream()>>>(p.x, copy, p.N * p.C, hw);
+			LTEN_HIP_LAUNCH_CHECK();
+			p.src = copy;
+		}
+		switch (best) {
+		case 0: launch_split<64, 512, 1, 4, 210>(p, t3); break;
+		case 1: launch_split<32, 512, 1, 4, 210>(p, t3); break;
+		case 2: launch_split<128, 256, 2, 2, 162>(p, t3); break;
+		case 3: launch_split<64, 256, 1, 4, 162>(p, t3); break;
+		case 4: launch_split<32, 256, 1, 4, 162>(p, t3); break;
+		case 5: launch_split<64, 128, 2, 2, 98>(p, t3); break;
+		default: launch_split<64, 128, 2, 2, 210>(p, t3); break;
+		}
+		LTEN_HIP_LAUNCH_CHECK();
 	}
-	LTEN_HIP_LAUNCH_CHECK();
 	return 0;
 }
 

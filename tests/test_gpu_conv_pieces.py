@@ -420,3 +420,29 @@ def test_weight_gradient_staging_on_integers(gpu, geo):
     x = rng.integers(-8, 9, geo[:4]).astype(np.float32)
     dy = rng.integers(-8, 9, (geo[0], geo[4], *out_hw(geo))).astype(np.float32)
     assert np.array_equal(run_wgrad(gpu, geo, x, dy), wgrad64(geo, x, dy))
+
+
+@pytest.mark.parametrize("entry", ["forward", "dgrad"])
+def test_planes_of_less_than_a_quad_in_groups_of_images(gpu, entry):
+    """2100 images of 16384 planes of one value: the copy that they are staged from holds 2048 images at a time.  Exact in any order
+    (a window meets a plane with its centre tap only)."""
+    N, C, M = 2100, 16384, 40
+    rng = np.random.default_rng(N)
+    t = rng.integers(-8, 9, (N, C), dtype=np.int8).astype(np.float32)
+    w = rng.integers(-8, 9, (M, C, 3, 3) if entry == "forward" else (C, M, 3, 3), dtype=np.int8).astype(np.float32)
+    bias = rng.integers(-8, 9, M).astype(np.float32)
+    D, l = gpu.DeviceBuffer, gpu.lib()
+    dT, dW, dB, out = D.from_numpy(t), D.from_numpy(w), D.from_numpy(bias), D.from_numpy(np.full((N, M), 7, np.float32))
+    gpu.set_option("conv_variant", 10)
+    try:
+        if entry == "forward":
+            gpu.check(l.lten_hip_conv2d_forward_f32(N, C, 1, 1, M, 3, 3, 1, 1, 1, 1, dT.ptr, dW.ptr, dB.ptr, out.ptr))
+        else:
+            geo = (N, M, 1, 1, C, 3, 3, 1, 1, 1, 1)
+            ws = D(max(int(l.lten_hip_conv2d_dgrad_workspace_bytes(*geo)), 16))
+            gpu.check(l.lten_hip_conv2d_dgrad_f32(*geo, dW.ptr, dT.ptr, out.ptr, ws.ptr))
+        assert gpu.last_kernel() == f"conv2d_pieces_{entry}"
+    finally:
+        gpu.set_option("conv_variant", 0)
+    want = t @ w[:, :, 1, 1].T + bias if entry == "forward" else t @ w[:, :, 1, 1]
+    assert np.array_equal(out.numpy(np.float32, (N, M)), want)

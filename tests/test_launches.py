@@ -1,0 +1,59 @@
+"""What the entry points would launch, seen without a GPU: calls at sizes no test could run, on a stand-in for the HIP runtime
+(hip_stub.c).  A process of its own, since the library takes the runtime it is loaded with."""
+import ctypes as C
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+DEVICE = lambda k: k << 40   # an address that nothing reads
+
+
+@pytest.fixture(scope="module")
+def launches(lt, tmp_path_factory):
+    """launches(entry point, arguments) -> {"rc", "error", "kernel", "launches": [[kernel, grid x, y, z, threads, LDS], ...]}.  An
+    argument {"qparams": [scales, zero points]} stands for lten_hip_qparams."""
+    stub = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", stub, os.path.join(HERE, "hip_stub.c")], check=True)
+
+    def run(name, *args):
+        out = subprocess.run([sys.executable, __file__, stub, name, json.dumps(args)], check=True, stdout=subprocess.PIPE, text=True)
+        return json.loads(out.stdout.splitlines()[-1])
+    return run
+
+
+def call_on_the_stub(stub_path, name, args):
+    stub = C.CDLL(stub_path, mode=C.RTLD_GLOBAL)   # before the library, whose HIP calls it takes
+    stub.stub_name.restype = C.c_char_p
+    sys.path.insert(0, HERE)
+    from conftest import load_package
+    lt = load_package()
+    rc = getattr(lt.lib(), name)(*[lt.qparams3(*a["qparams"]) if isinstance(a, dict) else a for a in args])
+    seen, dims = [], (C.c_uint64 * 5)()
+    for i in range(stub.stub_launches()):
+        stub.stub_dims(i, dims)
+        seen.append([stub.stub_name(i).decode(), *dims])
+    return {"rc": rc, "error": (lt.lib().lten_hip_last_error() or b"").decode() if rc else "", "kernel": lt.last_kernel(), "launches": seen}
+
+
+@pytest.mark.parametrize("N,C_in,H,W", [(65535, 4100, 1, 1), (1100, 1 << 18, 1, 3), (65535, 2, 2, 1)])
+@pytest.mark.parametrize("entry", ["forward", "dgrad"])
+def test_planes_of_less_than_a_quad_stay_within_32_bits(launches, entry, N, C_in, H, W):
+    """Such planes are staged from a copy with four values each, by offsets of 32 bits: no part of it may reach 2^32 bytes, and
+    the parts are all planes."""
+    if entry == "forward":
+        r = launches("lten_hip_conv2d_forward_f32", N, C_in, H, W, 64, 3, 3, 1, 1, 1, 1, DEVICE(1), DEVICE(2), None, DEVICE(3))
+    else:
+        r = launches("lten_hip_conv2d_dgrad_f32", N, 64, H, W, C_in, 3, 3, 1, 1, 1, 1, DEVICE(1), DEVICE(2), DEVICE(3), DEVICE(4))
+    assert r["rc"] == 0, r["error"]
+    copies = [x * threads for name, x, _, _, threads, _ in r["launches"] if "pad_planes" in name]
+    assert ("pieces" in r["kernel"]) == bool(copies), r["kernel"]
+    assert all(planes * 16 <= 1 << 32 for planes in copies), copies
+    assert not copies or N * C_in <= sum(copies) < N * C_in + 256 * len(copies)
+
+
+if __name__ == "__main__":
+    print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
