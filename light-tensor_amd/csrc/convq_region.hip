@@ -384,7 +384,7 @@ static bool region_plan(const ConvGeo& g, RegionPlan& pl, double limit_us)
 			const int inside = std::min(top + (rows - 1) * g.sh + g.kh, g.H) - std::max(top, 0);
 			whole = whole && inside > 0 && (int64_t)inside * g.W >= 16;
 		}
-		if (!whole || (int64_t)g.N * bands >= (1ll << 31)) continue;
+		if (!whole || (int64_t)g.N * bands >= (1ll << 32) / 512) continue;  // (HIP launches fewer than 2^32 threads in a dimension)
 		const int fn = pl.rows == 64 && pairs > 4 ? 2 : 1;
 		const int units = pairs * (pl.rows / (32 * fn)), turns = (units + 7) / 8;
 		const double rounds = std::ceil((double)g.N * bands * pl.groups / 256.0);

@@ -55,5 +55,18 @@ def test_planes_of_less_than_a_quad_stay_within_32_bits(launches, entry, N, C_in
     assert not copies or N * C_in <= sum(copies) < N * C_in + 256 * len(copies)
 
 
+QP = {"qparams": [[0.02, 0.013, 0.9], [17, 125, 100]]}
+
+
+@pytest.mark.parametrize("geo", [(65535, 8, 16000, 9, 1, 3, 3, 1, 1, 1, 1),       # bands of a few rows, many of them
+                                 (16297, 5, 5225, 479, 124, 3, 3, 0, 2, 1, 1),
+                                 (38160, 4, 2927, 152, 71, 2, 2, 1, 1, 1, 1),     # at most 64 taps
+                                 (27108, 284, 3000, 29, 4, 3, 3, 2, 1, 1, 2)])    # no other kernel of one launch
+def test_conv2dq_of_very_many_bands(launches, geo):
+    """2^23 bands of 512 threads and more are no launch: the other kernels take the layer, or the same one with taller bands."""
+    r = launches("lten_hip_conv2dq_forward", *geo, DEVICE(1), DEVICE(2), None, QP, DEVICE(3), DEVICE(4))
+    assert r["rc"] == 0, r["error"]
+
+
 if __name__ == "__main__":
     print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
