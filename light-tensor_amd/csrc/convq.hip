@@ -459,14 +459,14 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	if (!out_acc && (variant == 0 || variant > 10) && (variant > 10 || (K <= CQ_MAXK ? Cout >= 48 : !conv2dq_image_takes(g, w)))) {
 		uint64_t bytes = 0;
 		const double here = conv2dq_pixels_us(g, bytes), band_us = conv2dq_band_us(g), band = rows_ahead && K > CQ_MAXK ? -1.0 : band_us;
-		if (variant == 0 || variant == 20) {
+		const bool one_launch = K <= CQ_MAXK || band_us >= 0.0 || conv2dq_image_takes(g, w);
+		if ((variant == 0 || variant == 20) && (one_launch || workspace != nullptr)) {  // (the other layers' contract wants a workspace, whatever they run as)
 			// (two launches that the estimate has at its least, 8.1 us, were 8.6 to 9.1 over 20 such layers: 4 x 52 x 16 x 16 -> 82 8.8 us
 			// and 7.0 here, 8 x 138 x 27 x 27 -> 117 1 x 1 8.6 and 7.1, 30 x 56 x 13 x 13 -> 72 8.8 and 7.5)
 			const double other = std::min(here < 0.0 ? 1e30 : std::max(here, 8.6), band_us < 0.0 ? 1e30 : band_us);
 			const int rc = conv2dq_region_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), variant == 20 ? 1e30 : 0.85 * other);
 			if (rc >= 0) return rc;
 		}
-		const bool one_launch = K <= CQ_MAXK || band_us >= 0.0 || conv2dq_image_takes(g, w);
 		const uint64_t allowed = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);  // (no more than the workspace would hold in any case)
 		if (variant != 20 && here >= 0.0 && bytes <= allowed && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
 			// images in groups whose pixels the library's memory holds, one at least

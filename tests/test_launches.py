@@ -68,5 +68,16 @@ def test_conv2dq_of_very_many_bands(launches, geo):
     assert r["rc"] == 0, r["error"]
 
 
+@pytest.mark.parametrize("geo,kernel", [((4, 128, 120, 120, 32, 3, 3, 1, 1, 1, 1), "conv2dq_region"),
+                                        ((127, 50, 10, 92, 15, 5, 5, 2, 4, 1, 1), "conv2dq_region"),
+                                        ((64, 256, 100, 100, 256, 3, 3, 1, 1, 1, 1), "conv2dq_pixels")])
+def test_conv2dq_layers_that_want_a_workspace(launches, geo, kernel):
+    """Windows without a plan of one launch in 64 KB of LDS are refused without a workspace, whatever they run as with one."""
+    r = launches("lten_hip_conv2dq_forward", *geo, DEVICE(1), DEVICE(2), None, QP, DEVICE(3), None)
+    assert (r["rc"], r["error"]) == (2, "conv2dq: workspace is null")
+    r = launches("lten_hip_conv2dq_forward", *geo, DEVICE(1), DEVICE(2), None, QP, DEVICE(3), DEVICE(4))
+    assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
+
+
 if __name__ == "__main__":
     print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
