@@ -4,11 +4,11 @@
 // and memory latency, not arithmetic, so the kernel is one dependent chain as short as possible: a workgroup
 // owns one 16 x 16 output tile, its wavefronts split K in 64-byte steps (wavefront w takes steps w, w + WAVES,
 // ...), the loads of U of its steps at once, and the zero-point byte sums come from the same registers with dot4
-// instructions — no separate row-sum launch.  What bounds it is a CU's loads: with 16 bytes of 16 different rows on
-// neighbouring lanes, as the 16x16x64 int8 MFMA wants its operands (row lane % 16, k-group lane / 16), every lane was an
-// access of its own and a load took 67 clocks; four lanes of a row next to each other are one access, and a pass through
-// two KB of LDS brings the bytes into the operand layout.  64 x 50 x 5760: 7.4 -> 5.4 us, 128 x 48 x 12288 12.9 -> 8.2, 300 x
-// 1000 x 1024 7.0 -> 5.1, 400 x 400 x 2048 7.8 -> 5.3, 4096 x 50 x 5760 22.7 -> 18.1 (a launch that does nothing: 3 to 4).
+// instructions — no separate row-sum launch.  What bounds it is a CU's loads.  The 16x16x64 int8 MFMA wants 16 bytes of 16
+// different rows on neighbouring lanes (row lane % 16, k-group lane / 16); loaded like that, rows a multiple of 128 bytes apart
+// are slow.  There four lanes of a row load next to each other, and a pass through two KB of LDS brings the bytes into the
+// operand layout (64 x 50 x 5760: 7.3 -> 5.2 us, 128 x 48 x 12288 12.7 -> 8.2, 300 x 1000 x 1024 6.8 -> 4.7, 400 x 400 x 2048 7.7 -> 5.1,
+// 4096 x 50 x 5760 22.6 -> 17.9; a launch that does nothing: 3 to 4); qdirect_dispatch has the line.
 // The partial tiles and sums meet in LDS and wavefront 0 applies the identity of qgemm.hip and the requantize of
 // l-ten/math_fns.cpp:1469-1474.
 //
@@ -33,8 +33,8 @@ __device__ __forceinline__ v4i drop_bytes(v4i v, int count)
 }
 
 // RAGGED: the rows of A as they lie, p.K - p.k_pad bytes long and one behind the other, where those of B are padded to p.K.
-// U: steps in flight per wavefront and pass.
-template <int WAVES, int U, int OUT, bool RAGGED = false>
+// U: steps in flight per wavefront and pass.  DIRECT: operands loaded as the matrix instruction takes them, not through LDS.
+template <int WAVES, int U, int OUT, bool RAGGED = false, bool DIRECT = false>
 __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const int32_t* bias, int coef_a, int coef_b)
 {
 	__shared__ __attribute__((aligned(16))) uint8_t slabs[WAVES][2048];  // a step of A and of B; a wavefront's sums at the end
@@ -44,9 +44,8 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 	const int lrow = lane & 15, lgrp = lane >> 4;
 	const int tiles_n = (p.N + 15) / 16;
 	const int m0 = (blockIdx.x / tiles_n) * 16, n0 = (blockIdx.x % tiles_n) * 16;
-	// loads: four lanes to a row, 64 bytes next to each other (with 16 rows on neighbouring lanes, as the matrix instruction
-	// wants them, the memory pipeline takes every lane for an access of its own: 67 clocks a load)
-	const int ldrow = lane >> 2, ldgrp = lane & 3;
+	// loads: in the operand layout, or four lanes to a row, 64 bytes next to each other
+	const int ldrow = DIRECT ? lrow : lane >> 2, ldgrp = DIRECT ? lgrp : lane & 3;
 	const bool a_ok = m0 + ldrow < p.M, b_ok = n0 + ldrow < p.N;
 	const uint8_t* arow = p.A + (int64_t)(m0 + ldrow) * p.a_rs + ldgrp * 16;
 	const uint8_t* brow = p.B + (int64_t)(n0 + ldrow) * p.b_rs + ldgrp * 16;
@@ -59,8 +58,7 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 
 	v4i acc = { 0, 0, 0, 0 };
 	int sa = 0, sb = 0;
-	for (int s0 = wave; s0 < steps; s0 += WAVES * U) {
-		v4i fa[U], fb[U];
+	auto fetch = [&](int s0, v4i (&fa)[U], v4i (&fb)[U]) {
 #pragma unroll
 		for (int u = 0; u < U; u++) {
 			const int k = (s0 + u * WAVES) * 64 + ldgrp * 16;
@@ -93,10 +91,25 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 				if (b_ok) fb[u] = *reinterpret_cast<const v4i*>(brow + (int64_t)(s0 + u * WAVES) * 64);
 			}
 		}
-#pragma unroll
-		for (int u = 0; u < U; u++) {
+	};
+	// A step's operands are asked for back from LDS before the step before is multiplied (LDS serves a wavefront in order, so one
+	// slab does): with each step waiting for its own, the way through LDS stood in the chain once a step.
+	auto multiply = [&](int s0, v4i (&fa)[U], v4i (&fb)[U]) {
+		v4i ma[2], mb[2];
+		auto exchange = [&](int u) {
 			if (RAGGED && real >= 16 && (s0 + u * WAVES) * 64 + ldgrp * 16 == p.K - 16) fa[u] = drop_bytes(fa[u], p.k_pad);
 			const v4i a = flip_sign_bits(fa[u]), b = flip_bits(fb[u], p.b_flip);
+			if (DIRECT) {
+				ma[u & 1] = a;
+				mb[u & 1] = b;
+			} else {
+				*reinterpret_cast<v4i*>(to) = a;
+				*reinterpret_cast<v4i*>(to + 1024) = b;
+				__builtin_amdgcn_wave_barrier();
+				ma[u & 1] = *reinterpret_cast<const v4i*>(from);
+				mb[u & 1] = *reinterpret_cast<const v4i*>(from + 1024);
+				__builtin_amdgcn_wave_barrier();
+			}
 			sa = __builtin_amdgcn_sdot4(a.x, 0x01010101, sa, false);
 			sa = __builtin_amdgcn_sdot4(a.y, 0x01010101, sa, false);
 			sa = __builtin_amdgcn_sdot4(a.z, 0x01010101, sa, false);
@@ -105,17 +118,24 @@ __global__ __launch_bounds__(WAVES * 64) void qdirect_kernel(QProblem p, const i
 			sb = __builtin_amdgcn_sdot4(b.y, 0x01010101, sb, false);
 			sb = __builtin_amdgcn_sdot4(b.z, 0x01010101, sb, false);
 			sb = __builtin_amdgcn_sdot4(b.w, 0x01010101, sb, false);
-			*reinterpret_cast<v4i*>(to) = a;
-			*reinterpret_cast<v4i*>(to + 1024) = b;
-			__builtin_amdgcn_wave_barrier();
-			const v4i ma = *reinterpret_cast<const v4i*>(from), mb = *reinterpret_cast<const v4i*>(from + 1024);
+		};
+		exchange(0);
+#pragma unroll
+		for (int u = 0; u < U; u++) {
+			if (u + 1 < U) exchange(u + 1);
 			// lane (lrow, lgrp), register e holds out[m = 4*lgrp + e][n = lrow]
-			acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ma, mb, acc, 0, 0, 0);
+			acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ma[u & 1], mb[u & 1], acc, 0, 0, 0);
 		}
+	};
+	for (int s0 = wave; s0 < steps; s0 += WAVES * U) {
+		v4i fa[U], fb[U];
+		fetch(s0, fa, fb);
+		multiply(s0, fa, fb);
 	}
 	// a lane holds the byte sums of its 16-byte k-groups only: fold the four lanes of a row
-	sa += __shfl_xor(sa, 1, 64); sa += __shfl_xor(sa, 2, 64);
-	sb += __shfl_xor(sb, 1, 64); sb += __shfl_xor(sb, 2, 64);
+	constexpr int FOLD = DIRECT ? 16 : 1;
+	sa += __shfl_xor(sa, FOLD, 64); sa += __shfl_xor(sa, 2 * FOLD, 64);
+	sb += __shfl_xor(sb, FOLD, 64); sb += __shfl_xor(sb, 2 * FOLD, 64);
 	if (ldgrp == 0) { sums_a[wave][ldrow] = sa; sums_b[wave][ldrow] = sb; }
 	*reinterpret_cast<v4i*>(slabs[wave] + lane * 16) = acc;
 	__syncthreads();
@@ -151,8 +171,10 @@ bool qdirect_takes(const QProblem& p)
 	if (!(p.a_ks == 1 && p.b_ks == 1 && p.vec_ok && p.K % 16 == 0 && p.M >= 1 && p.N >= 1 && p.K >= 1)) return false;
 	const int64_t tiles = (int64_t)ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16);
 	// Up to 8192 tiles, as long as this kernel is ahead of the 128 x 128 direct-to-LDS tiles where those apply (at least
-	// 64 output columns, K >= 512 or at least 64 such tiles: qgemm_dispatch).  It takes at most 2.3 us + 3 us per million
-	// (tiles x K) up to a K of 1024 and 3.5 above (4 us and 1.8 in the mean of 40 layers), they about 5.4 us + 0.33 us per k-step of 128 bytes of a workgroup's share of K while they run in one
+	// 64 output columns, K >= 512 or at least 64 such tiles: qgemm_dispatch).  Its estimate is 2.3 us + 3 us per million
+	// (tiles x K), 3.5 above a K of 1024.  From 64 tiles up it takes 0.6 to 1.9 times that (over 930 layers; 0.8 to 1.3 in the median of a
+	// range of sizes).  Below, the chain over K counts, which has no term, and it takes up to four times that (8 us for one tile at K =
+	// 16320): there they take longer still.  They take about 5.4 us + 0.33 us per k-step of 128 bytes of a workgroup's share of K while they run in one
 	// round, 4 us more when workgroups share tiles (split K, as qgemm_dispatch picks it), 2 us more when N is no multiple
 	// of 4 (rows of the output that start on any byte), 2.5 us more with a partial last k-step.  Raw weights, here and there: 851 x
 	// 736 x 896 6.8 and 11.3 us, 393 x 1859 x 1040 12.9 and 16.3, 318 x 1338 x 2192 11.0 and 23.1, 463 x 440 x 5296 12.2 and
@@ -175,13 +197,13 @@ bool qdirect_takes(const QProblem& p)
 	return true;
 }
 
-template <int WAVES, int U, bool RAGGED = false>
+template <int WAVES, int U, bool RAGGED = false, bool DIRECT = false>
 static int launch_qdirect(const QProblem& p, int out, const int32_t* bias, int coef_a, int coef_b)
 {
 	const dim3 grid((unsigned)(ceil_div((uint64_t)p.M, 16) * ceil_div((uint64_t)p.N, 16))), block(WAVES * 64);
-	if (out == Q_OUT_U8_FAST) qdirect_kernel<WAVES, U, Q_OUT_U8_FAST, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
-	else if (out == Q_OUT_U8_EXACT) qdirect_kernel<WAVES, U, Q_OUT_U8_EXACT, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
-	else qdirect_kernel<WAVES, U, Q_OUT_ACC, RAGGED><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	if (out == Q_OUT_U8_FAST) qdirect_kernel<WAVES, U, Q_OUT_U8_FAST, RAGGED, DIRECT><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	else if (out == Q_OUT_U8_EXACT) qdirect_kernel<WAVES, U, Q_OUT_U8_EXACT, RAGGED, DIRECT><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
+	else qdirect_kernel<WAVES, U, Q_OUT_ACC, RAGGED, DIRECT><<<grid, block, 0, stream()>>>(p, bias, coef_a, coef_b);
 	LTEN_HIP_LAUNCH_CHECK();
 	return 0;
 }
@@ -191,24 +213,33 @@ int qdirect_dispatch(const QProblem& p, int out, const int32_t* bias, int zp_a, 
 {
 	if (!qdirect_takes(p)) return -1;
 	const int coef_a = 128 - zp_b, coef_b = 128 - zp_a;
-	// A wavefront alone up to four steps: 2000 x 200 x 256 4.7 -> 4.0 us, 500 x 500 x 256 4.6 -> 4.1; above, the loads of one
-	// wavefront are the longer way (300 x 1000 x 1024: 6.3 with one, 5.0 with four).
+	// Two steps of a wavefront in flight: places that a wavefront's share of K leaves empty cost more than what they hide (432 x 1406 x
+	// 1056: 9.3 us with two, 11.0 with four).  A wavefront alone up to K = 256 (2000 x 200 x 256: 3.6, 4.1 with four wavefronts), four up to
+	// 1024 (300 x 1000 x 1024: 4.7, 5.4 with eight; one 6.3), eight above (400 x 400 x 2048: 5.1, 5.3 with four).
 	if (p.K <= 256) {
 		set_kernel_name("qdirect_16x16_w1");
-		return launch_qdirect<1, 4>(p, out, bias, coef_a, coef_b);
+		return launch_qdirect<1, 2>(p, out, bias, coef_a, coef_b);
 	}
-	// Steps in flight: as many as a wavefront has (2000 x 200 x 256 in four places of which one is used: 5.3 us, in one or two
-	// 4.5), on a longer K the number of the two that leaves fewer places empty (400 x 400 x 2048: 5.3 with four, 5.9 with six; 64 x
-	// 50 x 5760 5.7 and 5.4; 600 x 60 x 8192 6.7 and 6.9; 40 x 40 x 9216 7.4 and 7.0; twelve in flight, or sixteen wavefronts, are behind).
+	// Operands through LDS where rows lie a multiple of 128 bytes apart (300 x 1000 x 1024: 6.8 us in the operand layout, 4.7 through
+	// LDS; 400 x 400 x 2048 7.5 and 5.1).  On other lengths the operand layout is as quick or quicker up to K = 2048 (219 x 2203 x 752:
+	// 5.6 and 6.1; 432 x 1406 x 1056: 8.4 and 9.3) and slower above (53 x 1183 x 5392: 8.6 and 7.4; 145 x 861 x 5680 11.4 and 9.3), but
+	// where one operand has few rows, whose loads are few accesses either way, the pass through LDS is a longer chain (3 x 15 x 4256:
+	// 3.9 and 4.2; 2961 x 1 x 16336: 10.7 and 12.5).  Against the operand layout with four steps in flight everywhere, over 930 layers:
+	// 0.915 of the time in the mean, 11 of them 3 to 6 % behind.
+	const bool lines = p.K % 128 == 0, few = std::min(p.M, p.N) <= 12;
+	const bool direct = lines ? few && p.K <= 4096 : few || p.K <= 2048;
 	if (p.K <= 1024) {
 		set_kernel_name("qdirect_16x16_w4");
-		if (p.K <= 512) return launch_qdirect<4, 2>(p, out, bias, coef_a, coef_b);
-		return launch_qdirect<4, 4>(p, out, bias, coef_a, coef_b);
+		if (direct) return launch_qdirect<4, 2, false, true>(p, out, bias, coef_a, coef_b);
+		return launch_qdirect<4, 2>(p, out, bias, coef_a, coef_b);
 	}
+	// (four steps in flight on the longest chains: 2961 x 1 x 16336 11.7 us with two, 10.7 with four; 4096 x 50 x 5760 18.9 and 17.9; not
+	// through LDS on other lengths, 85 x 612 x 9168 9.3 and 9.9)
 	set_kernel_name("qdirect_16x16_w8");
-	const int each = (int)ceil_div((uint64_t)p.K, 8 * 64);
-	if ((each + 5) / 6 * 6 <= (each + 3) / 4 * 4) return launch_qdirect<8, 6>(p, out, bias, coef_a, coef_b);
-	return launch_qdirect<8, 4>(p, out, bias, coef_a, coef_b);
+	if (direct && p.K > 8192) return launch_qdirect<8, 4, false, true>(p, out, bias, coef_a, coef_b);
+	if (direct) return launch_qdirect<8, 2, false, true>(p, out, bias, coef_a, coef_b);
+	if (lines && p.K > 4096) return launch_qdirect<8, 4>(p, out, bias, coef_a, coef_b);
+	return launch_qdirect<8, 2>(p, out, bias, coef_a, coef_b);
 }
 
 // A with rows of K - k_pad bytes (RAGGED) where the padded problem would come here with at most four wavefronts: the copy that
@@ -221,6 +252,7 @@ int qdirect_ragged_dispatch(const QProblem& p, int out, const int32_t* bias, int
 	if (p.K > 1024 || !qdirect_takes(p)) return -1;
 	set_kernel_name("qdirect_16x16_w4");
 	if (p.K <= 256) return launch_qdirect<4, 1, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
+	if (p.K <= 512) return launch_qdirect<4, 2, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
 	return launch_qdirect<4, 4, true>(p, out, bias, 128 - zp_b, 128 - zp_a);
 }
 

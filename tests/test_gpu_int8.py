@@ -921,7 +921,7 @@ def test_long_reductions_and_many_columns_stay_off_the_tiles_that_share_k(gpu, k
 
 
 @pytest.mark.parametrize("shape,kernel", [((64, 10, 50), "w4"), ((17, 33, 1001), "w4"), ((3, 5, 7), "w4"), ((1, 16, 15), "w4"), ((16, 17, 1007), "w4"),
-                                          ((100, 30, 33), "w4"), ((130, 258, 1020), "w4")])
+                                          ((100, 30, 33), "w4"), ((130, 258, 1020), "w4"), ((20, 35, 257), "w4"), ((33, 18, 511), "w4")])
 def test_ragged_rows_are_read_as_they_lie(gpu, shape, kernel):
     """Small outputs of prepared weights whose activation rows are no multiple of 16 bytes, on and off a 16-byte boundary: one load, a
     last chunk of 1 to 15 bytes, nothing but that; every zero-point form."""
@@ -947,10 +947,12 @@ def test_ragged_rows_are_read_as_they_lie(gpu, shape, kernel):
 
 
 @pytest.mark.parametrize("shape", [(1, 1, 16), (15, 17, 240), (16, 16, 256), (33, 20, 272), (17, 31, 512), (31, 18, 528), (16, 48, 1024), (50, 15, 1040),
-                                   (17, 33, 2048), (20, 21, 2576), (64, 50, 5760), (19, 17, 6144), (18, 30, 16384)])
+                                   (17, 33, 2048), (20, 21, 2576), (64, 50, 5760), (19, 17, 6144), (18, 30, 16384),
+                                   (30, 12, 4096), (12, 30, 8176), (30, 12, 4224), (40, 7, 8208), (9, 40, 16368), (18, 30, 16368), (20, 13, 2064), (3, 40, 272)])
 def test_one_launch_kernel_at_the_edges_of_its_steps(gpu, shape):
-    """One, four and eight wavefronts a tile with one, two, four or six steps of 64 in flight each: the smallest and largest K of each, steps that
-    wavefronts have more or fewer of, a last step of 16 bytes; ragged rows and columns, raw and prepared weights.  Exact."""
+    """One, four and eight wavefronts a tile with two or four steps of 64 in flight each, operands through LDS and in the operand layout: the
+    smallest and largest K of each, steps that wavefronts have more or fewer of, a last step of 16 bytes; ragged rows and columns, raw
+    and prepared weights.  Exact."""
     M, N, K = shape
     rng = np.random.default_rng(M + 31 * N + K)
     X, W = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(0, 256, (N, K), dtype=np.uint8)
