@@ -448,27 +448,26 @@ static int conv2dq_run(uint64_t N, uint64_t Cin, uint64_t H, uint64_t W, uint64_
 	// Bytes out of a layer with some work: pixels of channels and an implicit GEMM (convq_pixels.hip; int32 sums, which only
 	// checks ask for, keep the kernels below).  Ahead of the three launches and of the decomposition image by image wherever
 	// those were taken (1.6 to 5 times over 60 layers); ahead of the band kernel by the two estimates, with a margin for
-	// their errors (8 x 116 x 24 x 24 -> 25 channels 3 x 3: 12.9 -> 8.0 us, 12 x 18 x 56 x 56 -> 144: 28.2 -> 11.2; 11 x 36 x
-	// 14 x 14 -> 32 stays, 7.4 against 8).  Option "conv_variant" 11 to 16 forces a tile.
+	// their errors (8 x 116 x 24 x 24 -> 25 channels 3 x 3: 12.9 -> 8.0 us, 12 x 18 x 56 x 56 -> 144: 27.3 -> 11.4; 18 x 4 x 12 x 12 -> 61
+	// stays, 5.3 against 6.8).  Option "conv_variant" 11 to 16 forces a tile.
 	// Layers that one of the kernels of one launch could take leave the caller's workspace as it is, whatever they run as: the
 	// header says so.  What they fill is memory of the library's; the others fill the workspace.
 	// Before that the kernel that has a band of the input and its weights in LDS (convq_region.hip), one launch without memory of
-	// its own, where it is ahead of both by the estimates with the same margin: 32 x 64 x 56 x 56 -> 64 channels 3 x 3 15.7 ->
-	// 11.1 us (two launches), 4 x 8 x 52 x 52 -> 149 9.9 -> 6.2 (bands); 59 x 37 x 16 x 16 -> 39 5 x 5 stays, 9.5 against 12.9, and
-	// 18 x 4 x 12 x 12 -> 61, 5.6 against 5.8.  Option "conv_variant" 20 forces it.
+	// its own, where it is ahead of both by the estimates with such margins: 32 x 64 x 56 x 56 -> 64 channels 3 x 3 16.1 -> 12.0 us (two
+	// launches), 4 x 8 x 52 x 52 -> 149 9.8 -> 6.4 (bands) or 7.0; 59 x 37 x 16 x 16 -> 39 5 x 5 stays, 9.5 against 14.5, 8 x 138 x 27 x 27 ->
+	// 117 1 x 1, 7.2 against 7.3, and 18 x 4 x 12 x 12 -> 61, 5.3 against 5.9.  Option "conv_variant" 20 forces it.
 	if (!out_acc && (variant == 0 || variant > 10) && (variant > 10 || (K <= CQ_MAXK ? Cout >= 48 : !conv2dq_image_takes(g, w)))) {
 		uint64_t bytes = 0;
-		const double here = conv2dq_pixels_us(g, bytes), band_us = conv2dq_band_us(g), band = rows_ahead && K > CQ_MAXK ? -1.0 : band_us;
+		double here = conv2dq_pixels_us(g, bytes);
+		if (bytes > lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw)) here = -1.0;  // (no more than the workspace would hold in any case)
+		const double band_us = conv2dq_band_us(g), band = rows_ahead && K > CQ_MAXK ? -1.0 : band_us;
 		const bool one_launch = K <= CQ_MAXK || band_us >= 0.0 || conv2dq_image_takes(g, w);
 		if ((variant == 0 || variant == 20) && (one_launch || workspace != nullptr)) {  // (the other layers' contract wants a workspace, whatever they run as)
-			// (two launches that the estimate has at its least, 8.1 us, were 8.6 to 9.1 over 20 such layers: 4 x 52 x 16 x 16 -> 82 8.8 us
-			// and 7.0 here, 8 x 138 x 27 x 27 -> 117 1 x 1 8.6 and 7.1, 30 x 56 x 13 x 13 -> 72 8.8 and 7.5)
-			const double other = std::min(here < 0.0 ? 1e30 : std::max(here, 8.6), band_us < 0.0 ? 1e30 : band_us);
-			const int rc = conv2dq_region_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), variant == 20 ? 1e30 : 0.85 * other);
+			const double limit_us = std::min(here < 0.0 ? 1e30 : 0.95 * here, band_us < 0.0 ? 1e30 : 0.95 * band_us);
+			const int rc = conv2dq_region_dispatch(g, x, w, bias, zp_in, zp_w, mult, zp_out, static_cast<uint8_t*>(y), variant == 20 ? 1e30 : limit_us);
 			if (rc >= 0) return rc;
 		}
-		const uint64_t allowed = lten_hip_conv2dq_workspace_bytes(N, Cin, H, W, Cout, kh, kw, ph, pw, sh, sw);  // (no more than the workspace would hold in any case)
-		if (variant != 20 && here >= 0.0 && bytes <= allowed && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.85 * band))) {
+		if (variant != 20 && here >= 0.0 && (variant > 10 || (band < 0.0 ? K > CQ_MAXK : here < 0.93 * band))) {
 			// images in groups whose pixels the library's memory holds, one at least
 			ConvGeo part = g;
 			if (one_launch && bytes > LIBRARY_LIMIT) {

@@ -634,22 +634,25 @@ double conv2dq_band_estimate_us(const ConvGeo& g)
 	return wgs * ((double)pl.RH * pl.RW * pl.PP + (double)pl.ncb * 16 * pl.wpitch) / 1.3e6;
 }
 
-// The same, term by term, where the other side of the choice is the two launches of convq_pixels.hip (negative: no plan):
-// per workgroup of a round of 512 a start, the region's bytes, the weights' by the way they are staged, k-steps times
-// passes, and the output.  Fitted to 180 layers (14 % rms, 38 % at most).
+// The same, term by term, where the other side of the choice is the two launches of convq_pixels.hip or the band in LDS of
+// convq_region.hip (negative: no plan): the region's bytes, the weights' by the way they are staged, k-steps times passes and a
+// start, all of it for the first workgroup of a CU, what it adds for every further one, and the output.  Fitted to 2323 layers of 1 to
+// 256 images, 1 to 512 channels, 1 x 1 to 7 x 7 windows, strides 1 to 3 (13 % rms; with the rounds counted in 512 workgroups and the
+// weights of any multiple of four channels taken for permuted in registers it was 23 %).
 double conv2dq_band_us(const ConvGeo& g)
 {
 	BandPlan pl;
 	if (!band_plan(g, pl)) return -1.0;
 	const int T = g.kh * g.kw;
 	const int64_t HW = (int64_t)g.Ho * g.Wo;
+	const bool permuted = g.Cin % 4 == 0 && (T == 1 || T == 9 || T == 25 || T == 49);
 	const double wgs = (double)g.N * ((g.Ho + pl.TB - 1) / pl.TB) * ((((g.Cout + 15) / 16) + pl.ncb - 1) / pl.ncb);
-	const double region = 1e-4 * (double)pl.RH * pl.RW * pl.PP * (g.W % 4 != 0 ? 1.1 : 1.0);
-	const double weights = 1e-4 * (double)pl.ncb * 16 * pl.wpitch * (g.Cin % 4 == 0 ? 1.07 : (int64_t)g.Cin * T % 4 == 0 ? 6.8 : 3.8);
-	const int passes = ((pl.TB * g.Wo + 15) / 16 + 15) / 16;
-	const double us = std::max(1.0, wgs / 512) * (2.34 * region + weights + 0.195 * (pl.Kp / 64) * passes + 3.82) +
-	                  1.23e-6 * (double)g.N * (double)HW * g.Cout * (HW % 4 != 0 ? 1.94 : 1.0);
-	return std::max(us, 4.5);
+	const double region = 1e-4 * (double)pl.RH * pl.RW * pl.PP * (g.W % 4 != 0 ? 1.2 : 1.0);
+	const double weights = 1e-4 * (double)pl.ncb * 16 * pl.wpitch * (permuted ? 1.07 : g.Cin % 4 == 0 ? 2.55 : (int64_t)g.Cin * T % 4 == 0 ? 2.34 : 3.34);
+	const double walk = (double)(pl.Kp / 64) * (((pl.TB * g.Wo + 15) / 16 + 15) / 16);
+	const double us = 3.7 + 1.38 * region + weights + 0.2 * walk + std::max(0.0, wgs / 256 - 1.0) * (1.43 + 1.15 * region + 0.14 * weights + 0.31 * walk) +
+	                  1.24e-6 * (double)g.N * (double)HW * g.Cout * (HW % 4 != 0 ? 1.48 : 1.0);
+	return std::max(us, 5.2);
 }
 
 // 0 = launched; -1 = not a shape for this route

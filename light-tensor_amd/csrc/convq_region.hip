@@ -350,17 +350,17 @@ __global__ __launch_bounds__(512, 4) void conv2dq_region_kernel(ConvGeo g, Regio
 	}
 }
 
-static unsigned align16u(int64_t v) { return (unsigned)((v + 15) & ~15ll); }
+static int64_t align16(int64_t v) { return (v + 15) & ~15ll; }
 
-// The band's height: the one whose launch is expected to be over first, if that is within limit_us; what is expected: per round
-// of 256 workgroups the region's bytes, the weights' (where they are ordered byte by byte) and the k-steps of a SIMD's
-// wavefronts, and something for every further one (52 x 68 x 76 x 76 -> 85 1 x 1, three rounds: 37.5 us, 33.8 in two launches); the
-// output.  Fitted to 44 layers of 1 to 64 images, 4 to 250 channels, 1 x 1 to 5 x 5 windows, strides 1 and 2
-// (5 % rms).
+// The band's height: the one whose launch is expected to be over first, if that is within limit_us; what is expected: a launch and
+// the output; per round of 256 workgroups the region's bytes and the passes over it, the weights (as their channels come in fours or
+// are gathered byte by byte) and the k-steps of a SIMD's wavefronts.  Fitted to 4700 layers of 1 to 256 images, 1 to 512 channels, 1 x
+// 1 to 7 x 7 windows, strides 1 to 3 (9 % rms, 7 % in one round; a fit to 44 layers had sent 209 of 3485 here, or to a band of
+// another height, that took up to 1.5 times as long as elsewhere).
 static bool region_plan(const ConvGeo& g, RegionPlan& pl, double limit_us)
 {
 	const int64_t T = (int64_t)g.kh * g.kw, K = (int64_t)g.Cin * T;
-	const double least = 4.87 + 0.296e-6 * (double)g.N * g.Ho * g.Wo * g.Cout;
+	const double least = 4.0 + 0.23e-6 * (double)g.N * g.Ho * g.Wo * g.Cout;
 	if (least >= limit_us) return false;
 	if (g.dh != 1 || g.dw != 1 || g.ph >= g.kh || g.pw >= g.kw || T > 256 || g.Cin > 1024 || (int64_t)g.H * g.W >= (1 << 24) || (int64_t)g.Ho * g.Wo >= (1 << 24)) return false;
 	pl.UC = (g.Cin + 15) / 16;
@@ -372,11 +372,16 @@ static bool region_plan(const ConvGeo& g, RegionPlan& pl, double limit_us)
 	pl.groups = (g.Cout + 63) / 64;
 	pl.RW = (g.Wo - 1) * g.sw + g.kw;
 	const bool in_fours = g.Cin % 4 == 0 && (T == 9 || T == 25 || T == 1);
+	const int64_t weights = (int64_t)pl.rows * pl.wpitch, raw = std::min(pl.rows, g.Cout) * K;
+	const double order = in_fours ? 1.7e-5 * (double)raw : 1.6e-5 * (double)weights + 0.88 * ((pl.steps + 7) / 8) * (pl.rows / 64.0);
+	if (least + order + 0.64 + 0.55 + 0.1 * pl.steps >= limit_us) return false;  // (one round of the shortest bands)
 	double best = limit_us;
-	for (int tb = 1; tb <= g.Ho && (int64_t)tb * g.Wo <= 1024; tb++) {
-		const int rh = (tb - 1) * g.sh + g.kh, bands = (g.Ho + tb - 1) / tb, pairs = (tb * g.Wo + 63) / 64;
-		const int64_t region = (int64_t)rh * pl.RW * pl.PP, weights = (int64_t)pl.rows * pl.wpitch, raw = std::min(pl.rows, g.Cout) * K;
-		const int64_t bytes = align16u(region) + weights + align16u(raw) + 8 * pl.steps + 16 + pairs * 256 + 9 * 256;
+	// of the heights that cut an image into the same number of bands the least
+	for (int tb = 1, bands = 0; tb <= g.Ho && (int64_t)tb * g.Wo <= 1024; tb = bands > 1 ? (g.Ho + bands - 2) / (bands - 1) : g.Ho + 1) {
+		bands = (g.Ho + tb - 1) / tb;
+		const int rh = (tb - 1) * g.sh + g.kh, pairs = (tb * g.Wo + 63) / 64;
+		const int64_t region = (int64_t)rh * pl.RW * pl.PP;
+		const int64_t bytes = align16(region) + weights + align16(raw) + 8 * pl.steps + 16 + pairs * 256 + 9 * 256;
 		if (bytes > 160 * 1024) break;
 		bool whole = true;  // every band has the 16 bytes of a channel that a load takes (the first and the last have the fewest rows inside the image)
 		for (int b = 0; b < bands; b += std::max(bands - 1, 1)) {
@@ -387,16 +392,16 @@ static bool region_plan(const ConvGeo& g, RegionPlan& pl, double limit_us)
 		if (!whole || (int64_t)g.N * bands >= (1ll << 32) / 512) continue;  // (HIP launches fewer than 2^32 threads in a dimension)
 		const int fn = pl.rows == 64 && pairs > 4 ? 2 : 1;
 		const int units = pairs * (pl.rows / (32 * fn)), turns = (units + 7) / 8;
-		const double rounds = std::ceil((double)g.N * bands * pl.groups / 256.0);
-		const double t = least + rounds * (2.43e-5 * (double)region + (in_fours ? 0.1e-5 : 6.5e-5) * (double)weights + turns * (0.486 * fn + 0.0426 * pl.steps * (fn + 1))) +
-		                 1.5 * (rounds - 1.0);
+		const double rounds = (double)(((int64_t)g.N * bands * pl.groups + 255) / 256);
+		const int passes = (int)((((int64_t)rh * g.W + 127) / 128 * ((pl.UC + 1) / 2) + 7) / 8);  // tiles of 8 x 16 pixels of 32 channels a wavefront stages
+		const double t = least + rounds * (3.2e-5 * (double)region + 0.64 * passes + order + turns * (0.55 * fn + 0.05 * pl.steps * (fn + 1)));
 		if (t < best) {
 			best = t;
 			pl.TB = tb; pl.RH = rh; pl.bands = bands; pl.pairs = pairs;
-			pl.off_w = align16u(region);
+			pl.off_w = (unsigned)align16(region);
 			pl.off_raw = pl.off_w + (unsigned)weights;
-			pl.off_tab = pl.off_raw + align16u(raw);
-			pl.off_pos = pl.off_tab + align16u(8 * pl.steps);
+			pl.off_tab = pl.off_raw + (unsigned)align16(raw);
+			pl.off_pos = pl.off_tab + (unsigned)align16(8 * pl.steps);
 			pl.off_row = pl.off_pos + (unsigned)pairs * 256;
 			pl.off_sum = pl.off_row + 8 * 256;
 			pl.bytes = pl.off_sum + 256;

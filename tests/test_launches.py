@@ -79,5 +79,18 @@ def test_conv2dq_layers_that_want_a_workspace(launches, geo, kernel):
     assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
 
 
+@pytest.mark.parametrize("geo,kernel", [((32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), "conv2dq_region"),    # us in the band in LDS, two launches, the band kernel: 12.0, 16.1, 28.6
+                                        ((52, 173, 32, 32, 80, 1, 1, 0, 0, 2, 2), "conv2dq_region"),   # 9.4, -, 23.0 (the pixels would not fit the workspace)
+                                        ((3, 25, 72, 72, 32, 3, 3, 1, 1, 1, 1), "conv2dq_pixels"),     # 8.2, 6.9, -
+                                        ((60, 48, 72, 72, 112, 3, 3, 1, 1, 2, 2), "conv2dq_pixels"),   # 24.2, 20.2, -
+                                        ((1, 52, 15, 15, 220, 3, 3, 1, 1, 2, 2), "conv2dq_pixels"),    # 8.1, 6.3, -
+                                        ((2, 26, 36, 36, 16, 3, 3, 1, 1, 2, 2), "conv2dq_band"),       # 8.0, -, 6.8
+                                        ((21, 1, 89, 7, 473, 3, 3, 1, 1, 3, 3), "conv2dq_pixels")])    # 9.6, 7.1, -
+def test_conv2dq_layers_run_as_what_is_quickest(launches, geo, kernel):
+    """Layers whose kernels lie well apart, at the values of a measurement."""
+    r = launches("lten_hip_conv2dq_forward", *geo, DEVICE(1), DEVICE(2), None, QP, DEVICE(3), DEVICE(4))
+    assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
+
+
 if __name__ == "__main__":
     print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
