@@ -596,6 +596,33 @@ void launch_split(const SplitConv& p, bool t3)
 	else conv_split_kernel<BM, BN, WM, WN, Q, false><<<grid, dim3(512), 0, stream()>>>(p);
 }
 
+// The most consecutive pixels of a strip w columns wide whose patch the tile's quads hold, at most BN (tiles start at multiples of it).
+int split_step(const SplitClass& c, const SplitConv& p, const SplitTile& t, int w, int patch_q)
+{
+	const int budget = t.quads / patch_q, window = std::max(c.kh, p.sh), all_rows = p.N * c.Ho;
+	if (budget < window) return 0;
+	// rows that lie anywhere touch up to (rows - 2 + Ho) / Ho + 1 images, each with the rest of a window
+	auto images = [&](int rows) { return std::min(p.N, (rows - 2 + c.Ho) / c.Ho + 1); };
+	const int most = std::min(all_rows, (budget - window) / p.sh + 1);
+	auto fits = [&](int rows) { return rows * p.sh + images(rows) * (window - p.sh) <= budget; };
+	const int cap = std::min(most, (t.BN - 2 + w) / w + 1);
+	int any = cap;
+	if (!fits(any)) {
+		any = std::max(1, (budget - images(any) * (window - p.sh)) / p.sh);  // (with as many images as that: then up)
+		while (any < cap && fits(any + 1)) any++;
+	}
+	if (any == all_rows) return t.BN;
+	// whole rows of the strip: those, whole images, or a divisor of an image's rows
+	int whole = std::min(any, t.BN / w);
+	const int per_image = (c.Ho - 1) * p.sh + window, full = std::min({ p.N, budget / per_image, t.BN / w / c.Ho });
+	whole = std::max(whole, full * c.Ho);
+	for (int rows = std::min({ most, t.BN / w, c.Ho }); rows > whole; rows--)
+		if (c.Ho % rows == 0) whole = rows;
+	if (whole == all_rows) return t.BN;
+	// ((rows - 1) w + 1 pixels lie in up to `rows`)
+	return std::max(whole * w, std::min(t.BN, (any - 1) * w + 1));
+}
+
 // Lays the classes out in strips and tiles of the given kind; false when a patch would not fit.
 bool split_layout(SplitConv& p, const SplitTile& t)
 {
@@ -603,25 +630,25 @@ bool split_layout(SplitConv& p, const SplitTile& t)
 	uint64_t tiles = 0;
 	for (int k = 0; k < p.classes; k++) {
 		SplitClass& c = p.cls[k];
-		// strips of at most 128 columns, more and narrower ones where a patch would not fit; where none does, tiles of fewer pixels
+		// strips of at most 128 columns; where a patch would not fit, up to three more, and tiles of fewer pixels: of these the
+		// fewest tiles
 		const int first = (int)ceil_div((uint64_t)c.Wo, 128);
-		int64_t pixels = 0;
-		bool fits = false;
-		for (c.step = t.BN; c.step >= t.BN / 2 && !fits; c.step -= 16)
-			for (int strips = first; strips < first + 4 && !fits; strips++) {
-				c.strips = strips;
-				c.strip_w = (int)ceil_div((uint64_t)c.Wo, (uint64_t)strips);
-				c.patch_q = ((c.strip_w - 1) * p.sw + c.kw + 3) / 4;
-				pixels = (int64_t)p.N * c.Ho * c.strip_w;
-				if (pixels >= (1ll << 30)) return false;
-				// the most rows and images that `step` consecutive pixels touch (tiles start at multiples of it)
-				const int64_t w = c.strip_w, all_rows = (int64_t)p.N * c.Ho, step = c.step;
-				const int64_t rows = std::min(all_rows, step % w == 0 ? step / w : w % step == 0 ? 1 : (step - 2) / w + 2);
-				const int64_t images = std::min<int64_t>(p.N, step % w == 0 && c.Ho % rows == 0 ? 1 : step % w == 0 && rows % c.Ho == 0 ? rows / c.Ho : (rows - 2 + c.Ho) / c.Ho + 1);
-				fits = ((rows - images) * p.sh + images * std::max(c.kh, p.sh)) * c.patch_q <= t.quads;
+		int64_t pixels = 0, least = INT64_MAX;
+		for (int strips = first; strips < first + 4; strips++) {
+			const int strip_w = (int)ceil_div((uint64_t)c.Wo, (uint64_t)strips), patch_q = ((strip_w - 1) * p.sw + c.kw + 3) / 4;
+			const int64_t strip_pixels = (int64_t)p.N * c.Ho * strip_w;
+			if (strip_pixels >= (1ll << 30)) return false;
+			const int step = split_step(c, p, t, strip_w, patch_q);
+			if (step < t.BN / 2) continue;
+			const int64_t tiles_here = (int64_t)((strip_pixels + step - 1) / step) * strips;
+			if (tiles_here < least) {
+				least = tiles_here;
+				c.step = step; c.strips = strips; c.strip_w = strip_w; c.patch_q = patch_q;
+				pixels = strip_pixels;
 			}
-		c.step += 16;  // (as the loop left it)
-		if (!fits) return false;
+			if (step == t.BN) break;
+		}
+		if (least == INT64_MAX) return false;
 		c.pixels = (int)pixels;
 		c.tiles_n = (int)ceil_div((uint64_t)pixels, (uint64_t)c.step);
 		if (tiles > (1ull << 28)) return false;
@@ -640,15 +667,18 @@ bool split_t3(const SplitConv& p)
 	return true;
 }
 
-// What a launch takes, in us: the two launches, rounds of tiles on 256 CUs; a chunk as long as its matrix instructions (taps that
-// are counted at run time cost 10 % more) or its staging (9.5 ns a quad); the start and the store of a tile.  Classes of one to four
-// taps switch between the two limits and store every other pixel.
+// What a launch takes, in us: the two launches, rounds of tiles on 256 CUs; a chunk as long as its matrix instructions (where taps are
+// counted at run time 10 % more; the tiles of eight blocks, which never have them written out, have the nine taps' time in theirs) or
+// its staging (9.5 ns a quad); the start and the store of a tile.  Where CUs stay idle the others run at a higher clock (32 x 64 x 32 x
+// 32 -> 32 5 x 5: 32.3 us in 128 tiles of 32 x 256, 38.4 in 256 of 64 x 128, half of them padding).  Classes of one to four taps switch
+// between the two limits and store every other pixel.  Over 4300 layers and 25 thousand (layer, tile) pairs it is 10 % above the time,
+// 12 to 16 % rms, and the tile it picks 1.2 % behind the quickest in the mean.
 double split_us(const SplitConv& p, const SplitTile& t)
 {
-	const double rounds = (double)ceil_div(ceil_div((uint64_t)p.tiles, 8), 32), slower = split_t3(p) ? 1.0 : 1.1;
+	const double rounds = (double)ceil_div(ceil_div((uint64_t)p.tiles, 8), 32), slower = split_t3(p) ? 1.0 : 1.1, clock = 0.8 + 0.2 * p.tiles / (256.0 * rounds);
 	double chunk_us = 0;
-	for (int k = 0; k < p.classes; k++) chunk_us += std::max(p.cls[k].kh * p.cls[k].kw * 6e-3 * t.blocks * t.mfma_ns * slower, t.quads * 9.5e-3) / p.classes;
-	if (p.classes > 1) return 9.0 + rounds * (p.chunks * chunk_us * (t.blocks == 8 ? 1.6 : 1.25) + t.round_us * 1.4);
+	for (int k = 0; k < p.classes; k++) chunk_us += std::max(p.cls[k].kh * p.cls[k].kw * 6e-3 * t.blocks * t.mfma_ns * slower * clock, t.quads * 9.5e-3) / p.classes;
+	if (p.classes > 1) return 0.95 * (9.0 + rounds * (p.chunks * chunk_us * (t.blocks == 8 ? 1.6 : 1.25) + t.round_us * 1.4));
 	return 9.0 + rounds * (p.chunks * chunk_us + t.round_us);
 }
 

@@ -391,6 +391,9 @@ def test_weight_gradient_of_wide_layers_on_integers(gpu, N, Cin, Cout):
     (12, 90, 7, 7, 70, 3, 3, 1, 1, 1, 1),      # narrow maps: more positions to a tile than pixels, tiles of fewer than 256 pixels
     (20, 20, 33, 33, 40, 5, 5, 2, 2, 2, 2),    # a window and stride that fit with narrow strips or small tiles only
     (3, 16, 31, 43, 64, 3, 3, 0, 0, 2, 2),     # 3 x 3 at stride 2, one chunk, no padding
+    (9, 20, 22, 22, 13, 5, 5, 4, 2, 2, 2),     # tiles of 122 pixels
+    (5, 33, 40, 41, 35, 3, 3, 1, 1, 2, 2),     # tiles of 75 and 133 pixels, strips of columns
+    (30, 18, 5, 9, 33, 7, 7, 3, 3, 1, 1),      # whole images to a tile
 ])
 def test_patches_of_quads_on_integers(gpu, geo):
     """The quads at the ends of a plane, patches that do not fit at a full tile, one chunk to six.  Exact in any order."""

@@ -92,5 +92,25 @@ def test_conv2dq_layers_run_as_what_is_quickest(launches, geo, kernel):
     assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
 
 
+@pytest.mark.parametrize("geo,kernel", [((23, 5, 111, 107, 15, 3, 3, 1, 0, 1, 1), "conv2d_patch_forward_3x3_32x4x128"),    # us there and on pieces: 22, 30
+                                        ((18, 7, 100, 100, 205, 3, 3, 0, 1, 1, 1), "conv2d_patch_forward_3x3_32x4x128"),   # 86, 108 to 144
+                                        ((23, 3, 88, 88, 20, 7, 7, 0, 0, 1, 1), "conv2d_forward_32x128x32"),               # 41, 50
+                                        ((53, 8, 29, 29, 32, 5, 5, 0, 0, 1, 1), "conv2d_pieces_forward"),                  # 22, 17
+                                        ((21, 372, 13, 124, 6, 3, 3, 1, 2, 1, 1), "conv2d_pieces_forward")])               # 199, 59
+def test_conv2d_layers_run_as_what_is_quickest(launches, geo, kernel):
+    """Forward layers whose routes lie well apart, at the values of a measurement."""
+    r = launches("lten_hip_conv2d_forward_f32", *geo, DEVICE(1), DEVICE(2), None, DEVICE(3))
+    assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
+
+
+@pytest.mark.parametrize("geo,tile,tiles", [((208, 48, 22, 22, 13, 5, 5, 4, 2, 2, 2), "ILi64ELi128ELi2ELi2ELi210E", 244),   # 122 pixels to a tile: one round
+                                            ((32, 64, 32, 32, 32, 5, 5, 2, 2, 1, 1), "ILi32ELi256E", 128)])              # not 64 rows for 32 channels
+def test_conv2d_tiles_on_pieces(launches, geo, tile, tiles):
+    """The tile and, up to the CUs, how many of them: pixels to a tile in no steps of 16, no tile half of whose rows are padding."""
+    r = launches("lten_hip_conv2d_forward_f32", *geo, DEVICE(1), DEVICE(2), None, DEVICE(3))
+    seen = [(name, x) for name, x, *_ in r["launches"] if "conv_split_kernel" in name]
+    assert len(seen) == 1 and tile in seen[0][0] and seen[0][1] == (tiles + 7) // 8 * 8, seen
+
+
 if __name__ == "__main__":
     print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
