@@ -322,6 +322,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 		// Operands of column blocks are read DB blocks ahead: with one row block to a column block its six matrix instructions are
 		// over before an LDS read that queues behind the staging half's writes has come back.
 		constexpr int DB = FM == 1 ? 2 : 1, SETS = FM == 2 ? 2 : D == 2 ? 3 : 4;
+		static_assert(!T3 || 9 % (D + 1) == 0, "a k-step's weights are the same in every chunk");
 		static_assert((T3 ? 9 : D + 1) * FN % SETS == 0 && SETS > DB, "a block's operand set is the same in every round of k-steps");
 		bf16x8 fa[D + 1][FM][3], fb[SETS][3];
 		// (the loads run up to D k-steps past a block: into the next one, or what the buffer has behind the last one)
@@ -372,8 +373,8 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 			for (int b = 0; b < DB; b++)
 #pragma unroll
 				for (int v = 0; v < 3; v++) read_b(b, slot_at(b, 0, stage_at), v);
-			auto k_step = [&](auto phase_c, auto tap_c) {
-				constexpr int TAP = decltype(tap_c)::value, NEXT = (TAP + 1) % 9, SET = (TAP + decltype(phase_c)::value) % (D + 1), FIRST = TAP * FN;
+			auto k_step = [&](auto tap_c) {
+				constexpr int TAP = decltype(tap_c)::value, NEXT = (TAP + 1) % 9, SET = TAP % (D + 1), FIRST = TAP * FN;
 #pragma unroll
 				for (int j = 0; j < FN; j++) {
 					const bool ahead = j >= FN - DB;  // the block that is read is of the next k-step
@@ -398,24 +399,17 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 					}
 				}
 			};
-			auto chunk = [&](auto phase_c) {
-				k_step(phase_c, std::integral_constant<int, 0>{});
-				k_step(phase_c, std::integral_constant<int, 1>{});
-				k_step(phase_c, std::integral_constant<int, 2>{});
-				k_step(phase_c, std::integral_constant<int, 3>{});
-				k_step(phase_c, std::integral_constant<int, 4>{});
-				k_step(phase_c, std::integral_constant<int, 5>{});
-				k_step(phase_c, std::integral_constant<int, 6>{});
-				k_step(phase_c, std::integral_constant<int, 7>{});
-				k_step(phase_c, std::integral_constant<int, 8>{});
-			};
 			for (int left = p.chunks;;) {
-				chunk(std::integral_constant<int, 0>{});
+				k_step(std::integral_constant<int, 0>{});
+				k_step(std::integral_constant<int, 1>{});
+				k_step(std::integral_constant<int, 2>{});
+				k_step(std::integral_constant<int, 3>{});
+				k_step(std::integral_constant<int, 4>{});
+				k_step(std::integral_constant<int, 5>{});
+				k_step(std::integral_constant<int, 6>{});
+				k_step(std::integral_constant<int, 7>{});
+				k_step(std::integral_constant<int, 8>{});
 				if (--left == 0) break;
-				if (9 % (D + 1) != 0) {
-					chunk(std::integral_constant<int, 9 % (D + 1)>{});
-					if (--left == 0) break;
-				}
 			}
 			stage = stage_at != 0;
 		} else {
