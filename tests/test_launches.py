@@ -19,18 +19,19 @@ def launches(lt, tmp_path_factory):
     stub = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
     subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", stub, os.path.join(HERE, "hip_stub.c")], check=True)
 
-    def run(name, *args):
-        out = subprocess.run([sys.executable, __file__, stub, name, json.dumps(args)], check=True, stdout=subprocess.PIPE, text=True)
+    def run(name, *args, variant=0):
+        out = subprocess.run([sys.executable, __file__, stub, name, json.dumps(args), str(variant)], check=True, stdout=subprocess.PIPE, text=True)
         return json.loads(out.stdout.splitlines()[-1])
     return run
 
 
-def call_on_the_stub(stub_path, name, args):
+def call_on_the_stub(stub_path, name, args, variant):
     stub = C.CDLL(stub_path, mode=C.RTLD_GLOBAL)   # before the library, whose HIP calls it takes
     stub.stub_name.restype = C.c_char_p
     sys.path.insert(0, HERE)
     from conftest import load_package
     lt = load_package()
+    lt.set_option("conv_variant", variant)
     rc = getattr(lt.lib(), name)(*[lt.qparams3(*a["qparams"]) if isinstance(a, dict) else a for a in args])
     seen, dims = [], (C.c_uint64 * 5)()
     for i in range(stub.stub_launches()):
@@ -92,6 +93,19 @@ def test_conv2dq_layers_run_as_what_is_quickest(launches, geo, kernel):
     assert (r["rc"], r["kernel"]) == (0, kernel), r["error"]
 
 
+# (bands of an image, blocks of 32 channels a wavefront multiplies at once) of the layers that the GPU tests force on the band in LDS
+@pytest.mark.parametrize("geo,bands,fn", [((32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), 8, 2), ((64, 16, 112, 112, 60, 3, 3, 1, 1, 2, 2), 4, 2),
+                                          ((64, 16, 56, 56, 32, 3, 3, 1, 1, 1, 1), 4, 1), ((64, 15, 57, 55, 29, 3, 3, 1, 1, 1, 1), 4, 1),
+                                          ((40, 14, 111, 109, 70, 3, 3, 1, 1, 2, 2), 8, 2), ((64, 48, 28, 28, 120, 1, 1, 0, 0, 1, 1), 2, 2),
+                                          ((3, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1), 56, 1)])
+def test_conv2dq_region_bands(launches, geo, bands, fn):
+    N, Cout = geo[0], geo[4]
+    r = launches("lten_hip_conv2dq_forward", *geo, DEVICE(1), DEVICE(2), None, QP, DEVICE(3), DEVICE(4), variant=20)
+    assert (r["rc"], r["kernel"], len(r["launches"])) == (0, "conv2dq_region", 1), r["error"]
+    name, x, y, z, *_ = r["launches"][0]
+    assert (x, y, z) == (N * bands, (Cout + 63) // 64, 1) and f"ELi{fn}E" in name, r["launches"]
+
+
 @pytest.mark.parametrize("geo,kernel", [((23, 5, 111, 107, 15, 3, 3, 1, 0, 1, 1), "conv2d_patch_forward_3x3_32x4x128"),    # us there and on pieces: 22, 30
                                         ((18, 7, 100, 100, 205, 3, 3, 0, 1, 1, 1), "conv2d_patch_forward_3x3_32x4x128"),   # 86, 108 to 144
                                         ((23, 3, 88, 88, 20, 7, 7, 0, 0, 1, 1), "conv2d_forward_32x128x32"),               # 41, 50
@@ -113,4 +127,4 @@ def test_conv2d_tiles_on_pieces(launches, geo, tile, tiles):
 
 
 if __name__ == "__main__":
-    print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]))))
+    print(json.dumps(call_on_the_stub(sys.argv[1], sys.argv[2], json.loads(sys.argv[3]), int(sys.argv[4]))))
