@@ -22,12 +22,12 @@
 // Measured (forward; fp32 matrix instructions or column matrices -> here): 32 x 32 x 128 x 128 -> 64 channels 3 x 3
 // 155 -> 111 us (174 TFLOP/s), 32 x 256 x 14 x 14 -> 256 81 -> 50, 16 x 64 x 57 x 57 -> 128 at stride 2 40 -> 22, 17 x 352 x
 // 50 x 50 -> 48 427 -> 90, 30 x 176 x 14 x 14 -> 320 5 x 5 205 -> 88.  One wavefront to a SIMD multiplies, so what stands
-// between two of its matrix instructions is lost: a k-step of the small tiles took 560 clocks of which 384 are matrix
-// instructions while the taps were counted between k-steps and operands read one block ahead, and takes 430 with the nine
-// taps of a 3 x 3 window written out, loads and reads each behind a matrix instruction and operands read two blocks ahead
-// (32 x 256 x 14 x 14 -> 256: 60 -> 50 us; 40 x 50 x 28 x 28 -> 150 46 -> 40, 64 x 256 x 7 x 7 -> 512 58 -> 51).
-// Bound by the matrix cores (clocks in matrix instructions: 75 to 85 % of the main loop, 2.1 to 2.3 GHz); then the stores at the
-// end of a tile, which all CUs reach together (32 KB to 128 KB a CU: 2 to 8 us at 4.2 TB/s), and the first chunk (3 to 4.5 us).
+// between two of its matrix instructions is lost.  With the nine taps of a 3 x 3 window written out (not counted between k-steps),
+// loads and reads each behind a matrix instruction, operands read two blocks ahead and staging by quads, 32 x 256 x 14 x 14 -> 256
+// went from 60 to 50 us (its kernel from 114 to 88 thousand clocks, 42 of them in matrix instructions), 40 x 50 x 28 x 28 -> 150
+// 46 -> 40, 64 x 256 x 7 x 7 -> 512 58 -> 51.
+// Bound by the matrix cores (49 to 59 % of a whole launch's clocks at 32 x 32 x 128 x 128 -> 64, at about 2 GHz); then the stores at
+// the end of a tile, which all CUs reach together (32 KB to 128 KB a CU: 2 to 8 us at 4.2 TB/s), and the first chunk (3 to 4.5 us).
 //
 // 2-norm error against float64 over 22 layers each way, the routes before -> here: 0.31 to 0.5 of it in the tiles of four or
 // fewer blocks of 32 x 32, whose registers leave room for sums of their own (below), 0.8 to 0.9 in the tiles of eight; up to
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 		}
 		if constexpr (T3) {
 			// Nine k-steps to a chunk, written out.  (With the taps counted at run time the scalar instructions between two k-steps
-			// took the pipe 60 to 110 clocks of 384.)  Where registers are left, the addresses of a row's taps are kept.
+			// leave the pipe empty.)  Where registers are left, the addresses of a row's taps are kept.
 			constexpr bool KEPT = FM * FN == 2;
 			uint32_t slot3[KEPT ? FN : 1][3];
 			if (KEPT) {
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_kernel(SplitConv p)
 			advance();
 			// One k-step: the matrix instructions of every column block, the operands of a later block read under them, those of the
 			// next k-step's first blocks behind a barrier where that is the next chunk's.  Everything else stands behind a matrix
-			// instruction too: between two k-steps it left the pipe empty for 110 clocks.
+			// instruction too: between two k-steps it would leave the pipe empty.
 			auto k_step = [&](auto par_c) {
 				constexpr int PAR = decltype(par_c)::value, FIRST = PAR * FN;
 #pragma unroll

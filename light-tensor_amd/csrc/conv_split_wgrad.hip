@@ -14,10 +14,11 @@
 // half multiplies: two blocks of 32 channels x two halves of the chunk's k-steps of 16 pixels, nine accumulators each, added at
 // the end.  Measured (patch kernels, column matrices -> here): 32 x 32 x 128 x 128 -> 64 channels 171 -> 107 us (180 TFLOP/s),
 // 32 x 256 x 14 x 14 -> 256 120 -> 51, 27 x 124 x 35 x 35 -> 32 86 -> 38; at stride two a chunk's staging is the longer half (16
-// x 64 x 57 x 57 -> 128: 32.3 us against the implicit GEMM's 44).  What staging a chunk takes had bound stride one too, 5800
-// clocks to the 4000 of its products: loads that touched 64 cache lines each (3500 clocks of them), divisions, conversions of two
-// values at a time, in which every instruction waits for the one before.  Now it is 4300 (3800 at stride two, was 5100), and
-// the chip is at its power limit on long runs (1.7 GHz; 120 -> 107, 59 -> 51, 97 -> 86 us at 64 x 128 x 28 x 28).  Shifting the operands of the next tap
+// x 64 x 57 x 57 -> 128: 32.3 us against the implicit GEMM's 44).  Staging had bound stride one too: loads
+// that touched 64 cache lines each, divisions, conversions of two values at a time, in which every instruction waits for the one
+// before.  Without them the first kernel takes 175 thousand clocks, not 230, of which 111 are matrix instructions' (the second 87,
+// not 109, of which 48; 57, not 67, at stride two), and slower ones, for the power limit: 120 -> 107, 59 -> 51, 97 -> 86 us
+// at 64 x 128 x 28 x 28.  Shifting the operands of the next tap
 // between the products of this one instead of ahead of them made no difference.  The sums of the slices go to memory
 // of the library as [slice][tap][co][ci] and are added in order by a second launch.
 // 2-norm error against float64 over 16 layers, the routes before -> here: 0.07 to 0.95 of it on uniform values, 0.24 to 1.3 on
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(512, 2) void conv_split_wgrad_kernel(SplitWgrad p)
 		// x: two lanes to a slot.  A wavefront takes eight channels: all 32 slots of one at a time, at stride two 16 slots of two at a
 		// time and then the other four slots of all eight.  dy: two lanes to an octet, all octets of DY_LANES channels at a time.  So the
 		// lanes of a load read rows that lie next to each other (with 16 channels of four slots to a wavefront every lane had a cache
-		// line of its own, and the loads of a chunk took 3500 clocks).
+		// line of its own).
 		const int w = wave & 3, h = lane & 1;
 		constexpr int COLS = 4 * S, KINDS = S;    // columns of a lane; kinds of slots it takes: its first, its second
 		constexpr int DY_STEP = 4 * T::DY_LANES;  // channels from one unit to the next
@@ -520,8 +521,8 @@ int conv_split_wgrad(const ConvGeo& g, const float* x, const float* dy, float* d
 	p.slices = (int)ceil_div((uint64_t)p.chunks, (uint64_t)p.per_slice);
 	const uint64_t Mp = (uint64_t)p.tiles_m * 64, Cp = (uint64_t)(p.tiles / p.tiles_m) * 32, bytes = (uint64_t)p.slices * 9 * Mp * Cp * 4;
 	if (bytes > (1ull << 29) || (uint64_t)p.tiles * p.slices >= (1u << 24)) return -1;
-	// a chunk: two k-steps of 54 products (32 clocks each, 41 with what comes between), at stride two its staging (3900 clocks
-	// with 15 slots); a start and an end; the launches and the sums
+	// a chunk: two k-steps of 54 products (32 clocks each; 41 and, at stride two, the staging's 3900 with 15 slots are fitted to times);
+	// a start and an end; the launches and the sums
 	const double rounds = (double)ceil_div((uint64_t)p.tiles * p.slices, 256), chunk_clocks = S == 1 ? 2 * 54 * 41.0 : 3900.0 + 200.0 * (double)std::max<int64_t>(0, best_used - 16);
 	if (10.0 + rounds * (p.per_slice * chunk_clocks + 8000.0) / 1850.0 + 1.2 * (double)bytes / 4e6 >= limit_us) return -1;
 	p.partial = static_cast<float*>(library_scratch(bytes));

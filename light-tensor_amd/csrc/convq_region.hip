@@ -9,11 +9,12 @@
 // way before anything else is done, and turns them into 16 dwords of four channels.  The weights come in as they lie, 16 bytes
 // a thread, and are put in order out of LDS (fetched in order, a load touched 64 cache lines).
 //
-// 32 x 64 x 56 x 56 -> 64 channels 3 x 3: 15.7 -> 11.1 us (two launches of 4.3 and 9.7 us, the pixels written and read again
-// between them), of which a launch is 4.5, loads and LDS writes 2, the 18 k-steps of two wavefronts a SIMD 2.5 and the
-// stores 1.8.  16 x 32 x 28 x 28 -> 64 8.3 -> 6.2, 44 x 15 x 80 x 80 -> 29 16.8 -> 12.0, 24 x 24 x 48 x 48 -> 16 stride 2
-// 11.4 -> 6.1, 1 x 249 x 28 x 28 -> 128 1 x 1 stride 2 11.8 -> 7.1.  With copies between the operand sets and the weights'
-// sums in the loop the first took 11.7 us.
+// 32 x 64 x 56 x 56 -> 64 channels 3 x 3: 15.2 -> 11.4 us (two launches of 5.6 and 10.9 us on cold clocks, the pixels written and
+// read again between them, against one of 13.5), in 44 thousand clocks of which 4 are matrix instructions'.  Bound by its parts one
+// after the other: by the terms of the estimate below a launch 4.0, the stores 1.5, loads and LDS writes 2.0, the weights' order 0.6,
+// the 18 k-steps of two wavefronts a SIMD 3.8.  16 x 32 x 28 x 28 -> 64 8.3 -> 6.2, 44 x 15 x 80 x 80 -> 29 16.1 -> 12.0, 24 x 24 x
+// 48 x 48 -> 16 stride 2 11.4 -> 6.1, 1 x 249 x 28 x 28 -> 128 1 x 1 stride 2 11.8 -> 7.1.  With copies between the operand sets and
+// the weights' sums in the loop the first took 11.7 us.
 #include "conv_common.h"
 #include "qgemm_common.h"
 

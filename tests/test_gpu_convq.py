@@ -273,7 +273,7 @@ def test_conv2dq_region_vs_oracle(gpu, ob, geo):
 
 
 # Layers with enough images for bands of many rows: blocks of 64 channels a wavefront, several of them and several staging tiles one
-# after another (bands, blocks and tiles are in test_launches.py); and 1 x 1 windows, whose weights are ordered four channels at a time.
+# after another (the bands are asserted in test_launches.py); and 1 x 1 windows, whose weights are ordered four channels at a time.
 REGION_TALL_GEOS = [(32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),     # 7 rows: 7 blocks of 64 x 64
                     (64, 16, 112, 112, 60, 3, 3, 1, 1, 2, 2),   # 14 rows: 13 blocks, 26 staging tiles, four rows of weights empty
                     (64, 16, 56, 56, 32, 3, 3, 1, 1, 1, 1),     # 14 rows: 13 blocks of 64 x 32
